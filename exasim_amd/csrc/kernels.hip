@@ -11,6 +11,7 @@
 //
 // Every reduction has a fixed order and no atomics are used, so results are
 // bitwise reproducible from run to run.
+#include "blkval.hpp"
 #include "kernels.hpp"
 #include "models.hpp"
 #include "common.hpp"
@@ -1790,128 +1791,6 @@ __global__ void k_bj_apply(Dims d, const T* BE, const double* x, double* y, cons
   y[q] = s;
 }
 
-// Block entries as doubles: FP64 / FP32 storage, or BF16 kept as the upper 16 bits of an FP32
-// (unsigned short storage)
-template <typename T>
-__device__ __forceinline__ double blk_val(T x) { return static_cast<double>(x); }
-template <>
-__device__ __forceinline__ double blk_val<unsigned short>(unsigned short x) {
-  return static_cast<double>(__uint_as_float(static_cast<unsigned int>(x) << 16));
-}
-
-// hdgMatVec element part (matvec.cpp:377-380): we_e = H_e * v_e with v_e gathered
-// through elemcon.  One workgroup per element; each of the 4 waves owns a
-// quarter of the columns, lanes own VW consecutive rows (16-byte vector loads of
-// the column), accumulation is FP64, and the four partial sums are added in LDS
-// in a fixed order.
-// NRB > 0: exactly NRB row blocks of 64 VW rows (m > 64 VW (NRB - 1)), with CB columns' loads
-// issued before their FMAs (more bytes in flight per wave; a row's FMAs still run over the columns
-// in order); NRB = 0: any m <= 1024, one column at a time.
-template <typename T, int VW, int NRB>
-__global__ __launch_bounds__(256) void k_matvec_elem(Dims d, const T* H, const int* elemcon,
-                                                     const double* v, double* we, const int* einst,
-                                                     const double* emask) {
-  typedef T vecT __attribute__((ext_vector_type(VW)));
-  constexpr int MAXRB = NRB > 0 ? NRB : (1024 + 64 * VW - 1) / (64 * VW);  // m <= 1024
-  constexpr int CB = NRB > 0 ? (sizeof(T) <= 4 ? 4 : 2) : 1;
-  const int m = d.m, ncu = d.ncu, ndf = d.ndf;
-  const long e = blockIdx.x;
-  if (emask && einst && emask[einst[e]] == 0.0) {  // block-uniform: the element's instance is inactive
-    for (int r = threadIdx.x; r < m; r += 256) we[e * m + r] = 0.0;
-    return;
-  }
-  extern __shared__ double sm[];
-  double* ve = sm;          // m
-  double* red = sm + m;     // 4*m
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int t = tid; t < m; t += 256)
-    ve[t] = v[(t % ncu) + ncu * static_cast<long>(elemcon[t / ncu + ndf * e])];
-  __syncthreads();
-  const int cper = (m + 3) / 4;
-  const int c0 = wave * cper, c1 = min(m, c0 + cper);
-  const int nrb = (m + 64 * VW - 1) / (64 * VW);
-  double acc[MAXRB][VW];
-#pragma unroll
-  for (int rb = 0; rb < MAXRB; ++rb)
-#pragma unroll
-    for (int q = 0; q < VW; ++q) acc[rb][q] = 0.0;
-  const T* He = H + e * static_cast<long>(m) * m;
-  int cfirst = c0;
-  if (CB > 1) {
-    for (; cfirst + CB <= c1; cfirst += CB) {
-      vecT h[CB][MAXRB];
-#pragma unroll
-      for (int j = 0; j < CB; ++j) {
-        const T* col = He + static_cast<long>(m) * (cfirst + j);
-#pragma unroll
-        for (int rb = 0; rb < MAXRB; ++rb) {
-          const int r = VW * (lane + 64 * rb);
-          if (r < m) h[j][rb] = *reinterpret_cast<const vecT*>(col + r);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < CB; ++j) {
-        const double vc = ve[cfirst + j];
-#pragma unroll
-        for (int rb = 0; rb < MAXRB; ++rb) {
-          const int r = VW * (lane + 64 * rb);
-          if (r < m)
-#pragma unroll
-            for (int q = 0; q < VW; ++q) acc[rb][q] = fma(blk_val(h[j][rb][q]), vc, acc[rb][q]);
-        }
-      }
-    }
-  }
-  for (int c = cfirst; c < c1; ++c) {
-    const double vc = ve[c];
-    const T* col = He + static_cast<long>(m) * c;
-#pragma unroll
-    for (int rb = 0; rb < MAXRB; ++rb) {
-      const int r = VW * (lane + 64 * rb);
-      if (rb < nrb && r < m) {
-        const vecT h = *reinterpret_cast<const vecT*>(col + r);
-#pragma unroll
-        for (int q = 0; q < VW; ++q) acc[rb][q] = fma(blk_val(h[q]), vc, acc[rb][q]);
-      }
-    }
-  }
-#pragma unroll
-  for (int rb = 0; rb < MAXRB; ++rb) {
-    const int r = VW * (lane + 64 * rb);
-    if (rb < nrb && r < m)
-#pragma unroll
-      for (int q = 0; q < VW; ++q) red[wave * m + r + q] = acc[rb][q];
-  }
-  __syncthreads();
-  for (int r = tid; r < m; r += 256)
-    we[e * m + r] = ((red[r] + red[m + r]) + red[2 * m + r]) + red[3 * m + r];
-}
-
-// The same product for small trace blocks (m <= 96, e.g. 2D elements): one thread per row
-// of one element, the rows of consecutive elements in consecutive lanes, FP64 accumulation
-// over the columns in order.  emask/einst (optional): elements of an instance whose mask is 0
-// only write zeros (instances that have left a batched GMRES).
-template <typename T>
-__global__ __launch_bounds__(256) void k_matvec_small(Dims d, const T* H, const int* elemcon, const double* v,
-                                                      double* we, const int* einst, const double* emask) {
-  const int m = d.m, ncu = d.ncu, ndf = d.ndf;
-  const long q = blockIdx.x * 256L + threadIdx.x;
-  if (q >= static_cast<long>(m) * d.ne) return;
-  const long e = q / m;
-  const int r = static_cast<int>(q % m);
-  if (emask && einst && emask[einst[e]] == 0.0) {
-    we[q] = 0.0;
-    return;
-  }
-  const T* He = H + e * static_cast<long>(m) * m + r;
-  const int* ec = elemcon + ndf * e;
-  double acc = 0.0;
-  for (int c = 0; c < m; ++c)
-    acc = fma(blk_val(He[static_cast<long>(m) * c]), v[(c % ncu) + ncu * static_cast<long>(ec[c / ncu])],
-              acc);
-  we[q] = acc;
-}
-
 // hdgGetDUDG (matvec.cpp:219-238): du_e = Ru_e + DinvF_e * x_e.  One workgroup per element: the
 // element's trace values x_e are gathered into LDS once, then one thread per row reads DinvF_e
 // along its columns (the sum runs over t in order).
@@ -3300,33 +3179,6 @@ void bj_apply(const Dims& d, const T* BE, const double* x, double* y, hipStream_
 }
 
 template <typename T>
-void matvec_elem(const Dims& d, const T* H, const int* elemcon, const double* v, double* we, hipStream_t s,
-                 const int* einst, const double* emask) {
-  if (d.m > 1024) throw Error(5, "element trace block larger than 1024");
-  if (d.m <= MATVEC_SMALL_M) {
-    k_matvec_small<T><<<nblocks(static_cast<long>(d.m) * d.ne, 256), 256, 0, s>>>(d, H, elemcon, v, we, einst,
-                                                                                   emask);
-    EXA_HIP(hipGetLastError());
-    return;
-  }
-  size_t shm = static_cast<size_t>(5) * d.m * sizeof(double);
-  constexpr int VMAX = 16 / sizeof(T);  // 16-byte loads: 2 doubles, 4 floats or 8 BF16 per lane
-  if (d.m % VMAX == 0) {
-    const int nrb = (d.m + 64 * VMAX - 1) / (64 * VMAX);
-    if (nrb == 2) k_matvec_elem<T, VMAX, 2><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
-    else if (nrb == 3) k_matvec_elem<T, VMAX, 3><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
-    else k_matvec_elem<T, VMAX, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
-  } else if (sizeof(T) == 2 && d.m % 4 == 0) {  // BF16 blocks: 8-byte loads
-    k_matvec_elem<T, 4, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
-  } else if (d.m % 2 == 0) {
-    k_matvec_elem<T, 2, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
-  } else {
-    k_matvec_elem<T, 1, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
-  }
-  EXA_HIP(hipGetLastError());
-}
-
-template <typename T>
 void dudg(const Dims& d, const double* RuS, const T* DinvF, const int* elemcon, const double* x,
           double* du, hipStream_t s) {
   if (d.ne <= 0) return;
@@ -4012,12 +3864,6 @@ void seg_gemv_cols(const SegMap& m, double* x, const double* V, long ldv, int k,
 
 template void bj_apply<double>(const Dims&, const double*, const double*, double*, hipStream_t, const double*);
 template void bj_apply<float>(const Dims&, const float*, const double*, double*, hipStream_t, const double*);
-template void matvec_elem<double>(const Dims&, const double*, const int*, const double*, double*, hipStream_t,
-                                  const int*, const double*);
-template void matvec_elem<float>(const Dims&, const float*, const int*, const double*, double*, hipStream_t,
-                                 const int*, const double*);
-template void matvec_elem<unsigned short>(const Dims&, const unsigned short*, const int*, const double*, double*,
-                                          hipStream_t, const int*, const double*);
 template void dudg<double>(const Dims&, const double*, const double*, const int*, const double*, double*,
                            hipStream_t);
 template void dudg<float>(const Dims&, const double*, const float*, const int*, const double*, double*,

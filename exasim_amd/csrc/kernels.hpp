@@ -242,9 +242,6 @@ template <typename T>
 void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Y, double* Xo,
                 double* out, hipStream_t s, const double* act = nullptr);
 
-// trace blocks up to this size use the one-thread-per-row matvec
-constexpr int MATVEC_SMALL_M = 96;
-
 // ---- vector kernels (results stay on the device) ----
 int dot_partials_count(long n);
 void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out,

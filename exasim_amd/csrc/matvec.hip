@@ -1,0 +1,236 @@
+// matvec.hip -- the element products of the condensed operator and of the inverted Schwarz blocks
+// (hdgMatVec's element part, backend/Discretization/matvec.cpp:377-380).
+#include "blkval.hpp"
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace exa {
+
+namespace {
+
+// hdgMatVec element part (matvec.cpp:377-380): we_e = H_e * v_e with v_e gathered
+// through elemcon.  One workgroup per element; each of the 4 waves owns a
+// quarter of the columns, lanes own VW consecutive rows (16-byte vector loads of
+// the column), accumulation is FP64, and the four partial sums are added in LDS
+// in a fixed order.
+// NRB > 0: exactly NRB row blocks of 64 VW rows (m > 64 VW (NRB - 1)), with CB columns' loads
+// issued before their FMAs (more bytes in flight per wave; a row's FMAs still run over the columns
+// in order); NRB = 0: any m <= 1024, one column at a time.
+template <typename T, int VW, int NRB>
+__global__ __launch_bounds__(256) void k_matvec_elem(Dims d, const T* H, const int* elemcon,
+                                                     const double* v, double* we, const int* einst,
+                                                     const double* emask) {
+  typedef T vecT __attribute__((ext_vector_type(VW)));
+  constexpr int MAXRB = NRB > 0 ? NRB : (1024 + 64 * VW - 1) / (64 * VW);  // m <= 1024
+  constexpr int CB = NRB > 0 ? (sizeof(T) <= 4 ? 4 : 2) : 1;
+  const int m = d.m, ncu = d.ncu, ndf = d.ndf;
+  const long e = blockIdx.x;
+  if (emask && einst && emask[einst[e]] == 0.0) {  // block-uniform: the element's instance is inactive
+    for (int r = threadIdx.x; r < m; r += 256) we[e * m + r] = 0.0;
+    return;
+  }
+  extern __shared__ double sm[];
+  double* ve = sm;          // m
+  double* red = sm + m;     // 4*m
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int t = tid; t < m; t += 256)
+    ve[t] = v[(t % ncu) + ncu * static_cast<long>(elemcon[t / ncu + ndf * e])];
+  __syncthreads();
+  const int cper = (m + 3) / 4;
+  const int c0 = wave * cper, c1 = min(m, c0 + cper);
+  const int nrb = (m + 64 * VW - 1) / (64 * VW);
+  double acc[MAXRB][VW];
+#pragma unroll
+  for (int rb = 0; rb < MAXRB; ++rb)
+#pragma unroll
+    for (int q = 0; q < VW; ++q) acc[rb][q] = 0.0;
+  const T* He = H + e * static_cast<long>(m) * m;
+  int cfirst = c0;
+  if (CB > 1) {
+    for (; cfirst + CB <= c1; cfirst += CB) {
+      vecT h[CB][MAXRB];
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        const T* col = He + static_cast<long>(m) * (cfirst + j);
+#pragma unroll
+        for (int rb = 0; rb < MAXRB; ++rb) {
+          const int r = VW * (lane + 64 * rb);
+          if (r < m) h[j][rb] = *reinterpret_cast<const vecT*>(col + r);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < CB; ++j) {
+        const double vc = ve[cfirst + j];
+#pragma unroll
+        for (int rb = 0; rb < MAXRB; ++rb) {
+          const int r = VW * (lane + 64 * rb);
+          if (r < m)
+#pragma unroll
+            for (int q = 0; q < VW; ++q) acc[rb][q] = fma(blk_val(h[j][rb][q]), vc, acc[rb][q]);
+        }
+      }
+    }
+  }
+  for (int c = cfirst; c < c1; ++c) {
+    const double vc = ve[c];
+    const T* col = He + static_cast<long>(m) * c;
+#pragma unroll
+    for (int rb = 0; rb < MAXRB; ++rb) {
+      const int r = VW * (lane + 64 * rb);
+      if (rb < nrb && r < m) {
+        const vecT h = *reinterpret_cast<const vecT*>(col + r);
+#pragma unroll
+        for (int q = 0; q < VW; ++q) acc[rb][q] = fma(blk_val(h[q]), vc, acc[rb][q]);
+      }
+    }
+  }
+#pragma unroll
+  for (int rb = 0; rb < MAXRB; ++rb) {
+    const int r = VW * (lane + 64 * rb);
+    if (rb < nrb && r < m)
+#pragma unroll
+      for (int q = 0; q < VW; ++q) red[wave * m + r + q] = acc[rb][q];
+  }
+  __syncthreads();
+  for (int r = tid; r < m; r += 256)
+    we[e * m + r] = ((red[r] + red[m + r]) + red[2 * m + r]) + red[3 * m + r];
+}
+
+// The same product for trace blocks whose column fits one wave's vector loads (m <= 64 VW: 2D
+// elements and low-order 3D ones).  Bound by reading H.  WPE waves share an element and split its
+// columns; within a wave, m / VW lanes hold the rows of a column and G = 64 VW / m columns are read
+// side by side, so a wave's 16-byte loads cover G m consecutive entries, and U of these loads are in
+// flight before the first FMA.  At m = 96, FP64, 2025 elements: 24 us = 6.2 TB/s (one thread per row,
+// reading single entries with one load in flight, took 69 us); m = 192, BF16, 1864 elements: 23 us (the
+// row-block kernel, with 24 of 64 lanes reading, 38 us).  Every sum's order is fixed
+// by m and the storage alone, so an instance's products do not depend on the batch it is in.
+// emask/einst (optional): elements of an instance whose mask is 0 only write zeros (instances that
+// have left a batched GMRES).
+template <typename T, int VW, int WPE>
+__global__ __launch_bounds__(256) void k_matvec_small(Dims d, const T* H, const int* elemcon, const double* v,
+                                                      double* we, const int* einst, const double* emask) {
+  typedef T vecT __attribute__((ext_vector_type(VW)));
+  constexpr int EPB = 4 / WPE;  // elements of the workgroup
+  constexpr int U = 8;
+  extern __shared__ double sm[];
+  const int m = d.m, ncu = d.ncu, ndf = d.ndf;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int sub = wave / WPE, part = wave % WPE;
+  const int NL = m / VW, G = 64 / NL;
+  const long e = blockIdx.x * static_cast<long>(EPB) + sub;
+  const bool on = e < d.ne && !(emask && einst && emask[einst[e]] == 0.0);
+  double* ve = sm + sub * (1 + WPE * G) * m;  // m
+  double* red = ve + m;                       // WPE G m
+  const int te = tid - sub * (64 * WPE);
+  if (on)
+    for (int t = te; t < m; t += 64 * WPE) ve[t] = v[(t % ncu) + ncu * static_cast<long>(elemcon[t / ncu + ndf * e])];
+  __syncthreads();
+  const int rg = lane % NL, cg = lane / NL;
+  if (on && cg < G) {
+    const int cper = (m + WPE - 1) / WPE;
+    const int c0 = part * cper, c1 = min(m, c0 + cper);
+    const T* He = H + e * static_cast<long>(m) * m + VW * rg;
+    double acc[VW];
+#pragma unroll
+    for (int q = 0; q < VW; ++q) acc[q] = 0.0;
+    int cb = c0;
+    for (; cb + U * G <= c1; cb += U * G) {
+      vecT h[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j)
+        h[j] = *reinterpret_cast<const vecT*>(He + static_cast<long>(m) * (cb + cg + G * j));
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const double vc = ve[cb + cg + G * j];
+#pragma unroll
+        for (int q = 0; q < VW; ++q) acc[q] = fma(blk_val(h[j][q]), vc, acc[q]);
+      }
+    }
+    if (cb < c1) {  // the last round: columns past the part's end reread its last one, unused
+      vecT h[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const int c = min(cb + cg + G * j, c1 - 1);
+        h[j] = *reinterpret_cast<const vecT*>(He + static_cast<long>(m) * c);
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const int c = cb + cg + G * j;
+        if (c < c1) {
+          const double vc = ve[c];
+#pragma unroll
+          for (int q = 0; q < VW; ++q) acc[q] = fma(blk_val(h[j][q]), vc, acc[q]);
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < VW; ++q) red[(part * G + cg) * m + VW * rg + q] = acc[q];
+  }
+  __syncthreads();
+  if (e < d.ne)
+    for (int t = te; t < m; t += 64 * WPE) {
+      double s = 0.0;
+      if (on)
+        for (int g = 0; g < WPE * G; ++g) s += red[g * m + t];
+      we[e * m + t] = s;
+    }
+}
+
+template <typename T, int VW, int WPE>
+void launch_small(const Dims& d, const T* H, const int* elemcon, const double* v, double* we, hipStream_t s,
+                  const int* einst, const double* emask) {
+  constexpr int EPB = 4 / WPE;
+  const int G = 64 / (d.m / VW);
+  const size_t shm = static_cast<size_t>(EPB) * (1 + WPE * G) * d.m * sizeof(double);
+  k_matvec_small<T, VW, WPE><<<(d.ne + EPB - 1) / EPB, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+}
+
+// A block of at most 8 KB keeps one wave per element (its few loads are one round anyway);
+// larger blocks split their columns over four.
+template <typename T, int VW>
+void small_vw(const Dims& d, const T* H, const int* elemcon, const double* v, double* we, hipStream_t s,
+              const int* einst, const double* emask) {
+  if (static_cast<size_t>(d.m) * d.m * sizeof(T) <= 8192) launch_small<T, VW, 1>(d, H, elemcon, v, we, s, einst, emask);
+  else launch_small<T, VW, 4>(d, H, elemcon, v, we, s, einst, emask);
+}
+
+}  // namespace
+
+template <typename T>
+void matvec_elem(const Dims& d, const T* H, const int* elemcon, const double* v, double* we, hipStream_t s,
+                 const int* einst, const double* emask) {
+  if (d.ne <= 0) return;
+  if (d.m > 1024) throw Error(5, "element trace block larger than 1024");
+  // the widest load (up to 16 bytes: 2 doubles, 4 floats, 8 BF16) that the rows of a column divide
+  // into: a column starts at a multiple of m, so the loads are aligned
+  constexpr int VMAX = 16 / sizeof(T);
+  const int vw = d.m % VMAX == 0 ? VMAX : (VMAX > 4 && d.m % 4 == 0) ? 4 : d.m % 2 == 0 ? 2 : 1;
+  size_t shm = static_cast<size_t>(5) * d.m * sizeof(double);
+  if (d.m <= 64 * vw) {
+    if (vw == VMAX) small_vw<T, VMAX>(d, H, elemcon, v, we, s, einst, emask);
+    else if (vw == 4) small_vw<T, 4>(d, H, elemcon, v, we, s, einst, emask);
+    else if (vw == 2) small_vw<T, 2>(d, H, elemcon, v, we, s, einst, emask);
+    else small_vw<T, 1>(d, H, elemcon, v, we, s, einst, emask);
+  } else if (vw == VMAX) {
+    const int nrb = (d.m + 64 * VMAX - 1) / (64 * VMAX);
+    if (nrb == 2) k_matvec_elem<T, VMAX, 2><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+    else if (nrb == 3) k_matvec_elem<T, VMAX, 3><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+    else k_matvec_elem<T, VMAX, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+  } else if (vw == 4) {  // BF16 blocks: 8-byte loads
+    k_matvec_elem<T, 4, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+  } else if (vw == 2) {
+    k_matvec_elem<T, 2, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+  } else {
+    k_matvec_elem<T, 1, 0><<<d.ne, 256, shm, s>>>(d, H, elemcon, v, we, einst, emask);
+  }
+  EXA_HIP(hipGetLastError());
+}
+
+template void matvec_elem<double>(const Dims&, const double*, const int*, const double*, double*, hipStream_t,
+                                  const int*, const double*);
+template void matvec_elem<float>(const Dims&, const float*, const int*, const double*, double*, hipStream_t,
+                                 const int*, const double*);
+template void matvec_elem<unsigned short>(const Dims&, const unsigned short*, const int*, const double*, double*,
+                                          hipStream_t, const int*, const double*);
+
+}  // namespace exa
