@@ -2,16 +2,14 @@
 // of small dense products, uequation.cpp:559-775's schurMatrix* / the reference's batched BLAS
 // calls) on gfx950, and the tile autotuner that picks each product's workgroup tile by measurement.
 //
-// Products of FP64 operands with M, N <= 32 run on a plain LDS-tiled kernel; all others on the
-// matrix cores (v_mfma_f64_16x16x4f64, or v_mfma_f32_16x16x4f32 for FP32 products), with one of
-// five workgroup tiles (BM x BN = 64x64, 32x64, 64x32, 128x64, 64x128; four waves, K staged through
-// LDS 32 at a time).  Every tile runs the same MFMA instruction over the same K order for each
+// Every product runs on the matrix cores (v_mfma_f64_16x16x4f64, or v_mfma_f32_16x16x4f32 for FP32
+// products) with one of five workgroup tiles (BM x BN = 64x64, 32x64, 64x32, 128x64, 64x128), made of
+// independent waves.  Every tile runs the same MFMA instruction over the same K order for each
 // output element, so the tiles give bitwise-identical results and differ only in speed: the tuner
 // times them on the first call of a product shape -- (M, N, K, the batch count's power of two,
-// FP32 or FP64 products, operand storage) -- on the caller's own operands (an accumulating product
-// writes into a scratch copy of its C while it is timed), keeps the fastest for the process and
-// launches it from then on.  No counterpart in the reference (its batched GEMMs
-// are library calls).
+// FP32 or FP64 products) -- on the caller's own operands (an accumulating product writes into a
+// scratch copy of its C while it is timed), keeps the fastest for the process and launches it from
+// then on.  No counterpart in the reference (its batched GEMMs are library calls).
 #include "kernels.hpp"
 #include "common.hpp"
 
@@ -31,277 +29,277 @@ namespace exa {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Batched FP64 GEMM: LDS-tiled, 256 threads, each thread a TM x TN micro-tile (M, N <= 32).
-// ---------------------------------------------------------------------------
-template <int BM, int BN, int BK, int TM, int TN>
-__global__ __launch_bounds__(256) void k_gemm(Gemm g, int tilesM) {
-  const int tile = blockIdx.x % tilesM;
-  const long b = blockIdx.x / tilesM;
-  const int b0 = static_cast<int>(b % g.nb0);
-  const long t1 = b / g.nb0;
-  const int b1 = static_cast<int>(t1 % g.nb1);
-  const int b2 = static_cast<int>(t1 / g.nb1);
-  const long a0 = g.iA ? g.iA[b0] : b0, bb0 = g.iB ? g.iB[b0] : b0, c0 = g.iC ? g.iC[b0] : b0;
-  const double* A = g.A + g.sA0 * a0 + g.sA1 * b1 + g.sA2 * b2;
-  const double* B = g.B + g.sB0 * bb0 + g.sB1 * b1 + g.sB2 * b2;
-  double* C = g.C + g.sC0 * c0 + g.sC1 * b1 + g.sC2 * b2;
-  const int row0 = tile * BM, col0 = blockIdx.y * BN;
-  __shared__ double As[BK][BM + 1];
-  __shared__ double Bs[BK][BN + 1];
-  const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-  double acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = 0.0;
-  for (int k0 = 0; k0 < g.K; k0 += BK) {
-    for (int idx = threadIdx.x; idx < BM * BK; idx += 256) {
-      int r = idx % BM, kk = idx / BM;
-      int gr = row0 + r, gk = k0 + kk;
-      As[kk][r] = (gr < g.M && gk < g.K) ? A[gr + g.lda * gk] : 0.0;
-    }
-    for (int idx = threadIdx.x; idx < BK * BN; idx += 256) {
-      int kk = idx % BK, c = idx / BK;
-      int gk = k0 + kk, gc = col0 + c;
-      Bs[kk][c] = (gk < g.K && gc < g.N) ? B[gk + g.ldb * gc] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      double a[TM], bb[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = As[kk][tx + 16 * i];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bb[j] = Bs[kk][ty + 16 * j];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = fma(a[i], bb[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      int r = row0 + tx + 16 * i, c = col0 + ty + 16 * j;
-      if (r < g.M && c < g.N) {
-        double v = g.alpha * acc[i][j];
-        if (g.beta != 0.0) v = fma(g.beta, C[r + g.ldc * c], v);
-        C[r + g.ldc * c] = v;
-      }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Batched GEMM on the matrix cores.  Workgroup tile BM x BN, four waves in a 2 x 2 layout, each
-// wave (BM/2) x (BN/2) as (BM/32) x (BN/32) MFMA tiles of 16 x 16; K staged through LDS MG_BK at a
-// time with the next K-tile prefetched into registers.  Lane layout of the instruction: lane l
-// supplies A[l%16][l/16] and B[l/16][l%16] of a 16x4 / 4x16 step.
+// Batched GEMM on the matrix cores, operands straight from global memory.
+//
+// Each wave computes FM x FN MFMA tiles of 16 x 16 by itself: no LDS, no barrier.  A 16-deep K block
+// of both operands is held in registers while the next one's loads are in flight; the waves of one
+// product run side by side and share operands through the caches.  Lane l of a 16x16x4 step supplies
+// A[l%16][k] and B[k][l%16] with k = l/16 of the step; since a product's sum may take its K values in
+// any order, step s of a block uses k = 4 (l/16) + s, so that a lane's four B values are contiguous
+// and load as one vector.
+//
+// Bound by MFMA issue at the clock that the power limit leaves (counters of the 250 x 275 x 375 FP64
+// product: the matrix cores busy 71 % of the cycles at 1.9 GHz), small K by the traffic of C.  Against
+// the form with K tiles staged through LDS between two barriers, each on its best tile:
+//   250 x 275 x 375, batch 2400:   FP64 3.77 -> 2.72 ms (33 -> 46 TFLOP/s), FP32 1.99 -> 1.67 ms (62 -> 74)
+//   300 x 300 x 250, batch 1200:   FP64 1.94 -> 1.38 ms, FP32 1.10 -> 0.82 ms
+//   186 x 487 x 64, batch 1200:    FP64 0.76 -> 0.80 ms, FP32 0.47 -> 0.40 ms (reads and writes C)
+//   144 x 36 x 72, batch 8100:     FP64 0.62 -> 0.40 ms, FP32 0.35 -> 0.20 ms
+//   25 x 25 x 25, batch 25000:     FP64 117 -> 70 us
 // ---------------------------------------------------------------------------
 typedef double dbl4 __attribute__((ext_vector_type(4)));
 typedef float flt4 __attribute__((ext_vector_type(4)));
-constexpr int MG_BK = 32;
+constexpr int KB = 16;  // K block
 
-// LDS is fragment-major: element (row r, k) of the A tile sits at
-// (r/16)*16*MG_BK + k*16 + r%16, so the 64 lanes of one MFMA operand read 64
-// consecutive values (no bank conflicts); B likewise with its columns.
-__device__ inline int mg_off(int rc, int k) { return (rc >> 4) * (16 * MG_BK) + k * 16 + (rc & 15); }
-
-// One 16x16x4 step.  FP64: register i of lane l holds D[l/16 + 4i][l%16];
-// FP32 (inputs rounded to FP32, FP32 accumulation): D[4(l/16) + i][l%16].
-__device__ inline dbl4 mfma_step(double a, double b, dbl4 c) {
+// One 16x16x4 step.  FP64: register i of lane l holds D[l/16 + 4i][l%16]; FP32: D[4(l/16) + i][l%16].
+__device__ __forceinline__ dbl4 mfma_step(double a, double b, dbl4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
-__device__ inline flt4 mfma_step(float a, float b, flt4 c) {
+__device__ __forceinline__ flt4 mfma_step(float a, float b, flt4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ inline int mfma_row(double, int lk, int i) { return lk + 4 * i; }
-__device__ inline int mfma_row(float, int lk, int i) { return 4 * lk + i; }
+// The matrix row that row r of the A operand's tile holds: chosen so that register i of lane l is
+// row 4 (l/16) + i of the output tile in both types (four contiguous rows per lane).
+__device__ __forceinline__ int a_row(double, int r) { return 4 * (r & 3) + (r >> 2); }
+__device__ __forceinline__ int a_row(float, int r) { return r; }
 
-// Workgroup w is dispatched to XCD w % 8 (each XCD has its own L2).  The logical
-// tile id L = (w % 8) * (nwg / 8) + w / 8 gives every XCD a contiguous range of L,
-// and L runs over the M/N tiles of one batch entry before the next, so the tiles
-// that share an operand run together on one XCD and reuse it from its L2.
-constexpr int NXCD = 8;
+// four consecutive values at the alignment of one (global loads need no more)
+template <typename T> struct Vec4;
+template <> struct Vec4<double> {
+  typedef double type __attribute__((ext_vector_type(4), aligned(8)));
+};
+template <> struct Vec4<float> {
+  typedef float type __attribute__((ext_vector_type(4), aligned(4)));
+};
 
-// Operand storage: the double pointer, or the float one when the operand is stored in FP32.
+// operands in the product's type
+template <typename T> __device__ __forceinline__ T* gsel(double* d, float* f);
+template <> __device__ __forceinline__ double* gsel<double>(double* d, float*) { return d; }
+template <> __device__ __forceinline__ float* gsel<float>(double*, float* f) { return f; }
 template <typename T> __device__ __forceinline__ const T* gsel(const double* d, const float* f);
 template <> __device__ __forceinline__ const double* gsel<double>(const double* d, const float*) { return d; }
 template <> __device__ __forceinline__ const float* gsel<float>(const double*, const float* f) { return f; }
 
-// CT: MFMA type; TA, TB, TC: storage of A, B, C; BM x BN: the workgroup tile
-template <typename CT, typename TA, typename TB, typename TC, int BM, int BN>
-__global__ __launch_bounds__(256) void k_gemm_mfma(Gemm g, int tilesM, int tilesN, long ntiles) {
-  typedef CT acc4 __attribute__((ext_vector_type(4)));
-  constexpr int FM = BM / 32, FN = BN / 32;  // MFMA tiles per wave
-  const long nwg = static_cast<long>(gridDim.x);   // a multiple of NXCD
-  const long L = (blockIdx.x % NXCD) * (nwg / NXCD) + blockIdx.x / NXCD;
+// Workgroup w is dispatched to XCD w % 8 (each XCD has its own L2).  The logical
+// id (w % 8) * (nwg / 8) + w / 8 gives every XCD a contiguous range of tiles,
+// which run over the M/N tiles of one batch entry before the next, so the tiles
+// that share an operand run together on one XCD and reuse it from its L2.
+constexpr int NXCD = 8;
+
+// A workgroup of WM x WN waves; T: double or float throughout.  Two waves per SIMD (256 registers),
+// except for the FP64 4 x 4 tiles, whose accumulators and operand blocks take more.
+template <typename T, int FM, int FN, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) * FM * FN > 64 ? 1 : 2)))
+void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
+  typedef typename Vec4<T>::type v4;
+  typedef T acc4 __attribute__((ext_vector_type(4)));
+  const unsigned nwg = gridDim.x;  // a multiple of NXCD
+  const unsigned L = (blockIdx.x % NXCD) * (nwg / NXCD) + blockIdx.x / NXCD;
   if (L >= ntiles) return;
-  const int tpb = tilesM * tilesN;
-  const long b = L / tpb;
-  const int tt = static_cast<int>(L % tpb);
-  const int tile = tt % tilesM, tcol = tt / tilesM;
-  const int b0 = static_cast<int>(b % g.nb0);
-  const long t1 = b / g.nb0;
-  const int b1 = static_cast<int>(t1 % g.nb1);
-  const int b2 = static_cast<int>(t1 / g.nb1);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned tpb = tilesM * tilesN;
+  const unsigned b = L / tpb, tt = L - b * tpb;
+  const unsigned b0 = b % static_cast<unsigned>(g.nb0), t1 = b / static_cast<unsigned>(g.nb0);
+  const unsigned b1 = t1 % static_cast<unsigned>(g.nb1), b2 = t1 / static_cast<unsigned>(g.nb1);
+  const int M = g.M, N = g.N, K = g.K;
+  const int row0 = (tt % tilesM * WM + wave % WM) * (16 * FM), col0 = (tt / tilesM * WN + wave / WM) * (16 * FN);
+  if (row0 >= M || col0 >= N) return;
   const long a0 = g.iA ? g.iA[b0] : b0, bb0 = g.iB ? g.iB[b0] : b0, c0 = g.iC ? g.iC[b0] : b0;
-  const TA* A = gsel<TA>(g.A, g.Af) + g.sA0 * a0 + g.sA1 * b1 + g.sA2 * b2;
-  const TB* B = gsel<TB>(g.B, g.Bf) + g.sB0 * bb0 + g.sB1 * b1 + g.sB2 * b2;
-  TC* C = const_cast<TC*>(gsel<TC>(g.C, g.Cf)) + g.sC0 * c0 + g.sC1 * b1 + g.sC2 * b2;
-  const int row0 = tile * BM, col0 = tcol * BN;
-  // the K tiles of A and B; the output tile is staged in the same LDS afterwards when it fits in
-  // 48 KB (all FP32 tiles; the FP64 64x64, 32x64 and 64x32 tiles)
-  constexpr int CLD = BM + 1;  // leading dimension of the staged output tile
-  constexpr bool STAGE_C = static_cast<long>(BN) * CLD * sizeof(CT) <= 48 * 1024;
-  constexpr int NAB = (BM + BN) * MG_BK, NCS = STAGE_C ? BN * CLD : 0;
-  __shared__ CT smem[NAB > NCS ? NAB : NCS];
-  CT* As = smem;
-  CT* Bs = smem + BM * MG_BK;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wr = wave & 1, wc = wave >> 1;
-  // global -> register staging of element e = tid + 256 j: A row e % BM, k = e / BM;
-  // B k = e % MG_BK, column e / MG_BK
-  constexpr int NLA = BM * MG_BK / 256, NLB = BN * MG_BK / 256;
-  const int ar = tid % BM, ak = tid / BM;
-  const int bk = tid % MG_BK, bc = tid / MG_BK;
-  TA ra[NLA];
-  TB rb[NLB];
-  bool ma[NLA], mb[NLB];
-  // out-of-range elements read a clamped (valid) address and are zeroed when stored to
-  // LDS, so the loads need no branches and stay in flight through the MFMA loop
-  const bool rowok = row0 + ar < g.M;
-  const long arow = min(row0 + ar, g.M - 1);
-  auto load = [&](int k0) {
+  const T* A = gsel<T>(g.A, g.Af) + g.sA0 * a0 + g.sA1 * b1 + g.sA2 * b2;
+  const T* B = gsel<T>(g.B, g.Bf) + g.sB0 * bb0 + g.sB1 * b1 + g.sB2 * b2;
+  T* C = gsel<T>(g.C, g.Cf) + g.sC0 * c0 + g.sC1 * b1 + g.sC2 * b2;
+  const int li = lane & 15, lk = lane >> 4;
+  // Byte offsets of the lane's rows of A and columns of B, 32 bits each beside a uniform base.  Rows and
+  // columns past the end read the last one; their results are not written.
+  const unsigned lda = static_cast<unsigned>(g.lda);
+  const unsigned ka = lda * (4 * lk), kb = 4 * lk;
+  unsigned oa[FM], ob[FN];
 #pragma unroll
-    for (int j = 0; j < NLA; ++j) {
-      const int gk = k0 + ak + (256 / BM) * j;
-      ra[j] = A[arow + g.lda * min(gk, g.K - 1)];
-      ma[j] = rowok & (gk < g.K);
-    }
+  for (int i = 0; i < FM; ++i) oa[i] = (min(row0 + 16 * i + a_row(T(0), li), M - 1) + ka) * sizeof(T);
 #pragma unroll
-    for (int j = 0; j < NLB; ++j) {
-      const int gk2 = k0 + bk, gc = col0 + bc + (256 / MG_BK) * j;
-      rb[j] = B[min(gk2, g.K - 1) + g.ldb * static_cast<long>(min(gc, g.N - 1))];
-      mb[j] = (gk2 < g.K) & (gc < g.N);
-    }
-  };
+  for (int j = 0; j < FN; ++j)
+    ob[j] = (static_cast<unsigned>(g.ldb) * min(col0 + 16 * j + li, N - 1) + kb) * sizeof(T);
+  auto at_byte = [](const T* base, unsigned off) { return reinterpret_cast<const char*>(base) + off; };
   acc4 acc[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = acc4{0, 0, 0, 0};
-  load(0);
-  const int li = lane & 15, lk = lane >> 4;
-  for (int k0 = 0; k0 < g.K; k0 += MG_BK) {
+  // MFMA tiles of the wave that hold output (the others' loads are harmless, their products skipped)
+  const int fm = min(FM, (M - row0 + 15) / 16), fn = min(FN, (N - col0 + 15) / 16);
+  T av[2][FM][4];
+  v4 bv[2][FN];
+  auto load = [&](int buf, int k0) {
 #pragma unroll
-    for (int j = 0; j < NLA; ++j) As[mg_off(ar, ak + (256 / BM) * j)] = ma[j] ? static_cast<CT>(ra[j]) : CT(0);
+    for (int s = 0; s < 4; ++s) {
+      const T* Ak = A + g.lda * (k0 + s);
 #pragma unroll
-    for (int j = 0; j < NLB; ++j) Bs[mg_off(bc + (256 / MG_BK) * j, bk)] = mb[j] ? static_cast<CT>(rb[j]) : CT(0);
-    __syncthreads();
-    load(k0 + MG_BK);  // unconditional: past the end it reads clamped, unused values
+      for (int i = 0; i < FM; ++i) av[buf][i][s] = *reinterpret_cast<const T*>(at_byte(Ak, oa[i]));
+    }
+    const T* Bk = B + k0;
 #pragma unroll
-    for (int kk = 0; kk < MG_BK; kk += 4) {
-      const int kr = kk + lk;
-      CT av[FM], bv[FN];
+    for (int j = 0; j < FN; ++j) bv[buf][j] = *reinterpret_cast<const v4*>(at_byte(Bk, ob[j]));
+  };
+  // the products of the block in buffer buf, interleaved with the loads of the next one into the
+  // other (one load after every few products keeps both queues fed)
+  auto block = [&](int buf, int knext) {
+    load(buf ^ 1, knext);
 #pragma unroll
-      for (int i = 0; i < FM; ++i) av[i] = As[mg_off((BM / 2) * wr + 16 * i + li, kr)];
-#pragma unroll
-      for (int j = 0; j < FN; ++j) bv[j] = Bs[mg_off((BN / 2) * wc + 16 * j + li, kr)];
+    for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step(av[i], bv[j], acc[i][j]);
+        for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step(av[buf][i][s], bv[buf][j][s], acc[i][j]);
+    constexpr int NLOAD = 4 * FM + FN * (sizeof(T) == 8 ? 2 : 1), PER = 4 * FM * FN / NLOAD;
+#pragma unroll
+    for (int q = 0; q < NLOAD; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);   // one global load
+      __builtin_amdgcn_sched_group_barrier(0x8, PER, 0);  // PER products
     }
-    __syncthreads();
+    __builtin_amdgcn_sched_group_barrier(0x8, 4 * FM * FN - PER * NLOAD, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the same for a wave whose last MFMA tiles lie past the matrix: their products are skipped
+  auto block_edge = [&](int buf, int knext) {
+    load(buf ^ 1, knext);
+#pragma unroll
+    for (int j = 0; j < FN; ++j)
+      if (j < fn)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+          if (i < fm)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) acc[i][j] = mfma_step(av[buf][i][s], bv[buf][j][s], acc[i][j]);
+  };
+  // an accumulating product's C, read before the K loop where the registers allow (with few K blocks
+  // its latency would otherwise follow theirs)
+  constexpr bool EARLY_C = sizeof(T) * FM * FN <= 32;
+  const T alpha = static_cast<T>(g.alpha), beta = static_cast<T>(g.beta);
+  v4 cv[FM][FN];
+  auto load_c = [&](int i, int j) {
+    const int r = row0 + 16 * i + 4 * lk, c = col0 + 16 * j + li;
+    if (c < N && r + 4 <= M) cv[i][j] = *reinterpret_cast<const v4*>(C + r + g.ldc * c);
+  };
+  if (EARLY_C && beta != T(0)) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) load_c(i, j);
   }
-  if constexpr (STAGE_C) {
-    // the output tile through LDS (the K loop ended with a barrier): each column's rows are then
-    // read and written by consecutive threads, where the MFMA layout puts 16 columns in a store
-    CT* Cs = smem;
+  // A block's loads are always issued (past the end: the last block again, unused), so that the wait
+  // before the products counts only older loads.
+  const int nk = K / KB;
+  if (nk > 0) {
+    load(0, 0);
+    int t = 0;
+    if (fm == FM && fn == FN) {
+      for (; t + 2 <= nk; t += 2) {
+        block(0, KB * (t + 1));
+        block(1, KB * min(t + 2, nk - 1));
+      }
+      if (t < nk) block(0, KB * t);
+    } else {
+      for (; t + 2 <= nk; t += 2) {
+        block_edge(0, KB * (t + 1));
+        block_edge(1, KB * min(t + 2, nk - 1));
+      }
+      if (t < nk) block_edge(0, KB * t);
+    }
+  }
+  // the last K % 16 values, 4 per step (k = l/16 of the step; zeros past K)
+  const int kt = nk * KB;
+  if (kt < K) {
+    T at[4][FM], bt[4][FN];
 #pragma unroll
-    for (int ti = 0; ti < FM; ++ti)
+    for (int s = 0; s < 4; ++s)
+      if (kt + 4 * s < K) {
+        const int k = kt + 4 * s + lk, kc = min(k, K - 1);
 #pragma unroll
-      for (int tj = 0; tj < FN; ++tj)
+        for (int i = 0; i < FM; ++i) {
+          const T x = *reinterpret_cast<const T*>(at_byte(A, oa[i] + (lda * kc - ka) * unsigned(sizeof(T))));
+          at[s][i] = k < K ? x : T(0);
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          Cs[((BN / 2) * wc + 16 * tj + li) * CLD + (BM / 2) * wr + 16 * ti + mfma_row(CT(0), lk, i)] = acc[ti][tj][i];
-    __syncthreads();
-    for (int idx = tid; idx < BM * BN; idx += 256) {
-      const int rl = idx % BM, cl = idx / BM;
-      const int r = row0 + rl, c = col0 + cl;
-      if (r < g.M && c < g.N) {
-        double v = g.alpha * static_cast<double>(Cs[cl * CLD + rl]);
-        if (g.beta != 0.0) v = fma(g.beta, static_cast<double>(C[r + g.ldc * static_cast<long>(c)]), v);
-        C[r + g.ldc * static_cast<long>(c)] = static_cast<TC>(v);
+        for (int j = 0; j < FN; ++j) {
+          const T x = *reinterpret_cast<const T*>(at_byte(B, ob[j] + (kc - kb) * unsigned(sizeof(T))));
+          bt[s][j] = k < K ? x : T(0);
+        }
+      }
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      if (kt + 4 * s < K)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step(at[s][i], bt[s][j], acc[i][j]);
+  }
+#pragma unroll
+  for (int i = 0; i < FM; ++i)
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int r = row0 + 16 * i + 4 * lk, c = col0 + 16 * j + li;
+      if (c >= N || r >= M) continue;
+      T* p = C + r + g.ldc * c;
+      if (r + 4 <= M) {
+        v4 x;
+        if (beta != T(0)) {
+          if (!EARLY_C) load_c(i, j);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) x[q] = fma(beta, cv[i][j][q], alpha * acc[i][j][q]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) x[q] = alpha * acc[i][j][q];
+        }
+        *reinterpret_cast<v4*>(p) = x;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+          if (r + q < M) p[q] = beta != T(0) ? fma(beta, p[q], alpha * acc[i][j][q]) : alpha * acc[i][j][q];
       }
     }
-  } else {
-#pragma unroll
-    for (int ti = 0; ti < FM; ++ti)
-#pragma unroll
-      for (int tj = 0; tj < FN; ++tj)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = row0 + (BM / 2) * wr + 16 * ti + mfma_row(CT(0), lk, i);
-          const int c = col0 + (BN / 2) * wc + 16 * tj + li;
-          if (r < g.M && c < g.N) {
-            double v = g.alpha * static_cast<double>(acc[ti][tj][i]);
-            if (g.beta != 0.0) v = fma(g.beta, static_cast<double>(C[r + g.ldc * static_cast<long>(c)]), v);
-            C[r + g.ldc * static_cast<long>(c)] = static_cast<TC>(v);
-          }
-        }
-  }
 }
 
 // ---------------------------------------------------------------------------
-// Launchers: one per (MFMA type, operand storage, tile)
+// Launchers: one per (type, tile).  wrows, wcols: the rows and columns of a tile that one wave holds.
 // ---------------------------------------------------------------------------
 struct TileShape {
-  int bm, bn;
+  int bm, bn, wrows, wcols;
 };
 constexpr int NTILE = 5;
-constexpr TileShape TILES[NTILE] = {{64, 64}, {32, 64}, {64, 32}, {128, 64}, {64, 128}};
+constexpr TileShape TILES[NTILE] = {{64, 64, 64, 64}, {32, 64, 32, 32}, {64, 32, 64, 32}, {128, 64, 64, 32},
+                                    {64, 128, 32, 64}};
 
 typedef void (*MfmaLaunch)(const Gemm&, hipStream_t);
 
-template <typename CT, typename TA, typename TB, typename TC, int BM, int BN>
+template <typename T, int FM, int FN, int WM, int WN>
 void launch_mfma(const Gemm& g, hipStream_t s) {
+  constexpr int BM = 16 * FM * WM, BN = 16 * FN * WN;
   const long batch = static_cast<long>(g.nb0) * g.nb1 * g.nb2;
   const int tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN;
   const long ntiles = static_cast<long>(tm) * tn * batch;
   const long nwg = (ntiles + NXCD - 1) / NXCD * NXCD;
   if (nwg > 0x7fffffffL) throw Error(5, "GEMM batch too large for one launch");
-  k_gemm_mfma<CT, TA, TB, TC, BM, BN><<<static_cast<unsigned>(nwg), 256, 0, s>>>(g, tm, tn, ntiles);
+  k_gemm<T, FM, FN, WM, WN><<<static_cast<unsigned>(nwg), 64 * WM * WN, 0, s>>>(g, tm, tn,
+                                                                                 static_cast<unsigned>(ntiles));
 }
 
-template <typename CT, typename TA, typename TB, typename TC>
+template <typename T>
 constexpr std::array<MfmaLaunch, NTILE> tile_launchers() {
-  return {launch_mfma<CT, TA, TB, TC, 64, 64>, launch_mfma<CT, TA, TB, TC, 32, 64>,
-          launch_mfma<CT, TA, TB, TC, 64, 32>, launch_mfma<CT, TA, TB, TC, 128, 64>,
-          launch_mfma<CT, TA, TB, TC, 64, 128>};
+  return {launch_mfma<T, 4, 4, 1, 1>, launch_mfma<T, 2, 2, 1, 2>, launch_mfma<T, 4, 2, 1, 1>,
+          launch_mfma<T, 4, 2, 2, 2>, launch_mfma<T, 2, 4, 2, 2>};
 }
 
-// [fp32][storage code: A float 1, B float 2, C float 4][tile]
-template <typename CT>
-std::array<std::array<MfmaLaunch, NTILE>, 8> storage_launchers() {
-  return {tile_launchers<CT, double, double, double>(), tile_launchers<CT, float, double, double>(),
-          tile_launchers<CT, double, float, double>(),  tile_launchers<CT, float, float, double>(),
-          tile_launchers<CT, double, double, float>(),  tile_launchers<CT, float, double, float>(),
-          tile_launchers<CT, double, float, float>(),   tile_launchers<CT, float, float, float>()};
-}
-
-MfmaLaunch mfma_launcher(int fp32, int store, int tile) {
-  static const auto f64 = storage_launchers<double>();
-  static const auto f32 = storage_launchers<float>();
-  return fp32 ? f32[store][tile] : f64[store][tile];
+MfmaLaunch mfma_launcher(int fp32, int tile) {
+  static constexpr auto f64 = tile_launchers<double>();
+  static constexpr auto f32 = tile_launchers<float>();
+  return fp32 ? f32[tile] : f64[tile];
 }
 
 // ---------------------------------------------------------------------------
 // The autotuner
 // ---------------------------------------------------------------------------
-typedef std::tuple<int, int, int, int, int, int, int> TuneKey;  // device, M, N, K, log2 batch, fp32, store
+typedef std::tuple<int, int, int, int, int, int, int> TuneKey;  // device, M, N, K, log2 batch, fp32, storage
 struct TuneEntry {
   int tile = 0;
   long batch = 0;  // products in the timed call
@@ -344,15 +342,15 @@ bool rerunnable(const Gemm& g) {
   return c != a && c != b;
 }
 
-// A product computed in place (C is B, as the LU's X = T^{-1} X) is correct only when one workgroup
-// holds all rows of its columns (BM >= M: every row of B is read before any row of C is written);
-// C is A likewise needs BN >= N.
+// A product computed in place (C is B, as the LU's X = T^{-1} X) is correct only when one wave
+// holds all rows of its columns (every row of B is read before any row of C is written);
+// C is A likewise needs all columns in one wave.
 bool tile_ok(const Gemm& g, int t) {
   const void* c = g.Cf ? static_cast<const void*>(g.Cf) : static_cast<const void*>(g.C);
   const void* a = g.Af ? static_cast<const void*>(g.Af) : static_cast<const void*>(g.A);
   const void* b = g.Bf ? static_cast<const void*>(g.Bf) : static_cast<const void*>(g.B);
-  if (c == b && TILES[t].bm < g.M) return false;
-  if (c == a && TILES[t].bn < g.N) return false;
+  if (c == b && TILES[t].wrows < g.M) return false;
+  if (c == a && TILES[t].wcols < g.N) return false;
   return true;
 }
 
@@ -372,7 +370,7 @@ int pick_tile(const Gemm& g, int store, long batch, hipStream_t s) {
   const int mode = tune_override() >= 0 ? tune_override() : tune_mode();
   if (mode == 0) return 0;
   const long work = static_cast<long>((g.M + 63) / 64) * ((g.N + 63) / 64) * batch;
-  if (work < 64) return 0;  // a launch of a few workgroups: launch latency decides, not the tile
+  if (work < 64) return tile_ok(g, 1) ? 1 : 0;  // a launch of a few workgroups: the smallest tile spreads widest
   int dev = 0;
   EXA_HIP(hipGetDevice(&dev));
   const TuneKey key{dev, g.M, g.N, g.K, log2_bucket(batch), g.fp32, store};
@@ -410,7 +408,7 @@ int pick_tile(const Gemm& g, int store, long batch, hipStream_t s) {
       ent.us[t] = -1.0f;  // not a candidate for this product
       continue;
     }
-    const MfmaLaunch f = mfma_launcher(g.fp32, store, t);
+    const MfmaLaunch f = mfma_launcher(g.fp32, t);
     f(gt, s);  // warm-up
     float fastest = 0.0f;
     for (int r = 0; r < 5; ++r) {
@@ -447,15 +445,14 @@ void gemm(const Gemm& g, hipStream_t s) {
   const long batch = static_cast<long>(g.nb0) * g.nb1 * g.nb2;
   if (batch <= 0) return;
   const int store = (g.Af ? 1 : 0) | (g.Bf ? 2 : 0) | (g.Cf ? 4 : 0);
-  if (g.M <= 32 && g.N <= 32 && store == 0) {
-    int tm = (g.M + 31) / 32, tn = (g.N + 31) / 32;
-    dim3 grid(static_cast<unsigned>(tm * batch), tn);
-    k_gemm<32, 32, 16, 2, 2><<<grid, 256, 0, s>>>(g, tm);
-  } else {
-    const int tile = pick_tile(g, store, batch, s);
-    // (a product timed on its own C has left its result there; one more run writes the same values)
-    mfma_launcher(g.fp32, store, tile)(g, s);
-  }
+  if (store != (g.fp32 ? 7 : 0)) throw Error(5, "GEMM operands must be stored in the product's type");
+  // the kernel's offsets within one A or B are 32-bit
+  if (g.lda * static_cast<long>(g.K) + g.M > 0x1fffffffL || g.ldb * static_cast<long>(g.N) + g.K > 0x1fffffffL)
+    throw Error(5, "GEMM operand too large");
+  // products of at most one 32 x 32 tile run on it; the tuner picks the others' tile
+  const int tile = g.M <= 32 && g.N <= 32 && forced_tile() < 0 ? 1 : pick_tile(g, store, batch, s);
+  // (a product timed on its own C has left its result there; one more run writes the same values)
+  mfma_launcher(g.fp32, tile)(g, s);
   EXA_HIP(hipGetLastError());
 }
 

@@ -30,8 +30,8 @@ struct Gemm {
   const int* iA = nullptr;
   const int* iB = nullptr;
   const int* iC = nullptr;
-  int fp32 = 0;  // 1: operands rounded to FP32, FP32 MFMA products and accumulation
-  // operands stored in FP32 (set instead of A / B / C, in any combination)
+  int fp32 = 0;  // 1: FP32 operands, products and accumulation
+  // the operands of an FP32 product (set instead of A / B / C)
   const float* Af = nullptr;
   const float* Bf = nullptr;
   float* Cf = nullptr;
@@ -43,7 +43,7 @@ void set_gemm_autotune(int mode);
 // the block-ILU(0) apply of FP32 / BF16 factors: 1 one wave per superelement, 0 the 256-thread
 // kernel, -1 follows EXA_BILU_WAVE (default 1)
 void set_bilu_wave(int mode);
-// every MFMA product on tile 0..4 (64x64 32x64 64x32 128x64 64x128), or -1: the tuner's choice
+// every product on tile 0..4 (64x64 32x64 64x32 128x64 64x128), or -1: the tuner's choice
 void set_gemm_tile(int tile);
 // one line per tuned shape: M N K log2(batch) fp32 storage chosen-tile and the microseconds of each tile
 std::string gemm_tuning_report();
@@ -238,6 +238,9 @@ void bilu_invert_diag(const Dims& d, const IluDev& I, int i, float* BE, int* inf
 void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const double* Ltmp, double* BE,
                 hipStream_t s);
 void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const float* Ltmp, float* BE, hipStream_t s);
+// Rh_e -= K_e u_e of the eb elements of a block: K [m, n, eb], u_e = U + su e (n values), Rh [m, eb]
+template <typename T>
+void trace_rhs(const Dims& d, int eb, const T* K, const T* U, long su, double* Rh, hipStream_t s);
 template <typename T>
 void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Y, double* Xo,
                 double* out, hipStream_t s, const double* act = nullptr);

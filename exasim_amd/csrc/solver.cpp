@@ -980,12 +980,8 @@ void Solver::assemble() {
       g.nb0 = eb; g.nb1 = 1; g.nb2 = 1;
       g.fp32 = precision;
       gemm(g, s);
-      g.N = 1;
-      g.fp32 = 0;
-      g.Cf = nullptr;
-      opB(g, aug.p, aug32.p, n * (n + m));
-      g.C = Rh.p + e0 * m; g.sC0 = m;
-      gemm(g, s);
+      if (f32) trace_rhs(d, eb, K32b, aug32.p + n * (n + m), augs, Rh.p + e0 * m, s);
+      else trace_rhs(d, eb, Kt.p, aug.p + n * (n + m), augs, Rh.p + e0 * m, s);
     }
     if (f32) {  // DinvF straight into FP32; FP32 copy of this block's LU factors of D'
       const long E0 = e0;
