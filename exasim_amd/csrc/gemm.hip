@@ -297,6 +297,173 @@ MfmaLaunch mfma_launcher(int fp32, int tile) {
 }
 
 // ---------------------------------------------------------------------------
+// The elimination of q from the trace rows, K = K0 + G M^-1 C and H = H0 - G M^-1 E, for the eb elements
+// of a block.  A trace row of face l couples only with the q nodes on that face, so its products run over
+// the npf nd rows of M^-1 C and M^-1 E at the face's nodes (frow) instead of all npe nd, with G stored
+// without its zeros: G[t + m (j + npf d + npf nd c)], t = k + ncu (i + npf l) a trace row, j the face node, d, c
+// the direction and component of q.  K0 = K0c[t + m (j + npf c)] and H0 = H0c[t + m (c + ncu j)] lie at the
+// face's own nodes (finv: face node of an element node, or -1) and are added where they are, so that K
+// and H are written once and read by nothing before.
+//
+// Bound by MFMA issue and the writes of K and H.  One workgroup per element and 16 FN columns of
+// M^-1 C or M^-1 E, which are staged in LDS once (STAGE) and serve every face and component: the rows a
+// face gathers lie far apart in global memory (read from there, each load touched up to 64 cache lines: 20^3
+// hexes, p = 4, two components, 15.4 ms FP64 and 10.3 ms FP32 per assembly against 11.8 and 7.1).  A wave takes FM x FN MFMA tiles of a (face, component) pair at a time, G straight
+// from global memory a 16-deep block ahead.  The dense products it replaces needed 3.9 times the MFMAs
+// there, and G, K and H cleared first.
+// ---------------------------------------------------------------------------
+template <typename T, int FM, int FN, bool STAGE>
+__global__ __launch_bounds__(256) void k_face_elim(FaceElim<T> f, int kpad, int tilesM, int tilesK, int tilesH) {
+  typedef typename Vec4<T>::type v4;
+  typedef T acc4 __attribute__((ext_vector_type(4)));
+  extern __shared__ double face_sm[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int li = lane & 15, lk = lane >> 4;
+  const int ncu = f.ncu, npf = f.npf, npe = f.npe, nd = f.nd, nfe = f.nfe, m = f.m;
+  const int M = ncu * npf, K = npf * nd, ndf = npf * nfe, ldb = npe * nd;
+  const int ldl = ldb | 1;  // column stride in LDS: odd, so that 16 columns meet different banks
+  const unsigned tiles = tilesK + tilesH;
+  const unsigned nwg = gridDim.x;  // a multiple of NXCD
+  const unsigned L = (blockIdx.x % NXCD) * (nwg / NXCD) + blockIdx.x / NXCD;
+  if (L >= tiles * static_cast<unsigned>(f.eb)) return;
+  const long e = L / tiles;
+  const int tcol = L % tiles;
+  const bool isH = tcol >= tilesK;
+  const int N = isH ? ndf : npe;
+  const int col0 = (isH ? tcol - tilesK : tcol) * (16 * FN);
+  const T* B = isH ? f.ME + (f.e0 + e) * static_cast<long>(ldb) * ndf : f.MC + (f.e0 + e) * static_cast<long>(ldb) * npe;
+  int* rows = reinterpret_cast<int*>(face_sm);  // [nfe][kpad]: rows of M^-1 C / M^-1 E, K of them and zeros
+  T* Bs = reinterpret_cast<T*>(face_sm + (nfe * kpad + 1) / 2);  // [16 FN][ldl]
+  for (int l = wave; l < nfe; l += 4)
+    for (int k = lane; k < kpad; k += 64) rows[l * kpad + k] = k < K ? f.frow[l * K + k] : 0;
+  if (STAGE)
+    for (int c = wave; c < 16 * FN && col0 + c < N; c += 4) {
+      const T* Bc = B + static_cast<long>(ldb) * (col0 + c);
+      for (int r = lane; r < ldb; r += 64) Bs[c * ldl + r] = Bc[r];
+    }
+  __syncthreads();
+  // columns past the end read the last one; their results are not written
+  unsigned ob[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    const int c = min(col0 + 16 * j + li, N - 1);
+    ob[j] = STAGE ? (c - col0) * ldl : static_cast<unsigned>(ldb) * c;
+  }
+  const unsigned lda = static_cast<unsigned>(m) * unsigned(sizeof(T));
+  for (int task = wave; task < nfe * ncu * tilesM; task += 4) {
+    const int row0 = task % tilesM * (16 * FM), cp = task / tilesM % ncu, l = task / tilesM / ncu;
+    const T* A = f.G + e * static_cast<long>(m) * K * ncu + static_cast<long>(m) * K * cp + l * M;
+    unsigned oa[FM];
+#pragma unroll
+    for (int i = 0; i < FM; ++i) oa[i] = min(row0 + 16 * i + a_row(T(0), li), M - 1) * unsigned(sizeof(T));
+    acc4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j) acc[i][j] = acc4{0, 0, 0, 0};
+    T av[2][FM][4];
+    auto load = [&](int buf, int k0) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const char* Ak = reinterpret_cast<const char*>(A) + lda * min(k0 + 4 * lk + s, K - 1);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) av[buf][i][s] = *reinterpret_cast<const T*>(Ak + oa[i]);
+      }
+    };
+    auto products = [&](int buf, int k0) {
+      const int4 r = *reinterpret_cast<const int4*>(rows + l * kpad + k0 + 4 * lk);
+      const int rr[4] = {r.x, r.y, r.z, r.w};
+      T bv[FN][4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) bv[j][s] = STAGE ? Bs[ob[j] + rr[s]] : B[ob[j] + rr[s]];
+      if (k0 + KB > K)  // values past K count as zeros in both operands
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const bool ok = k0 + 4 * lk + s < K;
+#pragma unroll
+          for (int i = 0; i < FM; ++i) av[buf][i][s] = ok ? av[buf][i][s] : T(0);
+#pragma unroll
+          for (int j = 0; j < FN; ++j) bv[j][s] = ok ? bv[j][s] : T(0);
+        }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step(av[buf][i][s], bv[j][s], acc[i][j]);
+    };
+    // kpad is K rounded up to whole 16-deep blocks; a block past the end reads the last one, unused
+    load(0, 0);
+    for (int k0 = 0; k0 < kpad; k0 += 2 * KB) {
+      load(1, min(k0 + KB, kpad - KB));
+      products(0, k0);
+      if (k0 + KB >= kpad) break;
+      load(0, min(k0 + 2 * KB, kpad - KB));
+      products(1, k0 + KB);
+    }
+    T* C = isH ? f.H + (f.e0 + e) * static_cast<long>(m) * m : f.K + e * static_cast<long>(m) * f.n;
+    const T* X = isH ? f.H0c + e * static_cast<long>(m) * M : f.K0c + e * static_cast<long>(m) * M;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+      const int c = col0 + 16 * j + li;
+      if (c >= N) continue;
+      long at, x0 = -1;  // column of K or H, and of its face-node part
+      if (isH) {
+        at = cp + ncu * c;
+        if (c / npf == l) x0 = cp + ncu * (c - npf * l);
+      } else {
+        at = c + npe * cp;
+        const int v = f.finv[l * npe + c];
+        if (v >= 0) x0 = v + npf * cp;
+      }
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int r = row0 + 16 * i + 4 * lk;
+        T* p = C + m * at + l * M + r;
+        const T* x = X + m * max(x0, 0L) + l * M + r;
+        T v[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          v[t] = isH ? -acc[i][j][t] : acc[i][j][t];
+          if (x0 >= 0 && r + t < M) v[t] += x[t];
+        }
+        if (r + 4 <= M) *reinterpret_cast<v4*>(p) = v4{v[0], v[1], v[2], v[3]};
+        else
+#pragma unroll
+          for (int t = 0; t < 3; ++t)
+            if (r + t < M) p[t] = v[t];
+      }
+    }
+  }
+}
+
+template <typename T, int FM, int FN, bool STAGE>
+void launch_face_elim(const FaceElim<T>& f, size_t lds, hipStream_t s) {
+  const int M = f.ncu * f.npf, kpad = (f.npf * f.nd + KB - 1) / KB * KB;
+  const int tm = (M + 16 * FM - 1) / (16 * FM), tk = (f.npe + 16 * FN - 1) / (16 * FN),
+            th = (f.npf * f.nfe + 16 * FN - 1) / (16 * FN);
+  const long nwg = (static_cast<long>(tk + th) * f.eb + NXCD - 1) / NXCD * NXCD;
+  if (nwg > 0x7fffffffL) throw Error(5, "element block too large for one launch");
+  k_face_elim<T, FM, FN, STAGE><<<static_cast<unsigned>(nwg), 256, lds, s>>>(f, kpad, tm, tk, th);
+}
+
+// The columns of a workgroup: as many 16-column tiles (4, 2 or 1) as 56 KB of LDS hold, so that two
+// workgroups or more share a CU; elements whose single tile takes more read M^-1 C and M^-1 E from memory.
+template <typename T, int FM>
+void face_elim_fm(const FaceElim<T>& f, hipStream_t s) {
+  const int kpad = (f.npf * f.nd + KB - 1) / KB * KB;
+  const size_t idx = static_cast<size_t>((f.nfe * kpad + 1) / 2) * sizeof(double);
+  const size_t col16 = 16 * sizeof(T) * static_cast<size_t>(f.npe * f.nd | 1);
+  constexpr size_t LIMIT = 56 * 1024;
+  if (idx + 4 * col16 <= LIMIT) launch_face_elim<T, FM, 4, true>(f, idx + 4 * col16, s);
+  else if (idx + 2 * col16 <= LIMIT) launch_face_elim<T, FM, 2, true>(f, idx + 2 * col16, s);
+  else if (idx + col16 <= LIMIT) launch_face_elim<T, FM, 1, true>(f, idx + col16, s);
+  else launch_face_elim<T, FM, 2, false>(f, idx, s);
+}
+
+// ---------------------------------------------------------------------------
 // The autotuner
 // ---------------------------------------------------------------------------
 typedef std::tuple<int, int, int, int, int, int, int> TuneKey;  // device, M, N, K, log2 batch, fp32, storage
@@ -455,6 +622,19 @@ void gemm(const Gemm& g, hipStream_t s) {
   mfma_launcher(g.fp32, tile)(g, s);
   EXA_HIP(hipGetLastError());
 }
+
+template <typename T>
+void face_elim(const FaceElim<T>& f, hipStream_t s) {
+  if (f.eb <= 0) return;
+  // a wave's rows: one, two or four MFMA tiles, by the rows of a face
+  const int M = f.ncu * f.npf;
+  if (M <= 16) face_elim_fm<T, 1>(f, s);
+  else if (M <= 32) face_elim_fm<T, 2>(f, s);
+  else face_elim_fm<T, 4>(f, s);
+  EXA_HIP(hipGetLastError());
+}
+template void face_elim<double>(const FaceElim<double>&, hipStream_t);
+template void face_elim<float>(const FaceElim<float>&, hipStream_t);
 
 void set_gemm_autotune(int mode) { tune_override() = mode; }
 

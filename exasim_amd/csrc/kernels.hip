@@ -1496,9 +1496,10 @@ __global__ void k_face_res(Dims d, AsmArgs a, int l, int nf1, T* ru, long ldru, 
 
 // Jacobian parts of face l: D/B += int phi_a phi_b fhI_uq, F += int phi_a phi_b fhI_uh,
 // K/G = int phi_a phi_b fhB_uq, H = int phi_a phi_b fhB_uh
-// (assembleMatrixBD/F/GK/H, kokkosimpl.h:1661-1730).
+// (assembleMatrixBD/F/GK/H, kokkosimpl.h:1661-1730).  K, G and H couple a face's trace rows with its own
+// nodes only and are stored without the zeros, in the layouts of FaceElim's K0c, G and H0c.
 template <typename T>
-__global__ void k_face_jac(Dims d, AsmArgs a, int l, T* aug, T* Bfull, T* Kt, T* Gfull, T* H) {
+__global__ void k_face_jac(Dims d, AsmArgs a, int l, T* aug, T* Bfull, T* K0c, T* Gc, T* H0c) {
   const int npf = d.npf, ngf = d.ngf, ncu = d.ncu, nc = d.nc, npe = d.npe, nd = d.nd;
   const int n = d.n, m = d.m;
   const int ncol = nc + ncu;
@@ -1526,17 +1527,17 @@ __global__ void k_face_jac(Dims d, AsmArgs a, int l, T* aug, T* Bfull, T* Kt, T*
   const long trow = k + ncu * (aa + npf * l);
   if (c < ncu) {
     aug[e * augs + pa + npe * k + static_cast<long>(n) * (pbn + npe * c)] += static_cast<T>(sI);
-    Kt[e * m * static_cast<long>(n) + trow + static_cast<long>(m) * (pbn + npe * c)] += static_cast<T>(sB);
+    K0c[e * m * static_cast<long>(d.ncf) + trow + static_cast<long>(m) * (bb + npf * c)] = static_cast<T>(sB);
   } else if (c < nc) {
     const int cq = c - ncu, cp = cq % ncu, dd = cq / ncu;
     const long col = pbn + npe * dd + static_cast<long>(npe) * nd * cp;
     Bfull[e * n * static_cast<long>(n) * nd + pa + npe * k + n * col] += static_cast<T>(sI);
-    Gfull[e * m * static_cast<long>(n) * nd + trow + m * col] += static_cast<T>(sB);
+    Gc[e * m * static_cast<long>(d.ncf) * nd + trow + m * (bb + npf * (dd + static_cast<long>(nd) * cp))] =
+        static_cast<T>(sB);
   } else {
     const int c2 = c - nc;
     aug[e * augs + pa + npe * k + static_cast<long>(n) * (n + c2 + ncu * (bb + npf * l))] += static_cast<T>(sI);
-    H[(a.e0 + e) * static_cast<long>(m) * m + trow + static_cast<long>(m) * (c2 + ncu * (bb + npf * l))] =
-        static_cast<T>(sB);
+    H0c[e * m * static_cast<long>(d.ncf) + trow + static_cast<long>(m) * (c2 + ncu * bb)] = static_cast<T>(sB);
   }
 }
 
@@ -1547,14 +1548,14 @@ __global__ void k_face_jac(Dims d, AsmArgs a, int l, T* aug, T* Bfull, T* Kt, T*
 // (p = aa + npf bb), formed on the matrix cores: F^T (fields x points) from LDS as the A
 // operand, each lane's Q entry computed from the shape tables in LDS as the B operand.  In
 // the accumulators 16 lanes hold 16 consecutive pairs of one field, so their updates of
-// D/B/F (aug, Bfull) and K/G/H land in a few rows of one column, as in k_face_jac.  The
+// D/B/F (aug, Bfull) and their K/G/H entries land in a few rows of one column, as in k_face_jac.  The
 // faces run in order l = 0 .. nfe-1 with a barrier between them: entries that two faces
 // share (D and B at the nodes of a common edge) are updated face by face, in that order.
 constexpr int FJ_THREADS = 512;
 
 template <typename T>
-__global__ __launch_bounds__(FJ_THREADS) void k_face_jac_elem(Dims d, AsmArgs a, T* aug, T* Bfull, T* Kt, T* Gfull,
-                                                              T* H) {
+__global__ __launch_bounds__(FJ_THREADS) void k_face_jac_elem(Dims d, AsmArgs a, T* aug, T* Bfull, T* K0c, T* Gc,
+                                                              T* H0c) {
   extern __shared__ double fj_sm[];
   const int npf = d.npf, ngf = d.ngf, ncu = d.ncu, nc = d.nc, npe = d.npe, nd = d.nd, nfe = d.nfe;
   const int n = d.n, m = d.m;
@@ -1578,9 +1579,9 @@ __global__ __launch_bounds__(FJ_THREADS) void k_face_jac_elem(Dims d, AsmArgs a,
   const long augs = a.augs;
   T* augE = aug + e * augs;
   T* BE = Bfull + e * static_cast<long>(n) * n * nd;
-  T* KE = Kt + e * static_cast<long>(m) * n;
-  T* GE = Gfull + e * static_cast<long>(m) * n * nd;
-  T* HE = H + (a.e0 + e) * static_cast<long>(m) * m;
+  T* KE = K0c + e * static_cast<long>(m) * d.ncf;
+  T* GE = Gc + e * static_cast<long>(m) * d.ncf * nd;
+  T* HE = H0c + e * static_cast<long>(m) * d.ncf;
   for (int l = 0; l < nfe; ++l) {
     const long pb = (e * nfe + l) * ngf;
     __syncthreads();  // the previous face's reads of Fs and its updates are done
@@ -1621,16 +1622,16 @@ __global__ __launch_bounds__(FJ_THREADS) void k_face_jac_elem(Dims d, AsmArgs a,
             const int k = fl % ncu, c = fl / ncu;
             const long trow = k + ncu * (aa + npf * l);
             if (c < ncu) {
-              if (bpart) KE[trow + static_cast<long>(m) * (pbn + npe * c)] += vt;
+              if (bpart) KE[trow + static_cast<long>(m) * (bb + npf * c)] = vt;
               else augE[pa + npe * k + static_cast<long>(n) * (pbn + npe * c)] += vt;
             } else if (c < nc) {
               const int cq = c - ncu, cp = cq % ncu, dd = cq / ncu;
               const long col = pbn + npe * dd + static_cast<long>(npe) * nd * cp;
-              if (bpart) GE[trow + m * col] += vt;
+              if (bpart) GE[trow + static_cast<long>(m) * (bb + npf * (dd + nd * cp))] = vt;
               else BE[pa + npe * k + n * col] += vt;
             } else {
               const long col = (c - nc) + ncu * (bb + npf * l);
-              if (bpart) HE[trow + static_cast<long>(m) * col] = vt;
+              if (bpart) HE[trow + static_cast<long>(m) * (c - nc + ncu * bb)] = vt;
               else augE[pa + npe * k + static_cast<long>(n) * (n + col)] += vt;
             }
           }
@@ -2982,28 +2983,28 @@ void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, float* ru, long 
 }
 
 template <typename T>
-void face_jac_t(const Dims& d, const AsmArgs& a, T* aug, T* Bfull, T* Kt, T* Gfull, T* H, hipStream_t s) {
+void face_jac_t(const Dims& d, const AsmArgs& a, T* aug, T* Bfull, T* K0c, T* Gc, T* H0c, hipStream_t s) {
   if (a.eb <= 0) return;
   const size_t lds = face_jac_elem_lds(d);
   if (lds <= 64000) {
-    k_face_jac_elem<T><<<a.eb, FJ_THREADS, lds, s>>>(d, a, aug, Bfull, Kt, Gfull, H);
+    k_face_jac_elem<T><<<a.eb, FJ_THREADS, lds, s>>>(d, a, aug, Bfull, K0c, Gc, H0c);
     EXA_HIP(hipGetLastError());
     return;
   }
   // face tables too large for LDS: one launch per local face (no two writes of a launch collide)
   long n1 = static_cast<long>(d.npf) * d.npf * d.ncu * (d.nc + d.ncu) * a.eb;
   for (int l = 0; l < d.nfe; ++l) {
-    k_face_jac<T><<<nblocks(n1, 256), 256, 0, s>>>(d, a, l, aug, Bfull, Kt, Gfull, H);
+    k_face_jac<T><<<nblocks(n1, 256), 256, 0, s>>>(d, a, l, aug, Bfull, K0c, Gc, H0c);
     EXA_HIP(hipGetLastError());
   }
 }
-void face_jac(const Dims& d, const AsmArgs& a, double* aug, double* Bfull, double* Kt, double* Gfull, double* H,
+void face_jac(const Dims& d, const AsmArgs& a, double* aug, double* Bfull, double* K0c, double* Gc, double* H0c,
               hipStream_t s) {
-  face_jac_t(d, a, aug, Bfull, Kt, Gfull, H, s);
+  face_jac_t(d, a, aug, Bfull, K0c, Gc, H0c, s);
 }
-void face_jac(const Dims& d, const AsmArgs& a, float* aug, float* Bfull, float* Kt, float* Gfull, float* H,
+void face_jac(const Dims& d, const AsmArgs& a, float* aug, float* Bfull, float* K0c, float* Gc, float* H0c,
               hipStream_t s) {
-  face_jac_t(d, a, aug, Bfull, Kt, Gfull, H, s);
+  face_jac_t(d, a, aug, Bfull, K0c, Gc, H0c, s);
 }
 
 void post_schur(const Dims& d, int e0, int eb, const double* aug, long augs, double* DinvF, double* RuS,

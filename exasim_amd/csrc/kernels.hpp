@@ -37,6 +37,22 @@ struct Gemm {
   float* Cf = nullptr;
 };
 void gemm(const Gemm& g, hipStream_t s);
+// K = K0 + G M^-1 C and H = H0 - G M^-1 E of the elements of a block (gemm.hip, k_face_elim)
+template <typename T>
+struct FaceElim {
+  int nd, ncu, npe, npf, nfe, n, m, e0, eb;
+  const int* frow;  // [npf nd, nfe] rows of M^-1 C and M^-1 E at the face nodes
+  const int* finv;  // [npe, nfe] face node of an element node, or -1
+  const T* G;       // [m, npf nd, ncu, eb]
+  const T* K0c;     // [m, npf ncu, eb]
+  const T* H0c;     // [m, ncu npf, eb]
+  const T* MC;      // [npe nd, npe, ne]
+  const T* ME;      // [npe nd, ndf, ne]
+  T* K;             // [m, n, eb]
+  T* H;             // [m, m, ne]
+};
+template <typename T>
+void face_elim(const FaceElim<T>& f, hipStream_t s);
 // the tile autotuner of gemm (gemm.hip): mode 1 times the workgroup tiles on the first call of each
 // product shape, 0 always takes the default tile, -1 follows EXA_GEMM_AUTOTUNE (default 1)
 void set_gemm_autotune(int mode);
@@ -159,11 +175,12 @@ void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, double* ru, long
               hipStream_t s);
 void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, float* ru, long ldru, double* Rh,
               hipStream_t s);
-// Jacobian parts of every face of the block's elements (face by face, in local order)
-void face_jac(const Dims& d, const AsmArgs& a, double* aug, double* Bfull, double* Kt, double* Gfull, double* H,
+// Jacobian parts of every face of the block's elements (face by face, in local order): added to D, F
+// (aug) and B; K, G and H written without their zeros (FaceElim's K0c, G and H0c)
+void face_jac(const Dims& d, const AsmArgs& a, double* aug, double* Bfull, double* K0c, double* Gc, double* H0c,
               hipStream_t s);
-// the same into FP32 D/B/F, K, G and H blocks
-void face_jac(const Dims& d, const AsmArgs& a, float* aug, float* Bfull, float* Kt, float* Gfull, float* H,
+// the same into FP32 blocks
+void face_jac(const Dims& d, const AsmArgs& a, float* aug, float* Bfull, float* K0c, float* Gc, float* H0c,
               hipStream_t s);
 void post_schur(const Dims& d, int e0, int eb, const double* aug, long augs, double* DinvF, double* RuS,
                 hipStream_t s);

@@ -240,6 +240,17 @@ void Solver::init(SolData& sol) {
   }
   seg_setup();
   perm.upload(mesh.perm, st, s);
+  {  // FaceElim's index tables of a local face: rows of M^-1 C / M^-1 E, and the inverse of perm
+    std::vector<int> fr(static_cast<size_t>(d.nfe) * d.npf * d.nd), fi(static_cast<size_t>(d.nfe) * d.npe, -1);
+    for (int l = 0; l < d.nfe; ++l)
+      for (int j = 0; j < d.npf; ++j) {
+        const int i = mesh.perm[j + d.npf * l];
+        for (int k = 0; k < d.nd; ++k) fr[j + d.npf * (k + d.nd * l)] = i + d.npe * k;
+        fi[i + d.npe * l] = j;
+      }
+    frow.upload(fr, st, s);
+    finv.upload(fi, st, s);
+  }
   elemcon.upload(conn.elemcon, st, s);
   bf.upload(mesh.bf, st, s);
   bface_h.clear();
@@ -594,7 +605,8 @@ void Solver::alloc_workspace() {
   const long n = d.n, m = d.m;
   const long pts = static_cast<long>(d.nd + 1) * d.ncu * d.nge + static_cast<long>(d.nd + 1) * d.ncu * d.nc * d.nge +
                    2L * (d.ncu + d.ncu * d.nc + d.ncu * d.ncu) * d.nfe * d.ngf;
-  const long blocks = n * augcols() + n * n * d.nd + m * n * d.nd + static_cast<long>(d.npe) * d.nge * d.ncu * d.nc;
+  const long face = m * d.ncf;  // one face-node block of the trace rows (K0, H0; G has nd of them)
+  const long blocks = n * augcols() + n * n * d.nd + face * (d.nd + 2) + static_cast<long>(d.npe) * d.nge * d.ncu * d.nc;
   const double per = precision ? 8.0 * pts + 4.0 * blocks : 8.0 * (pts + blocks + m * n);
   long cap = static_cast<long>(ws_budget_bytes / per);
   neb = static_cast<int>(std::max(1L, std::min<long>(d.ne, cap)));
@@ -602,21 +614,29 @@ void Solver::alloc_workspace() {
     aug.release();
     Bfull.release();
     Kt.release();
-    Gfull.release();
+    Gc.release();
+    K0c.release();
+    H0c.release();
     W.release();
     aug32.alloc(static_cast<size_t>(neb) * n * augcols());
     Bfull32.alloc(static_cast<size_t>(neb) * n * n * d.nd);
-    Gfull32.alloc(static_cast<size_t>(neb) * m * n * d.nd);
+    Gc32.alloc(static_cast<size_t>(neb) * face * d.nd);
+    K0c32.alloc(static_cast<size_t>(neb) * face);
+    H0c32.alloc(static_cast<size_t>(neb) * face);
     W32.alloc(static_cast<size_t>(neb) * d.npe * d.nge * d.ncu * d.nc);
   } else {
     aug32.release();
     Bfull32.release();
-    Gfull32.release();
+    Gc32.release();
+    K0c32.release();
+    H0c32.release();
     W32.release();
     aug.alloc(static_cast<size_t>(neb) * n * augcols());
     Bfull.alloc(static_cast<size_t>(neb) * n * n * d.nd);
     Kt.alloc(static_cast<size_t>(neb) * m * n);
-    Gfull.alloc(static_cast<size_t>(neb) * m * n * d.nd);
+    Gc.alloc(static_cast<size_t>(neb) * face * d.nd);
+    K0c.alloc(static_cast<size_t>(neb) * face);
+    H0c.alloc(static_cast<size_t>(neb) * face);
     W.alloc(static_cast<size_t>(neb) * d.npe * d.nge * d.ncu * d.nc);
   }
   rv.alloc(static_cast<size_t>(neb) * (d.nd + 1) * d.ncu * d.nge);
@@ -865,17 +885,8 @@ void Solver::assemble() {
     AsmArgs a = asm_args(e0, eb);
     float* K32b = f32 ? K32.p + static_cast<long>(e0) * m * n : nullptr;  // K of this block, in place
     tic(T_ASSEMBLY, &t0);
-    if (f32) {
-      EXA_HIP(hipMemsetAsync(aug32.p, 0, sizeof(float) * augs * eb, s));
-      EXA_HIP(hipMemsetAsync(K32b, 0, sizeof(float) * m * n * eb, s));
-      EXA_HIP(hipMemsetAsync(Gfull32.p, 0, sizeof(float) * m * n * nd * eb, s));
-    } else {
-      EXA_HIP(hipMemsetAsync(aug.p, 0, sizeof(double) * augs * eb, s));
-      EXA_HIP(hipMemsetAsync(Kt.p, 0, sizeof(double) * m * n * eb, s));
-      EXA_HIP(hipMemsetAsync(Gfull.p, 0, sizeof(double) * m * n * nd * eb, s));
-    }
-    if (f32) EXA_HIP(hipMemsetAsync(H32.p + e0 * m * m, 0, sizeof(float) * m * m * eb, s));
-    else EXA_HIP(hipMemsetAsync(H.p + e0 * m * m, 0, sizeof(double) * m * m * eb, s));
+    if (f32) EXA_HIP(hipMemsetAsync(aug32.p, 0, sizeof(float) * augs * eb, s));
+    else EXA_HIP(hipMemsetAsync(aug.p, 0, sizeof(double) * augs * eb, s));
     // volume terms
     vol_points(d, a, true, s);
     if (f32) {
@@ -917,8 +928,8 @@ void Solver::assemble() {
       if (f32) face_res(d, a, l, true, aug32.p + n * (n + m), augs, Rh.p, s);
       else face_res(d, a, l, true, aug.p + n * (n + m), augs, Rh.p, s);
     }
-    if (f32) face_jac(d, a, aug32.p, Bfull32.p, K32b, Gfull32.p, H32.p, s);
-    else face_jac(d, a, aug.p, Bfull.p, Kt.p, Gfull.p, H.p, s);
+    if (f32) face_jac(d, a, aug32.p, Bfull32.p, K0c32.p, Gc32.p, H0c32.p, s);
+    else face_jac(d, a, aug.p, Bfull.p, K0c.p, Gc.p, H0c.p, s);
     // eliminate q: D += B*MinvC, F -= B*MinvE, K += G*MinvC, H -= G*MinvE (uequation.cpp:614-681)
     {
       Gemm g{};
@@ -938,23 +949,10 @@ void Solver::assemble() {
       opC(g, aug.p, aug32.p, n * n);
       g.ldc = n * ncu; g.sC0 = n; g.sC1 = augs;
       gemm(g, s);
-      Gemm k{};
-      k.M = m; k.N = npe; k.K = npe * nd; k.alpha = 1.0; k.beta = 1.0;
-      opA(k, Gfull.p, Gfull32.p, 0);
-      k.lda = m; k.sA0 = m * npe * nd; k.sA1 = m * n * nd;
-      opB(k, MCs.p, MCs32.p, e0 * npe * nd * npe);
-      k.ldb = npe * nd; k.sB0 = 0; k.sB1 = npe * nd * npe;
-      opC(k, Kt.p, K32b, 0);
-      k.ldc = m; k.sC0 = m * npe; k.sC1 = m * n;
-      k.nb0 = static_cast<int>(ncu); k.nb1 = eb; k.nb2 = 1;
-      k.fp32 = precision;
-      gemm(k, s);
-      k.N = static_cast<int>(ndf); k.alpha = -1.0;
-      opB(k, MEs.p, MEs32.p, e0 * npe * nd * ndf);
-      k.sB1 = npe * nd * ndf;
-      opC(k, H.p, H32.p, e0 * m * m);
-      k.ldc = m * ncu; k.sC0 = m; k.sC1 = m * m;
-      gemm(k, s);
+      if (f32) face_elim(FaceElim<float>{d.nd, d.ncu, d.npe, d.npf, d.nfe, d.n, d.m, e0, eb, frow.p, finv.p, Gc32.p,
+                                         K0c32.p, H0c32.p, MCs32.p, MEs32.p, K32b, H32.p}, s);
+      else face_elim(FaceElim<double>{d.nd, d.ncu, d.npe, d.npf, d.nfe, d.n, d.m, e0, eb, frow.p, finv.p, Gc.p,
+                                      K0c.p, H0c.p, MCs.p, MEs.p, Kt.p, H.p}, s);
     }
     toc(T_ASSEMBLY, t0);
     // condense u: [D | F | Ru] -> [LU | D^{-1}F | D^{-1}Ru] (the mixed form in FP32, with the

@@ -77,7 +77,7 @@ struct Solver {
   PluginFns plugin_fns;
   DevBuf<double> uinf_d, pbuf;
   void load_plugin();
-  DevBuf<int> perm, elemcon, bf, f2e, info, ifirst;
+  DevBuf<int> perm, frow, finv, elemcon, bf, f2e, info, ifirst;
   std::vector<int> bface_h;  // boundary faces E*nfe + l (bf > 0), ascending
   DevBuf<int> bface;
   DevBuf<long> src1, src2;
@@ -86,10 +86,10 @@ struct Solver {
   DevBuf<double> H, DinvF, RuS, Rh, b, BE, bjaug, we, du, RuR, bres;
   // per-block workspace
   int neb = 0;
-  DevBuf<double> aug, Bfull, Kt, Gfull, rv, rJ, W, fpt;
+  DevBuf<double> aug, Bfull, Kt, Gc, K0c, H0c, rv, rJ, W, fpt;
   // mixed precision: FP32 copies of H, DinvF, the LU factors of D', K' and the preconditioner blocks
   DevBuf<float> H32, DinvF32, LU32, K32, BE32, BEilu32, BEeas32, easaug32;
-  DevBuf<float> aug32, Bfull32, Gfull32, W32;  // FP32 element-block workspace (mixed form)
+  DevBuf<float> aug32, Bfull32, Gc32, K0c32, H0c32, W32;  // FP32 element-block workspace (mixed form)
   DevBuf<float> MCs32, MEs32, shapegt32;       // FP32 copies of M^-1 C, M^-1 E and the shape table
   bool q32_ready = false;
   bool dinvf_fp32 = false;  // the last assembly kept D^{-1}F in FP32 only (DinvF32)

@@ -13,7 +13,7 @@ CASES = [  # builder arguments, m
     ("poisson2d", dict(n=5, porder=1, pgauss=2), 8),
     ("poisson2d", dict(n=3, porder=4, pgauss=8, elemtype=0), 15),
     ("poisson2d", dict(n=5, porder=5, pgauss=10), 24),
-    ("poisson2d", dict(n=3, porder=8, pgauss=14), 36),
+    ("poisson2d", dict(n=3, porder=7, pgauss=14), 32),
     ("poisson2d", dict(n=2, porder=2, pgauss=4, nd=3), 54),
     ("poisson2d", dict(n=2, porder=3, pgauss=6, nd=3), 96),
     ("convdiff3d", dict(n=2, porder=2), 108),
