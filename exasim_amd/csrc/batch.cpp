@@ -182,6 +182,9 @@ void Solver::build_seg(SegDev& sd, const std::vector<long>& off) {
   sd.map.bbeg = sd.bbeg.p;
   sd.map.bend = sd.bend.p;
   sd.map.sbptr = sd.sbptr.p;
+  sd.map.maxblk = 0;
+  for (int sg = 0; sg < ns; ++sg) sd.map.maxblk = std::max(sd.map.maxblk, sbptr[sg + 1] - sbptr[sg]);
+  sd.map.shared = batch;
 }
 
 void Solver::seg_setup() {
@@ -206,7 +209,7 @@ void Solver::seg_alloc() {
   const long ns = ninst, n1 = restart + 1;
   const long nb = std::max(segT.map.nblk, segU.map.nblk);
   EXA_HIP(hipStreamSynchronize(s));
-  segpart.alloc(static_cast<size_t>(std::max(nb, 1L)) * (n1 + 1));
+  segpart.alloc(static_cast<size_t>(std::max(nb, 1L)) * std::max(n1 + 1, SEG_CHUNK / 64));
   hcol.alloc(static_cast<size_t>(n1 + 1) * ns);
   segy.alloc(static_cast<size_t>(n1) * ns);
   segcoef.alloc(static_cast<size_t>(4 * ns));
@@ -222,7 +225,7 @@ void Solver::seg_alloc() {
   gtol.alloc(1);
   gjcount.alloc(2);  // step counter, completion ticket of the step kernel
   gxmask.alloc(ns);
-  gbcount.alloc((ns + 15) / 16);
+  gbcount.alloc(1);
   clear_graphs();  // captured launches hold the old buffers
   if (!hstat) {  // per-step counts of iterating instances, written by the kernels into host memory
     EXA_HIP(hipHostMalloc(reinterpret_cast<void**>(&hstat), sizeof(int) * GM_RING,

@@ -58,43 +58,16 @@ void Solver::clear_graphs() {
 // rotations and convergence test, x += V y for instances that converged at this step.
 void Solver::gmres_step(const GmresDev& g, int i, double* xv) {
   const long N = d.N;
-  const int ns = ninst;
   double* vi = V.p + N * i;
   double* vm = V.p + N * (i + 1);
   matvec(vi, tmp.p);
   apply_precond_to(tmp.p, vm);
   hipEvent_t t0{};
   tic(T_ORTHO, &t0);
-  if (!batch) {  // one problem: the full-length kernels, skipped once the solve has finished
-    const double* act = g.act;
-    if (ortho == 0) {  // MGS (getpoly.cpp:24-42)
-      for (int k = 0; k <= i; ++k) {
-        dot(vm, V.p + N * k, N, partial.p, hcol.p + k, 0, s, act);
-        axpy_dev(vm, V.p + N * k, hcol.p + k, -1.0, N, s, act);
-      }
-    } else {  // CGS (gmres.cpp:81-88)
-      multidot(V.p, N, i + 1, vm, N, partial.p, hcol.p, s, act);
-      gemv_cols(vm, V.p, N, i + 1, hcol.p, -1.0, N, s, act);
-    }
-    dot(vm, vm, N, partial.p, hcol.p + i + 1, 1, s, act);
-    scale_inv_dev(vm, hcol.p + i + 1, N, s, act);
-  } else {  // per instance: segmented kernels over each instance's own unknowns
-    SegMap ma = segT.map;
-    ma.act = g.act;
-    if (ortho == 0) {
-      for (int k = 0; k <= i; ++k) {
-        seg_multidot(ma, V.p + N * k, N, 1, vm, segpart.p, hcol.p + static_cast<long>(k) * ns, 0, s);
-        seg_axpy(ma, vm, V.p + N * k, hcol.p + static_cast<long>(k) * ns, -1.0, s);
-      }
-    } else {
-      seg_multidot(ma, V.p, N, i + 1, vm, segpart.p, hcol.p, 0, s);
-      seg_gemv_cols(ma, vm, V.p, N, i + 1, hcol.p, -1.0, s);
-    }
-    seg_multidot(ma, vm, N, 1, vm, segpart.p, hcol.p + static_cast<long>(i + 1) * ns, 1, s);
-    seg_scale(segT.map, vm, vm, hcol.p + static_cast<long>(i + 1) * ns, 1, s);
-  }
+  SegMap ma = segT.map;
+  ma.act = g.act;
+  seg_arnoldi(ma, g, V.p, N, i, ortho == 0, vm, segpart.p, hcol.p, s);
   toc(T_ORTHO, t0);
-  gmres_dev_givens(g, i, hcol.p, s);
   (void)xv;  // instances that converge here update x at the end of the cycle
 }
 
@@ -102,13 +75,9 @@ void Solver::gmres_step(const GmresDev& g, int i, double* xv) {
 void Solver::gmres_update_x(const GmresDev& g, int k, double* xv) {
   if (k <= 0) return;
   const long N = d.N;
-  if (!batch) {
-    gemv_cols(xv, V.p, N, k, g.y, 1.0, N, s, g.xmask, true);
-  } else {
-    SegMap mx = segT.map;
-    mx.act = g.xmask;
-    seg_gemv_cols(mx, xv, V.p, N, k, g.y, 1.0, s, true);
-  }
+  SegMap mx = segT.map;
+  mx.act = g.xmask;
+  seg_gemv_cols(mx, xv, V.p, N, k, g.y, 1.0, s);
 }
 
 // End of a cycle of i steps (gmres.cpp:551-566): x += V y, r = P (b - A x), restart test, v_0.

@@ -2359,7 +2359,6 @@ int lu_panel_width_f32(int n) {
 // Vector kernels (fixed-order reductions)
 // ---------------------------------------------------------------------------
 constexpr int DOT_BS = 256;
-constexpr int DOT_MAXB = 1024;
 
 __global__ __launch_bounds__(DOT_BS) void k_dot_partial(const double* x, const double* y, long n,
                                                         double* partial, const double* act) {
@@ -2395,39 +2394,6 @@ __global__ __launch_bounds__(DOT_BS) void k_reduce(const double* partial, int nb
   if (threadIdx.x == 0) out[blockIdx.x] = sqrt_out ? sqrt(sh[0]) : sh[0];
 }
 
-// partial[v][b] for v < k: dot(V_v, w) -- blockIdx.y = v
-__global__ __launch_bounds__(DOT_BS) void k_multidot_partial(const double* V, long ldv,
-                                                             const double* w, long n, double* partial,
-                                                             const double* act) {
-  if (act && act[0] == 0.0) return;
-  __shared__ double sh[DOT_BS];
-  const double* x = V + ldv * blockIdx.y;
-  double s = 0.0;
-  for (long i = blockIdx.x * static_cast<long>(DOT_BS) + threadIdx.x; i < n;
-       i += static_cast<long>(gridDim.x) * DOT_BS)
-    s = fma(x[i], w[i], s);
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int st = DOT_BS / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[static_cast<long>(blockIdx.y) * gridDim.x + blockIdx.x] = sh[0];
-}
-
-__global__ void k_axpy_dev(double* y, const double* x, const double* coef, double scale, long n,
-                           const double* act) {
-  if (act && act[0] == 0.0) return;
-  const long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (i < n) y[i] = fma(scale * coef[0], x[i], y[i]);
-}
-
-__global__ void k_scale_inv_dev(double* x, const double* coef, long n, const double* act) {
-  if (act && act[0] == 0.0) return;
-  const long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (i < n) x[i] = x[i] * (1.0 / coef[0]);
-}
-
 __global__ void k_axpby(double* y, const double* x, double a, double b, long n) {
   const long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   // b == 0: y is not read (it may be fresh memory holding any bit pattern, NaN included)
@@ -2446,24 +2412,6 @@ __global__ void k_first_nonzero(const int* info, long n, int* out) {
 __global__ void k_copy(double* y, const double* x, long n) {
   const long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   if (i < n) y[i] = x[i];
-}
-
-// x += alpha * V[:, 0:k] y   (y on the device)
-// SKIPZ: columns whose coefficient is zero are not read (a basis column the solve has not
-// written in this cycle may hold anything)
-template <bool SKIPZ>
-__global__ void k_gemv_cols(double* x, const double* V, long ldv, int k, const double* y, double alpha,
-                            long n, const double* act) {
-  if (act && act[0] == 0.0) return;
-  const long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (i >= n) return;
-  double s = 0.0;
-  for (int j = 0; j < k; ++j) {
-    const double yj = y[j];
-    if (SKIPZ && yj == 0.0) continue;
-    s = fma(V[i + ldv * j], yj, s);
-  }
-  x[i] = fma(alpha, s, x[i]);
 }
 
 template <class M>
@@ -3296,9 +3244,9 @@ void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, do
   EXA_HIP(hipGetLastError());
 }
 
-int dot_partials_count(long n) {
+static int dot_partials_count(long n) {
   long b = (n + DOT_BS - 1) / DOT_BS;
-  return static_cast<int>(std::max(1L, std::min<long>(DOT_MAXB, b)));
+  return static_cast<int>(std::max(1L, std::min<long>(DOT_PARTIALS, b)));
 }
 
 void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out,
@@ -3306,26 +3254,6 @@ void dot(const double* x, const double* y, long n, double* partial, double* out,
   int nb = dot_partials_count(n);
   k_dot_partial<<<nb, DOT_BS, 0, s>>>(x, y, n, partial, act);
   k_reduce<<<1, DOT_BS, 0, s>>>(partial, nb, out, sqrt_out, act);
-  EXA_HIP(hipGetLastError());
-}
-
-void multidot(const double* V, long ldv, int k, const double* w, long n, double* partial, double* out,
-              hipStream_t s, const double* act) {
-  int nb = dot_partials_count(n);
-  dim3 grid(nb, k);
-  k_multidot_partial<<<grid, DOT_BS, 0, s>>>(V, ldv, w, n, partial, act);
-  k_reduce<<<k, DOT_BS, 0, s>>>(partial, nb, out, 0, act);
-  EXA_HIP(hipGetLastError());
-}
-
-void axpy_dev(double* y, const double* x, const double* coef, double scale, long n, hipStream_t s,
-              const double* act) {
-  k_axpy_dev<<<nblocks(n, 256), 256, 0, s>>>(y, x, coef, scale, n, act);
-  EXA_HIP(hipGetLastError());
-}
-
-void scale_inv_dev(double* x, const double* coef, long n, hipStream_t s, const double* act) {
-  k_scale_inv_dev<<<nblocks(n, 256), 256, 0, s>>>(x, coef, n, act);
   EXA_HIP(hipGetLastError());
 }
 
@@ -3345,521 +3273,17 @@ void copy(double* y, const double* x, long n, hipStream_t s) {
   EXA_HIP(hipGetLastError());
 }
 
-void gemv_cols(double* x, const double* V, long ldv, int k, const double* y, double alpha, long n,
-               hipStream_t s, const double* act, bool skip_zero) {
-  if (skip_zero) k_gemv_cols<true><<<nblocks(n, 256), 256, 0, s>>>(x, V, ldv, k, y, alpha, n, act);
-  else k_gemv_cols<false><<<nblocks(n, 256), 256, 0, s>>>(x, V, ldv, k, y, alpha, n, act);
-  EXA_HIP(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
-// Restarted GMRES with the Krylov scalars on the device (gmres.cpp:361-597): the Givens
-// rotations, the convergence test and the back substitution of every instance run in one small
-// kernel per Arnoldi step, so the host never waits on a step.  One block; thread t handles
-// instances t, t + 256, ...; stat[0] receives the number of instances still iterating.
-// ---------------------------------------------------------------------------
 namespace {
-
-constexpr int GM_BS = 1024;  // one block: 16 waves
-
-// cpuApplyGivensRotation (backend/Common/cpuimpl.h:167-197) on the new Hessenberg column of one
-// instance: the rotations k < i are applied in order with the running entry (the column's entry k
-// after rotation k-1) kept in a register, so the chain waits on FMAs only, not on memory; the
-// column comes from hcol (entry k at hc[k*ns]) and the rotated column goes to H.
-__device__ void dev_givens(const double* __restrict__ hc, int ns, double* __restrict__ H, double* __restrict__ s,
-                           double* __restrict__ cs, double* __restrict__ sn, int i) {
-  double carry = hc[0];
-  int k = 0;
-  for (; k + 8 <= i; k += 8) {  // the chunk's loads are issued before its FMAs
-    double h1[8], c[8], sg[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      h1[u] = hc[static_cast<long>(k + u + 1) * ns];
-      c[u] = cs[k + u];
-      sg[u] = sn[k + u];
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      H[k + u] = c[u] * carry + sg[u] * h1[u];
-      carry = -sg[u] * carry + c[u] * h1[u];
-    }
-  }
-  for (; k < i; ++k) {
-    const double h1 = hc[static_cast<long>(k + 1) * ns];
-    const double c = cs[k], sg = sn[k];
-    H[k] = c * carry + sg * h1;
-    carry = -sg * carry + c * h1;
-  }
-  const double a = carry, b = hc[static_cast<long>(i + 1) * ns];
-  double ci, si;
-  if (b == 0.0) {
-    ci = 1.0;
-    si = 0.0;
-  } else if (fabs(b) > fabs(a)) {
-    const double t = a / b;
-    si = 1.0 / sqrt(1.0 + t * t);
-    ci = t * si;
-  } else {
-    const double t = b / a;
-    ci = 1.0 / sqrt(1.0 + t * t);
-    si = t * ci;
-  }
-  cs[i] = ci;
-  sn[i] = si;
-  const double t = ci * s[i];
-  s[i + 1] = -si * s[i];
-  s[i] = t;
-  H[i] = ci * a + si * b;
-  H[i + 1] = 0.0;
-}
-
-// cpuBackSolve (cpuimpl.h:199-208) by one wave: y (stride ys) = R^{-1} s over rows 0..i, R the
-// leading (i+1) x (i+1) block of Hm (column-major, ld).  Column-oriented: lane l keeps the right-
-// hand sides of rows l, l + 64, ...; for k = i .. 0 the owner of row k divides, the value goes to
-// every lane, and each lane updates its rows above k; the columns' entries are loaded 8 columns
-// ahead.  Rows beyond 64 * GM_ROWS fall back to one lane.
-constexpr int GM_ROWS = 4;  // i + 1 <= 256 on the wave path
-__device__ void dev_back_solve_wave(double* __restrict__ y, int ys, const double* __restrict__ Hm,
-                                    const double* __restrict__ s, int i, int ld) {
-  const int lane = threadIdx.x & 63;
-  if (i + 1 > 64 * GM_ROWS) {
-    if (lane == 0) {
-      for (int j = i; j >= 0; --j) y[static_cast<long>(j) * ys] = s[j];
-      for (int j = i; j >= 0; --j) {
-        const double yj = y[static_cast<long>(j) * ys] / Hm[j + static_cast<long>(ld) * j];
-        y[static_cast<long>(j) * ys] = yj;
-        for (int k = j - 1; k >= 0; --k) y[static_cast<long>(k) * ys] -= Hm[k + static_cast<long>(ld) * j] * yj;
-      }
-    }
-    return;
-  }
-  double r[GM_ROWS];
-#pragma unroll
-  for (int q = 0; q < GM_ROWS; ++q) {
-    const int row = lane + 64 * q;
-    r[q] = row <= i ? s[row] : 0.0;
-  }
-  for (int k0 = i; k0 >= 0; k0 -= 8) {
-    double col[8][GM_ROWS], dg[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int k = k0 - u;
-      const int kk = k >= 0 ? k : 0;
-      dg[u] = Hm[kk + static_cast<long>(ld) * kk];
-#pragma unroll
-      for (int q = 0; q < GM_ROWS; ++q) {
-        const int row = lane + 64 * q;
-        col[u][q] = row < kk ? Hm[row + static_cast<long>(ld) * kk] : 0.0;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int k = k0 - u;
-      if (k < 0) break;
-      const int ql = k >> 6, owner = k & 63;
-      double rk = 0.0;
-#pragma unroll
-      for (int q = 0; q < GM_ROWS; ++q)
-        if (q == ql) rk = r[q];
-      rk = __shfl(rk, owner);
-      const double yk = rk / dg[u];
-      if (lane == owner) y[static_cast<long>(k) * ys] = yk;
-#pragma unroll
-      for (int q = 0; q < GM_ROWS; ++q) r[q] -= col[u][q] * yk;
-    }
-  }
-}
-
-__device__ void block_count(int mine, int* stat) {
-  __shared__ int cnt;
-  if (threadIdx.x == 0) cnt = 0;
-  __syncthreads();
-  if (mine) atomicAdd(&cnt, mine);
-  __syncthreads();
-  if (threadIdx.x == 0) stat[0] = cnt;
-}
-
-// start of a solve: an instance iterates unless ||b|| is zero, non-finite, or (Newton's own
-// solves) below the nonlinear tolerance (gmres.cpp:412-415)
-__global__ __launch_bounds__(GM_BS) void k_gmres_begin(GmresDev g, const double* nb, double tol, double ntol,
-                                                       int use_ntol) {
-  if (threadIdx.x == 0) {
-    g.tol[0] = tol;
-    g.jcount[0] = 0;
-    g.ticket[0] = 0;
-  }
-  int mine = 0;
-  for (int sg = threadIdx.x; sg < g.ns; sg += GM_BS) {
-    const double b = nb[sg];
-    const bool a = isfinite(b) && !(b == 0.0 || (use_ntol && b < ntol));
-    g.act[sg] = a ? 1.0 : 0.0;
-    g.jc[sg] = 0.0;
-    g.iters[sg] = 0;
-    mine += a;
-  }
-  block_count(mine, g.stat);
-}
-
-// first cycle: nrmb = ||P r0|| (gmres.cpp:431-445), s = (nrmb, 0, ...), coef = 1/||r|| scale of v_0
-__global__ __launch_bounds__(GM_BS) void k_gmres_start(GmresDev g, const double* nr, double* coef) {
-  int mine = 0;
-  const int n1 = g.n1;
-  for (int sg = threadIdx.x; sg < g.ns; sg += GM_BS) {
-    const double r = nr[sg];
-    if (g.act[sg] != 0.0 && !isfinite(r)) g.act[sg] = 0.0;
-    const bool a = g.act[sg] != 0.0;
-    g.nrmb[sg] = r;
-    double* sv = g.sv + static_cast<long>(sg) * (n1 + 1);
-    sv[0] = a ? r : 0.0;
-    for (int k = 1; k <= n1; ++k) sv[k] = 0.0;
-    coef[sg] = a ? r : 0.0;
-    mine += a;
-  }
-  block_count(mine, g.stat);
-}
-
-// Arnoldi step j (column i of the cycle): rotate the new column hcol[k*ns + sg] (k <= i+1), test
-// |s_{i+1}| / nrmb < tol; a converged instance gets y = R^{-1} s in y[k*ns + sg] (k <= i), jc = 1,
-// act = 0 and the reference's iteration count j; a non-finite rotation stops the instance.
-// Arnoldi step j: one wave per instance, 16 instances per block.  The wave stages the new column
-// (hcol[k*ns + sg], k <= i + 1) and the instance's rotations in LDS, lane 0 applies the rotations
-// in order and forms the new one (cpuApplyGivensRotation, cpuimpl.h:167-197, the same operations
-// as dev_givens), the lanes write the rotated column to H, and an instance with
-// |s_{i+1}| / nrmb < tol gets y = R^{-1} s (zero above row i), jc = 1 (x += V y at the end of the
-// cycle), act = 0 and the reference's iteration count j; a non-finite rotation stops the instance.
-// The last block to finish adds the blocks' counts in block order, writes them to stat[j % ring]
-// and advances jcount.
-constexpr int GM_WAVES = GM_BS / 64;
-constexpr int GM_LDS_N1 = 128;  // columns up to this length are staged in LDS
-__global__ __launch_bounds__(GM_BS) void k_gmres_givens(GmresDev g, int i, const double* hcol) {
-  __shared__ double lh[GM_WAVES][GM_LDS_N1 + 1], lc[GM_WAVES][GM_LDS_N1], ls[GM_WAVES][GM_LDS_N1];
-  __shared__ int flag[GM_WAVES];
-  __shared__ int cnt;
-  __shared__ bool last;
-  const int n1 = g.n1, ns = g.ns;
-  const int wave = static_cast<int>(threadIdx.x >> 6), lane = static_cast<int>(threadIdx.x & 63);
-  const int sg = static_cast<int>(blockIdx.x) * GM_WAVES + wave;
-  const int j = g.jcount[0];
-  const double tol = g.tol[0];
-  const bool live = sg < ns && g.act[sg] != 0.0;
-  const bool staged = n1 <= GM_LDS_N1;
-  if (threadIdx.x == 0) cnt = 0;
-  double* H = nullptr;
-  double *sv = nullptr, *cs = nullptr, *sn = nullptr;
-  if (live) {
-    H = g.Hm + static_cast<long>(sg) * n1 * n1 + static_cast<long>(n1) * i;
-    sv = g.sv + static_cast<long>(sg) * (n1 + 1);
-    cs = g.cs + static_cast<long>(sg) * (n1 + 1);
-    sn = g.sn + static_cast<long>(sg) * (n1 + 1);
-    if (staged) {
-      for (int k = lane; k <= i + 1; k += 64) lh[wave][k] = hcol[static_cast<long>(k) * ns + sg];
-      for (int k = lane; k < i; k += 64) {
-        lc[wave][k] = cs[k];
-        ls[wave][k] = sn[k];
-      }
-    }
-  }
-  __syncthreads();
-  if (live && lane == 0) {
-    if (staged) {
-      double* h = lh[wave];
-      const double* c = lc[wave];
-      const double* sg_ = ls[wave];
-      double carry = h[0];
-      for (int k = 0; k < i; ++k) {
-        const double h1 = h[k + 1];
-        h[k] = c[k] * carry + sg_[k] * h1;
-        carry = -sg_[k] * carry + c[k] * h1;
-      }
-      const double a0 = carry, b0 = h[i + 1];
-      double ci, si;
-      if (b0 == 0.0) {
-        ci = 1.0;
-        si = 0.0;
-      } else if (fabs(b0) > fabs(a0)) {
-        const double t = a0 / b0;
-        si = 1.0 / sqrt(1.0 + t * t);
-        ci = t * si;
-      } else {
-        const double t = b0 / a0;
-        ci = 1.0 / sqrt(1.0 + t * t);
-        si = t * ci;
-      }
-      cs[i] = ci;
-      sn[i] = si;
-      const double t = ci * sv[i];
-      sv[i + 1] = -si * sv[i];
-      sv[i] = t;
-      h[i] = ci * a0 + si * b0;
-      h[i + 1] = 0.0;
-    } else {
-      dev_givens(hcol + sg, ns, H, sv, cs, sn, i);
-    }
-    g.iters[sg] = j + 1;
-    const double s1 = sv[i + 1];
-    int f = 1;  // 1 iterating, 2 converged, 0 stopped
-    if (!isfinite(s1)) f = 0;
-    else if (fabs(s1) / g.nrmb[sg] < tol) f = 2;
-    if (f != 1) {
-      g.act[sg] = 0.0;
-      if (f == 2) {
-        g.iters[sg] = j;
-        g.jc[sg] = 1.0;
-      }
-    }
-    flag[wave] = f;
-  }
-  __syncthreads();
-  if (live) {
-    if (staged)
-      for (int k = lane; k <= i + 1; k += 64) H[k] = lh[wave][k];
-    if (flag[wave] == 2) {  // y = R^{-1} s, zero above row i
-      __threadfence_block();
-      dev_back_solve_wave(g.y + sg, ns, g.Hm + static_cast<long>(sg) * n1 * n1, sv, i, n1);
-      for (int k = i + 1 + lane; k < n1; k += 64) g.y[static_cast<long>(k) * ns + sg] = 0.0;
-    }
-    if (lane == 0 && flag[wave] == 1) atomicAdd(&cnt, 1);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    g.bcount[blockIdx.x] = cnt;
-    __threadfence();
-    last = atomicAdd(g.ticket, 1) == static_cast<int>(gridDim.x) - 1;
-  }
-  __syncthreads();
-  if (last && threadIdx.x == 0) {
-    __threadfence();
-    int tot = 0;
-    for (unsigned b = 0; b < gridDim.x; ++b) tot += atomicAdd(g.bcount + b, 0);
-    g.stat[j % g.ring] = tot;
-    g.jcount[0] = j + 1;
-    g.ticket[0] = 0;
-  }
-}
-
-// end of a cycle of i steps: y = R^{-1} s over rows 0..i-1 for the instances still iterating
-// (for x += V y, gmres.cpp:552, UpdateSolution); xmask marks them and the instances that converged
-// in this cycle (their y is set), one wave per instance
-__global__ __launch_bounds__(GM_BS) void k_gmres_cycle_y(GmresDev g, int i) {
-  const int n1 = g.n1, ns = g.ns;
-  const int lane = threadIdx.x & 63;
-  for (int sg = static_cast<int>(threadIdx.x >> 6); sg < ns; sg += GM_BS / 64) {
-    if (g.act[sg] != 0.0) {
-      dev_back_solve_wave(g.y + sg, ns, g.Hm + static_cast<long>(sg) * n1 * n1,
-                          g.sv + static_cast<long>(sg) * (n1 + 1), i - 1, n1);
-      for (int k = i + lane; k < n1; k += 64) g.y[static_cast<long>(k) * ns + sg] = 0.0;
-    }
-    if (lane == 0) g.xmask[sg] = (g.act[sg] != 0.0 || g.jc[sg] != 0.0) ? 1.0 : 0.0;
-  }
-}
-
-// end of a solve: x += V y still due for the instances that converged in the last cycle
-__global__ __launch_bounds__(GM_BS) void k_gmres_flush(GmresDev g) {
-  for (int sg = threadIdx.x; sg < g.ns; sg += GM_BS) {
-    g.xmask[sg] = g.jc[sg];
-    g.jc[sg] = 0.0;
-  }
-}
-
-// restart test (gmres.cpp:561-566): ||P(b - A x)|| / nrmb < tol stops the instance; the others
-// restart with s = (||r||, 0, ...) and v_0 = r / ||r||
-__global__ __launch_bounds__(GM_BS) void k_gmres_restart(GmresDev g, const double* nr, double* coef) {
-  int mine = 0;
-  const int n1 = g.n1;
-  const double tol = g.tol[0];
-  const int j = g.jcount[0] - 1;  // the step this cycle ended with
-  for (int sg = threadIdx.x; sg < g.ns; sg += GM_BS) {
-    g.jc[sg] = 0.0;  // their x update was made with the cycle's
-    const double r = nr[sg];
-    if (g.act[sg] != 0.0 && r / g.nrmb[sg] < tol) g.act[sg] = 0.0;
-    const bool a = g.act[sg] != 0.0;
-    if (a) {
-      double* sv = g.sv + static_cast<long>(sg) * (n1 + 1);
-      sv[0] = r;
-      for (int k = 1; k <= n1; ++k) sv[k] = 0.0;
-    }
-    coef[sg] = a ? r : 0.0;
-    mine += a;
-  }
-  block_count(mine, g.stat + j % g.ring);
-}
 
 __global__ void k_fill(double* y, double v, long n) {
   const long i = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
   if (i < n) y[i] = v;
 }
-
 }  // namespace
 
-void gmres_dev_begin(const GmresDev& g, const double* nb, double tol, double newton_tol, int use_newton_tol,
-                     hipStream_t s) {
-  k_gmres_begin<<<1, GM_BS, 0, s>>>(g, nb, tol, newton_tol, use_newton_tol);
-  EXA_HIP(hipGetLastError());
-}
-void gmres_dev_start(const GmresDev& g, const double* nr, double* coef, hipStream_t s) {
-  k_gmres_start<<<1, GM_BS, 0, s>>>(g, nr, coef);
-  EXA_HIP(hipGetLastError());
-}
-void gmres_dev_givens(const GmresDev& g, int i, const double* hcol, hipStream_t s) {
-  k_gmres_givens<<<(g.ns + GM_WAVES - 1) / GM_WAVES, GM_BS, 0, s>>>(g, i, hcol);
-  EXA_HIP(hipGetLastError());
-}
-void gmres_dev_cycle_y(const GmresDev& g, int i, hipStream_t s) {
-  k_gmres_cycle_y<<<1, GM_BS, 0, s>>>(g, i);
-  EXA_HIP(hipGetLastError());
-}
-void gmres_dev_flush(const GmresDev& g, hipStream_t s) {
-  k_gmres_flush<<<1, GM_BS, 0, s>>>(g);
-  EXA_HIP(hipGetLastError());
-}
-void gmres_dev_restart(const GmresDev& g, const double* nr, double* coef, hipStream_t s) {
-  k_gmres_restart<<<1, GM_BS, 0, s>>>(g, nr, coef);
-  EXA_HIP(hipGetLastError());
-}
 void fill(double* y, double v, long n, hipStream_t s) {
   if (n <= 0) return;
   k_fill<<<nblocks(n, 256), 256, 0, s>>>(y, v, n);
-  EXA_HIP(hipGetLastError());
-}
-
-// ---------------------------------------------------------------------------
-// Vectors split into per-instance segments (batched solves).  Every block covers
-// entries [bbeg, bend) of one segment, so a segment's sums and updates depend on
-// its own entries and length only.
-// ---------------------------------------------------------------------------
-namespace {
-
-constexpr int SEG_BS = 256;
-
-// partial[v*nblk + b] = sum over block b of V_v[i] * w[i]   (blockIdx.y = v)
-__global__ __launch_bounds__(SEG_BS) void k_seg_dot_partial(SegMap m, const double* V, long ldv,
-                                                            const double* w, double* partial) {
-  __shared__ double sh[SEG_BS];
-  const int b = blockIdx.x;
-  if (m.act && m.act[m.bseg[b]] == 0.0) {  // block-uniform
-    if (threadIdx.x == 0) partial[static_cast<long>(blockIdx.y) * m.nblk + b] = 0.0;
-    return;
-  }
-  const double* x = V + ldv * blockIdx.y;
-  double acc = 0.0;
-  for (long i = m.bbeg[b] + threadIdx.x; i < m.bend[b]; i += SEG_BS) acc = fma(x[i], w[i], acc);
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  for (int st = SEG_BS / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) partial[static_cast<long>(blockIdx.y) * m.nblk + b] = sh[0];
-}
-
-// partial[v*nblk + b] = <V_v, w> over block b for every v < k: one block per chunk, the chunk of
-// w staged in LDS once, wave q owns vectors q, q+4, ...; each lane sums its strided entries in
-// order and the wave adds its lanes with a fixed butterfly.
-__global__ __launch_bounds__(SEG_BS) void k_seg_multidot_partial(SegMap m, const double* V, long ldv, int k,
-                                                                 const double* w, double* partial) {
-  __shared__ double wl[SEG_CHUNK];
-  const int b = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (m.act && m.act[m.bseg[b]] == 0.0) {  // block-uniform
-    for (int v = threadIdx.x; v < k; v += SEG_BS) partial[static_cast<long>(v) * m.nblk + b] = 0.0;
-    return;
-  }
-  const long i0 = m.bbeg[b];
-  const int len = static_cast<int>(m.bend[b] - i0);
-  for (int t = threadIdx.x; t < len; t += SEG_BS) wl[t] = w[i0 + t];
-  __syncthreads();
-  for (int v = wave; v < k; v += SEG_BS / 64) {
-    const double* x = V + ldv * v + i0;
-    double acc = 0.0;
-    for (int t = lane; t < len; t += 64) acc = fma(x[t], wl[t], acc);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off);
-    if (lane == 0) partial[static_cast<long>(v) * m.nblk + b] = acc;
-  }
-}
-
-// out[v*nseg + s] = sum of segment s's partials (fixed order), sqrt if asked  (blockIdx.y = v)
-__global__ __launch_bounds__(SEG_BS) void k_seg_reduce(SegMap m, const double* partial, double* out,
-                                                       int sqrt_out) {
-  __shared__ double sh[SEG_BS];
-  const int sg = blockIdx.x;
-  const double* pv = partial + static_cast<long>(blockIdx.y) * m.nblk;
-  double acc = 0.0;
-  for (int i = m.sbptr[sg] + threadIdx.x; i < m.sbptr[sg + 1]; i += SEG_BS) acc += pv[i];
-  sh[threadIdx.x] = acc;
-  __syncthreads();
-  for (int st = SEG_BS / 2; st > 0; st >>= 1) {
-    if (threadIdx.x < st) sh[threadIdx.x] += sh[threadIdx.x + st];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[static_cast<long>(blockIdx.y) * m.nseg + sg] = sqrt_out ? sqrt(sh[0]) : sh[0];
-}
-
-// y += scale * coef[seg] * x
-__global__ __launch_bounds__(SEG_BS) void k_seg_axpy(SegMap m, double* y, const double* x, const double* coef,
-                                                     double scale) {
-  const int b = blockIdx.x;
-  if (m.act && m.act[m.bseg[b]] == 0.0) return;
-  const double c = scale * coef[m.bseg[b]];
-  if (c == 0.0) return;
-  for (long i = m.bbeg[b] + threadIdx.x; i < m.bend[b]; i += SEG_BS) y[i] = fma(c, x[i], y[i]);
-}
-
-// mode 0: y = coef[seg] * x;  mode 1: y = x / coef[seg] (0 where coef[seg] == 0)
-__global__ __launch_bounds__(SEG_BS) void k_seg_scale(SegMap m, double* y, const double* x, const double* coef,
-                                                      int mode) {
-  const int b = blockIdx.x;
-  const double cv = coef[m.bseg[b]];
-  const double c = mode == 0 ? cv : (cv != 0.0 ? 1.0 / cv : 0.0);
-  for (long i = m.bbeg[b] + threadIdx.x; i < m.bend[b]; i += SEG_BS) y[i] = c * x[i];
-}
-
-// x += alpha * sum_j V_j * y[j*nseg + seg]
-template <bool SKIPZ>
-__global__ __launch_bounds__(SEG_BS) void k_seg_gemv_cols(SegMap m, double* x, const double* V, long ldv, int k,
-                                                          const double* y, double alpha) {
-  const int b = blockIdx.x;
-  const int sg = m.bseg[b];
-  if (m.act && m.act[sg] == 0.0) return;
-  for (long i = m.bbeg[b] + threadIdx.x; i < m.bend[b]; i += SEG_BS) {
-    double acc = 0.0;
-    for (int j = 0; j < k; ++j) {
-      const double yj = y[static_cast<long>(j) * m.nseg + sg];
-      if (SKIPZ && yj == 0.0) continue;
-      acc = fma(V[i + ldv * j], yj, acc);
-    }
-    x[i] = fma(alpha, acc, x[i]);
-  }
-}
-
-}  // namespace
-
-void seg_multidot(const SegMap& m, const double* V, long ldv, int k, const double* w, double* partial,
-                  double* out, int sqrt_out, hipStream_t s) {
-  if (m.nblk == 0 || k == 0) return;
-  if (k >= 4) k_seg_multidot_partial<<<m.nblk, SEG_BS, 0, s>>>(m, V, ldv, k, w, partial);
-  else k_seg_dot_partial<<<dim3(m.nblk, k), SEG_BS, 0, s>>>(m, V, ldv, w, partial);
-  k_seg_reduce<<<dim3(m.nseg, k), SEG_BS, 0, s>>>(m, partial, out, sqrt_out);
-  EXA_HIP(hipGetLastError());
-}
-
-void seg_axpy(const SegMap& m, double* y, const double* x, const double* coef, double scale, hipStream_t s) {
-  if (m.nblk == 0) return;
-  k_seg_axpy<<<m.nblk, SEG_BS, 0, s>>>(m, y, x, coef, scale);
-  EXA_HIP(hipGetLastError());
-}
-
-void seg_scale(const SegMap& m, double* y, const double* x, const double* coef, int mode, hipStream_t s) {
-  if (m.nblk == 0) return;
-  k_seg_scale<<<m.nblk, SEG_BS, 0, s>>>(m, y, x, coef, mode);
-  EXA_HIP(hipGetLastError());
-}
-
-void seg_gemv_cols(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double alpha,
-                   hipStream_t s, bool skip_zero) {
-  if (m.nblk == 0 || k == 0) return;
-  if (skip_zero) k_seg_gemv_cols<true><<<m.nblk, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha);
-  else k_seg_gemv_cols<false><<<m.nblk, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha);
   EXA_HIP(hipGetLastError());
 }
 

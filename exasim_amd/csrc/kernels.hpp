@@ -263,23 +263,14 @@ void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, do
                 double* out, hipStream_t s, const double* act = nullptr);
 
 // ---- vector kernels (results stay on the device) ----
-int dot_partials_count(long n);
+constexpr int DOT_PARTIALS = 1024;  // partial sums of dot, at most
 void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out,
          hipStream_t s, const double* act = nullptr);
-void axpy_dev(double* y, const double* x, const double* coef, double scale, long n, hipStream_t s,
-              const double* act = nullptr);
-void scale_inv_dev(double* x, const double* coef, long n, hipStream_t s, const double* act = nullptr);
 // y = a x + b y; with b == 0 y is only written
 void axpby(double* y, const double* x, double a, double b, long n, hipStream_t s);
 void copy(double* y, const double* x, long n, hipStream_t s);
 // out[0] = lowest i < n with info[i] != 0, or INT_MAX (device int)
 void first_nonzero(const int* info, long n, int* out, hipStream_t s);
-// skip_zero: columns with a zero coefficient are not read
-void gemv_cols(double* x, const double* V, long ldv, int k, const double* y, double alpha, long n,
-               hipStream_t s, const double* act = nullptr, bool skip_zero = false);
-void multidot(const double* V, long ldv, int k, const double* w, long n, double* partial, double* out,
-              hipStream_t s, const double* act = nullptr);
-
 // y[0..n) = v
 void fill(double* y, double v, long n, hipStream_t s);
 
@@ -294,7 +285,7 @@ void fill(double* y, double v, long n, hipStream_t s);
 // do not depend on j, so one captured graph per column i serves every cycle.
 // jc [ns]: 1.0 for an instance that converged in the current cycle (its x += V y is made with the
 // cycle's, or by gmres_dev_flush at the end); xmask [ns]: the instances of the next x update;
-// bcount [(ns + 15) / 16], ticket [1]: the step kernel's per-block counts and completion ticket.
+// bcount [1], ticket [1]: the step's count of iterating instances and its completion ticket.
 struct GmresDev {
   int ns, n1, ring;
   double *Hm, *sv, *cs, *sn, *nrmb, *act, *jc, *y, *tol, *xmask;
@@ -304,7 +295,6 @@ struct GmresDev {
 void gmres_dev_begin(const GmresDev& g, const double* nb, double tol, double newton_tol, int use_newton_tol,
                      hipStream_t s);
 void gmres_dev_start(const GmresDev& g, const double* nr, double* coef, hipStream_t s);
-void gmres_dev_givens(const GmresDev& g, int i, const double* hcol, hipStream_t s);
 void gmres_dev_cycle_y(const GmresDev& g, int i, hipStream_t s);
 // xmask = jc, jc = 0: the x update still due at the end of a solve
 void gmres_dev_flush(const GmresDev& g, hipStream_t s);
@@ -322,6 +312,8 @@ struct SegMap {
   const long* bbeg = nullptr;
   const long* bend = nullptr;
   const int* sbptr = nullptr;
+  int maxblk = 0;       // blocks of the longest segment
+  bool shared = false;  // a batch's segments (a batch of one included)
   // optional per-segment activity (device, 1/0): the dot, axpy and gemv kernels skip the blocks
   // of inactive segments (dots over them read as 0, their entries are left unchanged)
   const double* act = nullptr;
@@ -329,12 +321,17 @@ struct SegMap {
 // out[v*nseg + s] = <V_v, w> over segment s (v < k; sqrt of it with sqrt_out); partial: k*nblk
 void seg_multidot(const SegMap& m, const double* V, long ldv, int k, const double* w, double* partial,
                   double* out, int sqrt_out, hipStream_t s);
+// Arnoldi step (column i of the cycle): w orthogonalised against V_0..V_i (CGS, gmres.cpp:81-88, or MGS,
+// getpoly.cpp:24-42) and normalised, and every instance's rotations and convergence test; the new
+// Hessenberg column in hcol[k*ns + s]; partial: nblk * max(i + 1, 8) values
+void seg_arnoldi(const SegMap& m, const GmresDev& g, const double* V, long n, int i, int mgs, double* w,
+                 double* partial, double* hcol, hipStream_t s);
 // y += scale * coef[s] * x on each segment s
 void seg_axpy(const SegMap& m, double* y, const double* x, const double* coef, double scale, hipStream_t s);
 // mode 0: y = coef[s] * x;  mode 1: y = x / coef[s], and 0 where coef[s] == 0
 void seg_scale(const SegMap& m, double* y, const double* x, const double* coef, int mode, hipStream_t s);
-// x += alpha * sum_{j<k} V_j * y[j*nseg + s]
+// x += alpha * sum_{j<k} V_j * y[j*nseg + s]; columns with a zero coefficient are not read
 void seg_gemv_cols(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double alpha,
-                   hipStream_t s, bool skip_zero = false);
+                   hipStream_t s);
 
 }  // namespace exa

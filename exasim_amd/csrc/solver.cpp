@@ -644,7 +644,7 @@ void Solver::alloc_workspace() {
   fpt.alloc(static_cast<size_t>(neb) * 2 * (d.ncu + d.ncu * d.nc + d.ncu * d.ncu) * d.nfe * d.ngf);
   if (model == MODEL_PLUGIN) pbuf.alloc(static_cast<size_t>(plugin_buffer_doubles(d, plugin_fns.nbc, neb)));
   V.alloc(static_cast<size_t>(restart + 1) * d.N);
-  partial.alloc(static_cast<size_t>(dot_partials_count(d.N)) * (restart + 2));
+  partial.alloc(DOT_PARTIALS);
   seg_alloc();
 }
 
@@ -655,7 +655,6 @@ void Solver::set_option(const std::string& name, double v) {
     if (v < 1 || v > 2000) throw Error(1, "gmres_restart out of range");
     restart = static_cast<int>(v);
     V.alloc(static_cast<size_t>(restart + 1) * d.N);
-    partial.alloc(static_cast<size_t>(dot_partials_count(d.N)) * (restart + 2));
     seg_alloc();
   } else if (name == "gmres_maxit") gmres_maxit = static_cast<int>(v);
   else if (name == "newton_tol") newton_tol = v;
