@@ -1,4 +1,5 @@
-// blkval.hpp -- entries of stored matrix blocks as doubles.
+// blkval.hpp -- device helpers of the block kernels: entries of stored matrix blocks as doubles, and a
+// wave's largest value with its index.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -12,6 +13,16 @@ __device__ __forceinline__ double blk_val(T x) { return static_cast<double>(x); 
 template <>
 __device__ __forceinline__ double blk_val<unsigned short>(unsigned short x) {
   return static_cast<double>(__uint_as_float(static_cast<unsigned int>(x) << 16));
+}
+
+// (v, i) of the wave's largest v, ties to the smaller i, on every lane
+__device__ inline void argmax_wave(double& v, int& i) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    double ov = __shfl_xor(v, off);
+    int oi = __shfl_xor(i, off);
+    if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
+  }
 }
 
 }  // namespace exa

@@ -42,551 +42,6 @@ __device__ inline flt4 mfma_step(float a, float b, flt4 c) {
 }
 
 // ---------------------------------------------------------------------------
-// Right-looking blocked LU of the augmented systems [D | RHS] (n x ncols, ld n),
-// one panel of BLU_NB columns at a time: k_lu_panel factors the panel of every
-// matrix in LDS (partial pivoting), swaps the rows of the columns right of the
-// panel and solves L11 U12 = A12; the trailing update A22 -= L21 U12 and the
-// back substitution's updates run on the MFMA GEMM.
-// ---------------------------------------------------------------------------
-constexpr int BLU_MIN_N = 64;  // smaller blocks use the single-kernel k_lu_solve
-
-__device__ inline void argmax_wave(double& v, int& i) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    double ov = __shfl_xor(v, off);
-    int oi = __shfl_xor(i, off);
-    if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
-  }
-}
-
-template <typename T, int BLU_NB>
-__global__ __launch_bounds__(256) void k_lu_panel(T* Aall, int n, int ncols, long stride, int k0,
-                                                  int* info, int* pivout) {
-  T* A = Aall + stride * blockIdx.x;
-  const int nb = min(BLU_NB, n - k0);
-  const int rows = n - k0;
-  extern __shared__ double lu_sm[];
-  T* P = reinterpret_cast<T*>(lu_sm);  // rows x nb, ld rows
-  __shared__ double wv[4];
-  __shared__ int wi[4];
-  __shared__ int piv[BLU_NB];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  for (int idx = tid; idx < rows * nb; idx += 256) {
-    int r = idx % rows, kk = idx / rows;
-    P[idx] = A[k0 + r + static_cast<long>(n) * (k0 + kk)];
-  }
-  __syncthreads();
-  int singular = 0;
-  for (int kk = 0; kk < nb; ++kk) {
-    double best = -1.0;
-    int bi = kk;
-    for (int r = kk + tid; r < rows; r += 256) {
-      double v = fabs(P[r + rows * kk]);
-      if (v > best) { best = v; bi = r; }
-    }
-    argmax_wave(best, bi);
-    if (lane == 0) { wv[wave] = best; wi[wave] = bi; }
-    __syncthreads();
-    if (tid == 0) {
-      double b = wv[0];
-      int p = wi[0];
-      for (int w = 1; w < 4; ++w)
-        if (wv[w] > b || (wv[w] == b && wi[w] < p)) { b = wv[w]; p = wi[w]; }
-      piv[kk] = p;
-    }
-    __syncthreads();
-    const int p = piv[kk];
-    if (p != kk && tid < nb) {
-      T t = P[kk + rows * tid];
-      P[kk + rows * tid] = P[p + rows * tid];
-      P[p + rows * tid] = t;
-    }
-    __syncthreads();
-    const T pv = P[kk + rows * kk];
-    if (pv == 0.0) singular = 1;
-    const T inv = T(1) / pv;
-    for (int r = kk + 1 + tid; r < rows; r += 256) P[r + rows * kk] *= inv;
-    __syncthreads();
-    const int rr = rows - kk - 1, cc = nb - kk - 1;
-    for (int idx = tid; idx < rr * cc; idx += 256) {
-      int r = kk + 1 + idx % rr, c = kk + 1 + idx / rr;
-      P[r + rows * c] = fma(-P[r + rows * kk], P[kk + rows * c], P[r + rows * c]);
-    }
-    __syncthreads();
-  }
-  for (int idx = tid; idx < rows * nb; idx += 256) {
-    int r = idx % rows, kk = idx / rows;
-    A[k0 + r + static_cast<long>(n) * (k0 + kk)] = P[idx];
-  }
-  // columns right of the panel: row swaps, then U12 = L11^{-1} A12
-  for (int j = k0 + nb + tid; j < ncols; j += 256) {
-    T* colj = A + static_cast<long>(n) * j + k0;
-    T x[BLU_NB];
-#pragma unroll
-    for (int kk = 0; kk < BLU_NB; ++kk) x[kk] = (kk < nb) ? colj[kk] : 0.0;
-    // pivots are applied in order; p < BLU_NB means both rows are in the register
-    // block (a last panel narrower than BLU_NB has rows == nb)
-#pragma unroll
-    for (int kk = 0; kk < BLU_NB; ++kk) {
-      if (kk < nb) {
-        const int p = piv[kk];
-        if (p != kk) {
-          if (p < BLU_NB) {
-#pragma unroll
-            for (int q = kk + 1; q < BLU_NB; ++q)
-              if (q == p) {
-                const T t = x[q];
-                x[q] = x[kk];
-                x[kk] = t;
-              }
-          } else {
-            const T t = colj[p];
-            colj[p] = x[kk];
-            x[kk] = t;
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int kk = 1; kk < BLU_NB; ++kk)
-#pragma unroll
-      for (int t = 0; t < kk; ++t)
-        if (kk < nb) x[kk] = fma(-P[kk + rows * t], x[t], x[kk]);
-#pragma unroll
-    for (int kk = 0; kk < BLU_NB; ++kk)
-      if (kk < nb) colj[kk] = x[kk];
-  }
-  if (tid == 0 && info) info[blockIdx.x] = (k0 == 0 ? 0 : info[blockIdx.x]) | singular;
-  // panel-relative pivots of this panel (row k0+kk was exchanged with row k0+piv[kk])
-  if (pivout && tid < nb) pivout[static_cast<long>(blockIdx.x) * n + k0 + tid] = piv[tid];
-}
-
-// The panel factorisation of k_lu_panel for panels of at most 256 rows, with the panel in
-// registers: thread t holds row t of the rows x nb panel.  Per column: wave argmax of |a[kk]|
-// (ties to the smaller row, as k_lu_panel) and a 4-entry combine, the pivot row and row kk
-// exchanged through a double-buffered LDS row, then each lower row scales its multiplier and
-// updates its own entries -- two barriers per column and no LDS traffic for the rank-1 update.
-// The operations on every entry are those of k_lu_panel, so the factors are the same.  The
-// columns right of the panel are left to k_lu_u12; the pivots go to piv_ws[blockIdx.x][nb]
-// (and to pivout as panel-relative rows).
-template <typename T, int BLU_NB>
-__global__ __launch_bounds__(256) void k_lu_panel_reg(T* Aall, int n, long stride, int k0, int* info,
-                                                      int* pivout, int* piv_ws) {
-  T* A = Aall + stride * blockIdx.x;
-  const int nb = min(BLU_NB, n - k0);
-  const int rows = n - k0;  // <= 256
-  __shared__ double wv[2][4];
-  __shared__ int wi[2][4];
-  __shared__ T prow[2][BLU_NB];
-  __shared__ T xrow[2][BLU_NB];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const bool mine = tid < rows;
-  T a[BLU_NB];
-#pragma unroll
-  for (int c = 0; c < BLU_NB; ++c)
-    a[c] = (mine && c < nb) ? A[k0 + tid + static_cast<long>(n) * (k0 + c)] : 0.0;
-  int singular = 0;
-#pragma clang loop unroll(full)
-  for (int kk = 0; kk < BLU_NB; ++kk) {
-    if (kk < nb) {
-      const int b = kk & 1;
-      double best = (mine && tid >= kk) ? fabs(a[kk]) : -1.0;
-      int bi = (mine && tid >= kk) ? tid : kk;
-      argmax_wave(best, bi);
-      if (lane == 0) {
-        wv[b][wave] = best;
-        wi[b][wave] = bi;
-      }
-      __syncthreads();
-      double bv = wv[b][0];
-      int p = wi[b][0];
-      for (int w = 1; w < 4; ++w)
-        if (wv[b][w] > bv || (wv[b][w] == bv && wi[b][w] < p)) { bv = wv[b][w]; p = wi[b][w]; }
-      if (tid == 0) {
-        piv_ws[static_cast<long>(blockIdx.x) * LU_PIV_WS + kk] = p;
-        if (pivout) pivout[static_cast<long>(blockIdx.x) * n + k0 + kk] = p;
-      }
-      // the pivot row and row kk trade places
-      if (tid == p)
-#pragma unroll
-        for (int c = 0; c < BLU_NB; ++c) prow[b][c] = a[c];
-      if (tid == kk && p != kk)
-#pragma unroll
-        for (int c = 0; c < BLU_NB; ++c) xrow[b][c] = a[c];
-      __syncthreads();
-      if (tid == kk) {
-#pragma unroll
-        for (int c = 0; c < BLU_NB; ++c) a[c] = prow[b][c];
-      } else if (tid == p) {
-#pragma unroll
-        for (int c = 0; c < BLU_NB; ++c) a[c] = xrow[b][c];
-      }
-      const T pv = prow[b][kk];
-      if (pv == 0.0) singular = 1;
-      if (mine && tid > kk) {
-        const T l = a[kk] * (T(1) / pv);
-        a[kk] = l;
-#pragma unroll
-        for (int c = kk + 1; c < BLU_NB; ++c)
-          if (c < nb) a[c] = fma(-l, prow[b][c], a[c]);
-      }
-    }
-  }
-  if (mine)
-#pragma unroll
-    for (int c = 0; c < BLU_NB; ++c)
-      if (c < nb) A[k0 + tid + static_cast<long>(n) * (k0 + c)] = a[c];
-  if (tid == 0 && info) info[blockIdx.x] = (k0 == 0 ? 0 : info[blockIdx.x]) | singular;
-}
-
-// The row exchanges of a panel factored by k_lu_panel_reg, applied to the columns right of the
-// panel.  Thread 0 turns the panel's swaps (row kk <-> row piv[kk], in order) into their net
-// permutation of the rows they touch; every column (one per lane, 64 per workgroup) then reads
-// all the moved values into registers before writing any, so a column costs one round of
-// independent loads instead of a dependent load/store round trip per exchange.
-template <typename T, int BLU_NB>
-__global__ __launch_bounds__(64) void k_lu_swap(T* Aall, int n, int ncols, long stride, int k0, const int* piv_ws) {
-  T* A = Aall + stride * blockIdx.x;
-  const int nb = min(BLU_NB, n - k0);
-  __shared__ int rows[2 * BLU_NB];  // touched rows (panel-relative), then the moved ones
-  __shared__ int held[2 * BLU_NB];  // the original row whose value rows[i] holds
-  __shared__ int dst[2 * BLU_NB], srcr[2 * BLU_NB];
-  __shared__ int cnt;
-  if (threadIdx.x == 0) {
-    int nr = nb;
-    for (int kk = 0; kk < nb; ++kk) {
-      rows[kk] = kk;
-      held[kk] = kk;
-    }
-    for (int kk = 0; kk < nb; ++kk) {
-      const int p = piv_ws[static_cast<long>(blockIdx.x) * LU_PIV_WS + kk];
-      if (p == kk) continue;
-      int pos = p;
-      if (p >= nb) {
-        pos = -1;
-        for (int i = nb; i < nr; ++i)
-          if (rows[i] == p) pos = i;
-        if (pos < 0) {
-          rows[nr] = p;
-          held[nr] = p;
-          pos = nr++;
-        }
-      }
-      const int t = held[kk];
-      held[kk] = held[pos];
-      held[pos] = t;
-    }
-    int c = 0;
-    for (int i = 0; i < nr; ++i)
-      if (held[i] != rows[i]) {
-        dst[c] = rows[i];
-        srcr[c] = held[i];
-        ++c;
-      }
-    cnt = c;
-  }
-  __syncthreads();
-  const int j = k0 + nb + blockIdx.y * 64 + threadIdx.x;
-  if (j >= ncols) return;
-  T* colj = A + static_cast<long>(n) * j + k0;
-  const int nm = cnt;
-  T v[2 * BLU_NB];
-#pragma unroll
-  for (int i = 0; i < 2 * BLU_NB; ++i)
-    if (i < nm) v[i] = colj[srcr[i]];
-#pragma unroll
-  for (int i = 0; i < 2 * BLU_NB; ++i)
-    if (i < nm) colj[dst[i]] = v[i];
-}
-
-// Columns right of a panel factored by k_lu_panel_reg, after k_lu_swap: U12 = L11^{-1} A12 (one
-// column per thread; blockIdx.y selects a chunk of 256 columns).  Each thread reads its column's
-// nb contiguous entries; a variant with one wave per 64 columns staged through LDS with coalesced
-// loads was measured slower (0.47 against 0.33 ms per launch, averaged over the FP64 LUs of the
-// 32^3, p = 4 mesh's set-up and assembly; k_lu_back 0.31 against 0.26 ms): the LDS tile cut
-// occupancy.
-template <typename T, int BLU_NB>
-__global__ __launch_bounds__(256) void k_lu_u12(T* Aall, int n, int ncols, long stride, int k0,
-                                                const int* piv_ws) {
-  T* A = Aall + stride * blockIdx.x;
-  const int nb = min(BLU_NB, n - k0);
-  // L11 with a run-time leading dimension: constant LDS addresses in the unrolled solve let the
-  // compiler hoist every load into registers (and spill)
-  __shared__ T L11[BLU_NB * BLU_NB];
-  const int ldl = nb;
-  const int tid = threadIdx.x;
-  for (int idx = tid; idx < nb * nb; idx += 256) {
-    const int r = idx % nb, c = idx / nb;
-    L11[r + ldl * c] = A[k0 + r + static_cast<long>(n) * (k0 + c)];
-  }
-  __syncthreads();
-  const int j = k0 + nb + blockIdx.y * 256 + tid;
-  if (j >= ncols) return;
-  T* colj = A + static_cast<long>(n) * j + k0;
-  T x[BLU_NB];
-#pragma unroll
-  for (int kk = 0; kk < BLU_NB; ++kk) x[kk] = (kk < nb) ? colj[kk] : 0.0;
-#pragma unroll
-  for (int kk = 1; kk < BLU_NB; ++kk)
-#pragma unroll
-    for (int t = 0; t < kk; ++t)
-      if (kk < nb) x[kk] = fma(-L11[kk + ldl * t], x[t], x[kk]);
-#pragma unroll
-  for (int kk = 0; kk < BLU_NB; ++kk)
-    if (kk < nb) colj[kk] = x[kk];
-}
-
-// Inverse of the unit lower triangle L11 (LOWER) or of the upper triangle U11 of the panel at
-// k0, one workgroup per matrix: thread c computes column c by substitution (static register
-// indices, predicated on c), written to W[blockIdx.x] (nb x nb, ld BLU_NB).  U12 = L11^{-1} A12
-// and X = U11^{-1} X then run as in-place GEMMs on the matrix cores: each output tile covers all
-// nb rows of its own columns, so it reads its B columns completely before writing them.
-template <typename T, int BLU_NB, bool LOWER>
-__global__ __launch_bounds__(64) void k_lu_tri_inv(const T* Aall, int n, long stride, int k0, T* W) {
-  const T* A = Aall + stride * blockIdx.x;
-  const int nb = min(BLU_NB, n - k0);
-  __shared__ T Ts[BLU_NB][BLU_NB + 1];
-  for (int idx = threadIdx.x; idx < nb * nb; idx += 64) {
-    const int r = idx % nb, c = idx / nb;
-    Ts[r][c] = A[k0 + r + static_cast<long>(n) * (k0 + c)];
-  }
-  __syncthreads();
-  const int c = threadIdx.x;
-  if (c >= nb) return;
-  T y[BLU_NB];
-  if (LOWER) {
-#pragma unroll
-    for (int r = 0; r < BLU_NB; ++r) {
-      if (r <= c || r >= nb) {
-        y[r] = (r == c) ? T(1) : T(0);
-      } else {
-        T s = T(0);
-#pragma unroll
-        for (int t = 0; t < r; ++t)
-          if (t >= c) s = fma(Ts[r][t], y[t], s);
-        y[r] = -s;
-      }
-    }
-  } else {
-#pragma unroll
-    for (int r = BLU_NB - 1; r >= 0; --r) {
-      if (r > c || r >= nb) {
-        y[r] = T(0);
-      } else if (r == c) {
-        y[r] = T(1) / Ts[r][r];
-      } else {
-        T s = T(0);
-#pragma unroll
-        for (int t = r + 1; t < BLU_NB; ++t)
-          if (t <= c) s = fma(Ts[r][t], y[t], s);
-        y[r] = -s / Ts[r][r];
-      }
-    }
-  }
-  T* Wm = W + static_cast<long>(blockIdx.x) * BLU_NB * BLU_NB;
-#pragma unroll
-  for (int r = 0; r < BLU_NB; ++r)
-    if (r < nb) Wm[r + BLU_NB * c] = y[r];
-}
-
-// X[k0:k0+nb, c] = U11^{-1} X[k0:k0+nb, c] for the right-hand-side columns c >= n
-template <typename T, int BLU_NB>
-__global__ __launch_bounds__(256) void k_lu_back(T* Aall, int n, int ncols, long stride, int k0) {
-  T* A = Aall + stride * blockIdx.x;
-  const int nb = min(BLU_NB, n - k0);
-  __shared__ T U[BLU_NB][BLU_NB + 1];
-  __shared__ T dinv[BLU_NB];
-  const int tid = threadIdx.x;
-  for (int idx = tid; idx < nb * nb; idx += 256) {
-    int r = idx % nb, c = idx / nb;
-    U[r][c] = A[k0 + r + static_cast<long>(n) * (k0 + c)];
-  }
-  __syncthreads();
-  if (tid < nb) dinv[tid] = T(1) / U[tid][tid];
-  __syncthreads();
-  // one right-hand-side column per thread (blockIdx.y selects a chunk of 256)
-  const int j = n + blockIdx.y * 256 + tid;
-  if (j >= ncols) return;
-  T* colj = A + static_cast<long>(n) * j + k0;
-  T x[BLU_NB];
-#pragma unroll
-  for (int kk = 0; kk < BLU_NB; ++kk) x[kk] = (kk < nb) ? colj[kk] : 0.0;
-#pragma unroll
-  for (int kk = BLU_NB - 1; kk >= 0; --kk) {
-    if (kk < nb) {
-      x[kk] *= dinv[kk];
-#pragma unroll
-      for (int t = 0; t < kk; ++t) x[t] = fma(-U[t][kk], x[kk], x[t]);
-    }
-  }
-#pragma unroll
-  for (int kk = 0; kk < BLU_NB; ++kk)
-    if (kk < nb) colj[kk] = x[kk];
-}
-
-// ---------------------------------------------------------------------------
-// Blocked LU with partial pivoting + back substitution, one workgroup per matrix.
-// ---------------------------------------------------------------------------
-constexpr int LU_NB = 16;
-constexpr int LU_CH = 64;
-
-__global__ __launch_bounds__(256) void k_lu_solve(double* Aall, int n, int ncols, long stride,
-                                                  int* info) {
-  double* A = Aall + stride * blockIdx.x;
-  extern __shared__ double P[];  // n x LU_NB panel (ld n)
-  __shared__ double Us[LU_NB][LU_CH + 1];
-  __shared__ double redv[256];
-  __shared__ int redi[256];
-  __shared__ int piv[LU_NB];
-  const int tid = threadIdx.x;
-  int singular = 0;
-  for (int k0 = 0; k0 < n; k0 += LU_NB) {
-    const int nb = min(LU_NB, n - k0);
-    const int rows = n - k0;
-    for (int idx = tid; idx < rows * nb; idx += 256) {
-      int r = k0 + idx % rows, kk = idx / rows;
-      P[r + n * kk] = A[r + static_cast<long>(n) * (k0 + kk)];
-    }
-    __syncthreads();
-    for (int kk = 0; kk < nb; ++kk) {
-      const int col = k0 + kk;
-      double best = -1.0;
-      int bi = col;
-      for (int r = col + tid; r < n; r += 256) {
-        double v = fabs(P[r + n * kk]);
-        if (v > best) { best = v; bi = r; }
-      }
-      redv[tid] = best;
-      redi[tid] = bi;
-      __syncthreads();
-      for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) {
-          double o = redv[tid + s];
-          int oi = redi[tid + s];
-          if (o > redv[tid] || (o == redv[tid] && oi < redi[tid])) { redv[tid] = o; redi[tid] = oi; }
-        }
-        __syncthreads();
-      }
-      const int p = redi[0];
-      if (tid == 0) piv[kk] = p;
-      if (p != col && tid < nb) {
-        double t = P[col + n * tid];
-        P[col + n * tid] = P[p + n * tid];
-        P[p + n * tid] = t;
-      }
-      __syncthreads();
-      const double pv = P[col + n * kk];
-      if (pv == 0.0) singular = 1;
-      for (int r = col + 1 + tid; r < n; r += 256) P[r + n * kk] /= pv;
-      __syncthreads();
-      const int rr = n - col - 1, cc = nb - kk - 1;
-      for (int idx = tid; idx < rr * cc; idx += 256) {
-        int r = col + 1 + idx % rr, c = kk + 1 + idx / rr;
-        P[r + n * c] -= P[r + n * kk] * P[col + n * c];
-      }
-      __syncthreads();
-    }
-    for (int idx = tid; idx < rows * nb; idx += 256) {
-      int r = k0 + idx % rows, kk = idx / rows;
-      A[r + static_cast<long>(n) * (k0 + kk)] = P[r + n * kk];
-    }
-    for (int j = tid; j < ncols; j += 256) {
-      if (j >= k0 && j < k0 + nb) continue;
-      double* colj = A + static_cast<long>(n) * j;
-      for (int kk = 0; kk < nb; ++kk) {
-        int p = piv[kk], r = k0 + kk;
-        if (p != r) { double t = colj[r]; colj[r] = colj[p]; colj[p] = t; }
-      }
-    }
-    __syncthreads();
-    for (int j = k0 + nb + tid; j < ncols; j += 256) {
-      double* colj = A + static_cast<long>(n) * j;
-      double x[LU_NB];
-#pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk) x[kk] = (kk < nb) ? colj[k0 + kk] : 0.0;
-#pragma unroll
-      for (int kk = 1; kk < LU_NB; ++kk)
-#pragma unroll
-        for (int t = 0; t < kk; ++t)
-          if (kk < nb) x[kk] -= P[k0 + kk + n * t] * x[t];
-#pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk)
-        if (kk < nb) colj[k0 + kk] = x[kk];
-    }
-    __syncthreads();
-    const int R = n - k0 - nb;
-    if (R > 0) {
-      for (int j0 = k0 + nb; j0 < ncols; j0 += LU_CH) {
-        const int cw = min(LU_CH, ncols - j0);
-        for (int idx = tid; idx < nb * cw; idx += 256) {
-          int t = idx % nb, c = idx / nb;
-          Us[t][c] = A[k0 + t + static_cast<long>(n) * (j0 + c)];
-        }
-        __syncthreads();
-        for (int idx = tid; idx < R * cw; idx += 256) {
-          int r = k0 + nb + idx % R, c = idx / R;
-          double* a = A + r + static_cast<long>(n) * (j0 + c);
-          double s = *a;
-          for (int t = 0; t < nb; ++t) s -= P[r + n * t] * Us[t][c];
-          *a = s;
-        }
-        __syncthreads();
-      }
-    }
-  }
-  // back substitution U X = Y for the right-hand-side columns
-  const int last = ((n - 1) / LU_NB) * LU_NB;
-  for (int k0 = last; k0 >= 0; k0 -= LU_NB) {
-    const int nb = min(LU_NB, n - k0);
-    const int rows = k0 + nb;
-    for (int idx = tid; idx < rows * nb; idx += 256) {
-      int r = idx % rows, kk = idx / rows;
-      P[r + n * kk] = A[r + static_cast<long>(n) * (k0 + kk)];
-    }
-    __syncthreads();
-    for (int j = n + tid; j < ncols; j += 256) {
-      double* colj = A + static_cast<long>(n) * j;
-      double x[LU_NB];
-#pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk) x[kk] = (kk < nb) ? colj[k0 + kk] : 0.0;
-#pragma unroll
-      for (int kk = LU_NB - 1; kk >= 0; --kk) {
-        if (kk < nb) {
-          double s = x[kk];
-#pragma unroll
-          for (int t = kk + 1; t < LU_NB; ++t)
-            if (t < nb) s -= P[k0 + kk + n * t] * x[t];
-          x[kk] = s / P[k0 + kk + n * kk];
-        }
-      }
-#pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk)
-        if (kk < nb) colj[k0 + kk] = x[kk];
-    }
-    __syncthreads();
-    if (k0 > 0) {
-      for (int j0 = n; j0 < ncols; j0 += LU_CH) {
-        const int cw = min(LU_CH, ncols - j0);
-        for (int idx = tid; idx < nb * cw; idx += 256) {
-          int t = idx % nb, c = idx / nb;
-          Us[t][c] = A[k0 + t + static_cast<long>(n) * (j0 + c)];
-        }
-        __syncthreads();
-        for (int idx = tid; idx < k0 * cw; idx += 256) {
-          int r = idx % k0, c = idx / k0;
-          double* a = A + r + static_cast<long>(n) * (j0 + c);
-          double s = *a;
-          for (int t = 0; t < nb; ++t) s -= P[r + n * t] * Us[t][c];
-          *a = s;
-        }
-        __syncthreads();
-      }
-    }
-  }
-  if (tid == 0 && info) info[blockIdx.x] = singular;
-}
-
-// ---------------------------------------------------------------------------
 // Geometry and setup
 // ---------------------------------------------------------------------------
 __device__ inline void adjugate(int nd, const double J[3][3], double* jac, double Xx[9]) {
@@ -2292,69 +1747,6 @@ __global__ void k_to_float_2d(float* dst, const S* src, long per, long sstride, 
   dst[b * dstride + rc] = static_cast<float>(src[b * sstride + rc]);
 }
 
-// One workgroup per element: RuS = D'^{-1} Ru from the stored FP32 LU factors of
-// D' (replaying the blocked factorisation: each panel's row exchanges, then the
-// unit-lower elimination), the upper-triangular solve, then Rh -= K' RuS.  The
-// panel width nbp is the one lu_solve used for the factorisation.
-__global__ __launch_bounds__(256) void k_refine_rhs(Dims d, int nbp, const float* LU, const int* piv,
-                                                    const float* K, const double* Ru, double* RuS,
-                                                    double* Rh) {
-  const int n = d.n, m = d.m;
-  const long e = blockIdx.x;
-  extern __shared__ double sm[];
-  double* y = sm;   // n
-  const float* Le = LU + e * static_cast<long>(n) * n;
-  const int* pe = piv + e * static_cast<long>(n);
-  for (int t = threadIdx.x; t < n; t += 256) y[t] = Ru[e * n + t];
-  __syncthreads();
-  for (int k0 = 0; k0 < n; k0 += nbp) {
-    const int nb = min(nbp, n - k0);
-    if (threadIdx.x == 0)
-      for (int kk = 0; kk < nb; ++kk) {
-        const int p = k0 + pe[k0 + kk];
-        if (p != k0 + kk) {
-          const double t = y[k0 + kk];
-          y[k0 + kk] = y[p];
-          y[p] = t;
-        }
-      }
-    __syncthreads();
-    for (int k = k0; k < k0 + nb; ++k) {
-      const double yk = y[k];
-      for (int r = k + 1 + threadIdx.x; r < n; r += 256)
-        y[r] = fma(-static_cast<double>(Le[r + static_cast<long>(n) * k]), yk, y[r]);
-      __syncthreads();
-    }
-  }
-  for (int k = n - 1; k >= 0; --k) {
-    if (threadIdx.x == 0) y[k] /= static_cast<double>(Le[k + static_cast<long>(n) * k]);
-    __syncthreads();
-    const double yk = y[k];
-    for (int r = threadIdx.x; r < k; r += 256)
-      y[r] = fma(-static_cast<double>(Le[r + static_cast<long>(n) * k]), yk, y[r]);
-    __syncthreads();
-  }
-  for (int t = threadIdx.x; t < n; t += 256) RuS[e * n + t] = y[t];
-  const float* Ke = K + e * static_cast<long>(m) * n;
-  for (int r = threadIdx.x; r < m; r += 256) {
-    double acc = 0.0;
-    for (int c = 0; c < n; ++c) acc = fma(static_cast<double>(Ke[r + static_cast<long>(m) * c]), y[c], acc);
-    Rh[e * m + r] -= acc;
-  }
-}
-
-// panel width lu_solve uses for an n x n factorisation (see lu_solve).  64-wide panels (up to
-// 150 KB of LDS at n = 300) were measured slower: one workgroup per CU leaves the latency-bound
-// panel factorisation without company (C2 LU 0.36 s -> 0.55 s per assembly).
-int lu_panel_width(int n) { return (static_cast<size_t>(n) * 32 * sizeof(double) <= 64000) ? 32 : 16; }
-// the FP32 LU (the mixed form): 64-wide panels up to n = 250 (an n x 64 FP32 panel in 64 KB of LDS,
-// 64 registers per row in the register panel), which halves the passes of the bandwidth-bound
-// trailing update; 32 or 16 beyond
-int lu_panel_width_f32(int n) {
-  if (n <= 250) return 64;
-  return (static_cast<size_t>(n) * 32 * sizeof(float) <= 64000) ? 32 : 16;
-}
-
 // ---------------------------------------------------------------------------
 // Vector kernels (fixed-order reductions)
 // ---------------------------------------------------------------------------
@@ -2673,136 +2065,6 @@ int generated_model(const std::string& name, int* nd, int* ncu, int* nv) {
   return -1;
 }
 
-// operands of a GEMM inside the LU: FP64 storage and products, or FP32 storage and products
-inline void lu_gemm_ptrs(Gemm& g, const double* A, const double* B, double* C) {
-  g.A = A;
-  g.B = B;
-  g.C = C;
-}
-inline void lu_gemm_ptrs(Gemm& g, const float* A, const float* B, float* C) {
-  g.Af = A;
-  g.Bf = B;
-  g.Cf = C;
-  g.fp32 = 1;
-}
-
-template <typename T, int NB>
-void blocked_lu(T* A, int n, int ncols, long stride, int batch, int* info, int* pivout, hipStream_t s,
-                int* piv_ws, T* tri_ws) {
-  // X[r0 : r0+nb, cols] = Tinv X[r0 : r0+nb, cols] in place (Tinv in tri_ws, ld NB)
-  auto apply_tri = [&](int nb, int r0, long c0, int ncol) {
-    Gemm g{};
-    g.M = nb; g.N = ncol; g.K = nb; g.alpha = 1.0; g.beta = 0.0;
-    T* X = A + r0 + static_cast<long>(n) * c0;
-    lu_gemm_ptrs(g, tri_ws, X, X);
-    g.lda = NB; g.sA0 = static_cast<long>(NB) * NB;
-    g.ldb = n; g.sB0 = stride;
-    g.ldc = n; g.sC0 = stride;
-    g.nb0 = batch; g.nb1 = 1; g.nb2 = 1;
-    gemm(g, s);
-  };
-  for (int k0 = 0; k0 < n; k0 += NB) {
-    const int nb = std::min(NB, n - k0);
-    if (piv_ws && n - k0 <= 256) {
-      k_lu_panel_reg<T, NB><<<batch, 256, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws);
-      const int right = ncols - k0 - nb;
-      if (right > 0) {
-        k_lu_swap<T, NB><<<dim3(batch, (right + 63) / 64), 64, 0, s>>>(A, n, ncols, stride, k0, piv_ws);
-        if (tri_ws) {
-          k_lu_tri_inv<T, NB, true><<<batch, 64, 0, s>>>(A, n, stride, k0, tri_ws);
-          apply_tri(nb, k0, k0 + nb, right);
-        } else {
-          k_lu_u12<T, NB><<<dim3(batch, (right + 255) / 256), 256, 0, s>>>(A, n, ncols, stride, k0, piv_ws);
-        }
-      }
-    } else {
-      size_t shm = static_cast<size_t>(n - k0) * nb * sizeof(T);
-      k_lu_panel<T, NB><<<batch, 256, shm, s>>>(A, n, ncols, stride, k0, info, pivout);
-    }
-    EXA_HIP(hipGetLastError());
-    if (k0 + nb < n) {  // A22 -= L21 * U12
-      Gemm g{};
-      g.M = n - k0 - nb; g.N = ncols - k0 - nb; g.K = nb; g.alpha = -1.0; g.beta = 1.0;
-      lu_gemm_ptrs(g, A + (k0 + nb) + static_cast<long>(n) * k0, A + k0 + static_cast<long>(n) * (k0 + nb),
-                   A + (k0 + nb) + static_cast<long>(n) * (k0 + nb));
-      g.lda = n; g.sA0 = stride;
-      g.ldb = n; g.sB0 = stride;
-      g.ldc = n; g.sC0 = stride;
-      g.nb0 = batch; g.nb1 = 1; g.nb2 = 1;
-      gemm(g, s);
-    }
-  }
-  const int last = ((n - 1) / NB) * NB;
-  for (int k0 = last; k0 >= 0; k0 -= NB) {
-    if (tri_ws) {
-      k_lu_tri_inv<T, NB, false><<<batch, 64, 0, s>>>(A, n, stride, k0, tri_ws);
-      EXA_HIP(hipGetLastError());
-      apply_tri(std::min(NB, n - k0), k0, n, ncols - n);
-    } else {
-      dim3 grid(static_cast<unsigned>(batch), static_cast<unsigned>((ncols - n + 255) / 256));
-      k_lu_back<T, NB><<<grid, 256, 0, s>>>(A, n, ncols, stride, k0);
-      EXA_HIP(hipGetLastError());
-    }
-    if (k0 > 0) {  // X[0:k0] -= U[0:k0, k0:k0+nb] * X[k0:k0+nb]
-      const int nb = std::min(NB, n - k0);
-      Gemm g{};
-      g.M = k0; g.N = ncols - n; g.K = nb; g.alpha = -1.0; g.beta = 1.0;
-      lu_gemm_ptrs(g, A + static_cast<long>(n) * k0, A + k0 + static_cast<long>(n) * n, A + static_cast<long>(n) * n);
-      g.lda = n; g.sA0 = stride;
-      g.ldb = n; g.sB0 = stride;
-      g.ldc = n; g.sC0 = stride;
-      g.nb0 = batch; g.nb1 = 1; g.nb2 = 1;
-      gemm(g, s);
-    }
-  }
-}
-
-template <typename T>
-void lu_blocked_any(T* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s, int* pivout,
-                    int* piv_ws, T* tri_ws) {
-  // 32-wide panels when an n x 32 panel fits the 64 KB of LDS, else 16-wide; with a pivot
-  // workspace, panels of up to 256 rows are factored in registers (64-wide register panels
-  // were measured: no gain at n = 250, slower at n = 100)
-  const int w = sizeof(T) == 4 ? lu_panel_width_f32(n) : lu_panel_width(n);
-  if constexpr (sizeof(T) == 4) {
-    if (w == 64) {
-      blocked_lu<T, 64>(A, n, ncols, stride, batch, info, pivout, s, piv_ws, tri_ws);
-      return;
-    }
-  }
-  if (w == 32)
-    blocked_lu<T, 32>(A, n, ncols, stride, batch, info, pivout, s, piv_ws, tri_ws);
-  else if (static_cast<size_t>(n) * 16 * sizeof(T) <= 64000)
-    blocked_lu<T, 16>(A, n, ncols, stride, batch, info, pivout, s, piv_ws, tri_ws);
-  else
-    throw Error(5, "dense block larger than 500 rows");
-}
-
-void lu_solve(double* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s, int* pivout,
-              int* piv_ws, void* tri_ws) {
-  if (batch <= 0) return;
-  // the FP64 form keeps the substitution kernels (k_lu_u12, k_lu_back): explicit triangle inverses
-  // amplify rounding by the triangle's condition number, which the FP64 form is not allowed to lose
-  (void)tri_ws;
-  if ((n >= BLU_MIN_N || pivout) && ncols > n) {
-    lu_blocked_any(A, n, ncols, stride, batch, info, s, pivout, piv_ws, static_cast<double*>(nullptr));
-    return;
-  }
-  if (pivout) throw Error(5, "pivot output needs right-hand-side columns");
-  // dynamic LDS panel n x LU_NB doubles next to ~12 KB of static LDS, kept within 64 KB
-  if (n > 400) throw Error(5, "dense block larger than 400 rows");
-  size_t shm = static_cast<size_t>(n) * LU_NB * sizeof(double);
-  k_lu_solve<<<batch, 256, shm, s>>>(A, n, ncols, stride, info);
-  EXA_HIP(hipGetLastError());
-}
-
-void lu_solve(float* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s, int* pivout,
-              int* piv_ws, void* tri_ws) {
-  if (batch <= 0) return;
-  if (ncols <= n) throw Error(5, "FP32 LU needs right-hand-side columns");
-  lu_blocked_any(A, n, ncols, stride, batch, info, s, pivout, piv_ws, static_cast<float*>(tri_ws));
-}
-
 void elem_geom(const Dims& d, const double* shapegt, const double* xdg, double* egeo, hipStream_t s) {
   long P = static_cast<long>(d.ne) * d.nge;
   k_elem_geom<<<nblocks(P, 256), 256, 0, s>>>(d, shapegt, xdg, egeo);
@@ -3053,13 +2315,6 @@ void to_bf16_t(unsigned short* dst, const S* src, long count, hipStream_t s) {
 }
 void to_bf16(unsigned short* dst, const double* src, long count, hipStream_t s) { to_bf16_t(dst, src, count, s); }
 void to_bf16(unsigned short* dst, const float* src, long count, hipStream_t s) { to_bf16_t(dst, src, count, s); }
-
-void refine_rhs(const Dims& d, const float* LU, const int* piv, const float* K, const double* Ru, double* RuS,
-                double* Rh, hipStream_t s) {
-  size_t shm = static_cast<size_t>(d.n) * sizeof(double);
-  k_refine_rhs<<<d.ne, 256, shm, s>>>(d, lu_panel_width_f32(d.n), LU, piv, K, Ru, RuS, Rh);
-  EXA_HIP(hipGetLastError());
-}
 
 void face_gather(long nnodes, int ncu, const long* src1, const long* src2, const double* we, double* w,
                  hipStream_t s) {

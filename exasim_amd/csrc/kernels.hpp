@@ -80,7 +80,7 @@ void lu_solve(float* A, int n, int ncols, long stride, int batch, int* info, hip
 // tri_ws (optional, device, >= LU_TRI_WS*batch doubles, owned by the caller): with it, the FP32
 // LU runs the triangular solves of each panel (U12 = L11^{-1} A12, X = U11^{-1} X) as an explicit
 // triangle inverse and an in-place GEMM (the FP64 LU always uses substitution)
-constexpr int LU_PIV_WS = 64;
+constexpr int LU_PIV_WS = 260;  // the moved rows of a panel of 64 columns: their number, (new, old) of each
 constexpr long LU_TRI_WS = 64L * 64L;
 
 // ---- setup ----
@@ -256,8 +256,8 @@ void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const double* 
                 hipStream_t s);
 void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const float* Ltmp, float* BE, hipStream_t s);
 // Rh_e -= K_e u_e of the eb elements of a block: K [m, n, eb], u_e = U + su e (n values), Rh [m, eb]
-template <typename T>
-void trace_rhs(const Dims& d, int eb, const T* K, const T* U, long su, double* Rh, hipStream_t s);
+template <typename T, typename TU>
+void trace_rhs(const Dims& d, int eb, const T* K, const TU* U, long su, double* Rh, hipStream_t s);
 template <typename T>
 void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Y, double* Xo,
                 double* out, hipStream_t s, const double* act = nullptr);

@@ -198,15 +198,15 @@ void small_vw(const Dims& d, const T* H, const int* elemcon, const double* v, do
 // [D | F | Ru]).  One workgroup per element: its four waves split the n columns, lanes hold VW rows
 // and, below 64 VW rows, G columns side by side, 8 loads in flight; FP64 sums in a fixed order.
 // Bound by reading K_e, which the K D^{-1}F product before it has just read.
-template <typename T, int VW>
-__global__ __launch_bounds__(256) void k_trace_rhs(int m, int n, const T* K, const T* U, long su, double* Rh) {
+template <typename T, typename TU, int VW>
+__global__ __launch_bounds__(256) void k_trace_rhs(int m, int n, const T* K, const TU* U, long su, double* Rh) {
   typedef T vecT __attribute__((ext_vector_type(VW)));
   constexpr int U8 = 8;
   __shared__ double red[4 * 64 * VW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long e = blockIdx.x;
   const T* Ke = K + e * static_cast<long>(m) * n;
-  const T* u = U + e * su;
+  const TU* u = U + e * su;
   double* out = Rh + e * m;
   const int cper = (n + 3) / 4;
   const int c0 = wave * cper, c1 = min(n, c0 + cper);
@@ -279,18 +279,19 @@ void matvec_elem(const Dims& d, const T* H, const int* elemcon, const double* v,
   EXA_HIP(hipGetLastError());
 }
 
-template <typename T>
-void trace_rhs(const Dims& d, int eb, const T* K, const T* U, long su, double* Rh, hipStream_t s) {
+template <typename T, typename TU>
+void trace_rhs(const Dims& d, int eb, const T* K, const TU* U, long su, double* Rh, hipStream_t s) {
   if (eb <= 0) return;
   constexpr int VMAX = 16 / sizeof(T);
-  if (d.m % VMAX == 0) k_trace_rhs<T, VMAX><<<eb, 256, 0, s>>>(d.m, d.n, K, U, su, Rh);
-  else if (d.m % 2 == 0) k_trace_rhs<T, 2><<<eb, 256, 0, s>>>(d.m, d.n, K, U, su, Rh);
-  else k_trace_rhs<T, 1><<<eb, 256, 0, s>>>(d.m, d.n, K, U, su, Rh);
+  if (d.m % VMAX == 0) k_trace_rhs<T, TU, VMAX><<<eb, 256, 0, s>>>(d.m, d.n, K, U, su, Rh);
+  else if (d.m % 2 == 0) k_trace_rhs<T, TU, 2><<<eb, 256, 0, s>>>(d.m, d.n, K, U, su, Rh);
+  else k_trace_rhs<T, TU, 1><<<eb, 256, 0, s>>>(d.m, d.n, K, U, su, Rh);
   EXA_HIP(hipGetLastError());
 }
 
 template void trace_rhs<double>(const Dims&, int, const double*, const double*, long, double*, hipStream_t);
 template void trace_rhs<float>(const Dims&, int, const float*, const float*, long, double*, hipStream_t);
+template void trace_rhs<float>(const Dims&, int, const float*, const double*, long, double*, hipStream_t);
 template void matvec_elem<double>(const Dims&, const double*, const int*, const double*, double*, hipStream_t,
                                   const int*, const double*);
 template void matvec_elem<float>(const Dims&, const float*, const int*, const double*, double*, hipStream_t,
