@@ -2478,13 +2478,13 @@ void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, do
                                   static_cast<int>(shm)));
     kern<<<I.nse, 256, shm, s>>>(d, I, BE, x, Xo, act);
   };
-  // one wave per superelement for FP32 / BF16 factors when a wave covers a block's rows
+  // one wave per superelement for small blocks, and for BF16 factors when a wave covers a block's rows
   const size_t shm_w = (static_cast<size_t>(I.nfse) * d.ncf + d.ncf) * sizeof(float);
-  bool wave = false;
+  bool wave = bilu_wave_enabled() && bilu_apply_small(d, I, BE, x, Xo, act, s);
   if constexpr (sizeof(T) == 2) {
     // the one-wave kernel's shapes: ncf = 50 (p = 4, two components on hex faces): 25 row pairs,
     // 2 parts of 25 columns
-    if (d.ncf == 50 && shm_w <= 64 * 1024 && I.wseg && bilu_wave_enabled()) {
+    if (!wave && d.ncf == 50 && shm_w <= 64 * 1024 && I.wseg && bilu_wave_enabled()) {
       wave = true;
       k_bilu_apply_wave<T, 2, 50><<<I.nse, 64, shm_w, s>>>(d, I, BE, x, Xo, act);
     }

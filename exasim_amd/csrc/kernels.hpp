@@ -56,7 +56,7 @@ void face_elim(const FaceElim<T>& f, hipStream_t s);
 // the tile autotuner of gemm (gemm.hip): mode 1 times the workgroup tiles on the first call of each
 // product shape, 0 always takes the default tile, -1 follows EXA_GEMM_AUTOTUNE (default 1)
 void set_gemm_autotune(int mode);
-// the block-ILU(0) apply of FP32 / BF16 factors: 1 one wave per superelement, 0 the 256-thread
+// the block-ILU(0) apply of small blocks and of BF16 factors: 1 one wave per superelement, 0 the 256-thread
 // kernel, -1 follows EXA_BILU_WAVE (default 1)
 void set_bilu_wave(int mode);
 // every product on tile 0..4 (64x64 32x64 64x32 128x64 64x128), or -1: the tuner's choice
@@ -233,6 +233,7 @@ void u_insert(const Dims& d, const double* src, double* udg, hipStream_t s);
 
 // ---- superelement block-ILU(0) (preconditioner = 2) ----
 struct IluDev {
+  int nprog;  // blocks in the apply's program (wblk, wvec)
   int nse, nfse, nnz;
   const int *face, *row_ptr, *col_ind, *row_of, *diag;
   const int *eptr, *elim_ji, *uptr, *upd_jl, *upd_il, *upd_ji;
@@ -258,6 +259,10 @@ void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const float* L
 // Rh_e -= K_e u_e of the eb elements of a block: K [m, n, eb], u_e = U + su e (n values), Rh [m, eb]
 template <typename T, typename TU>
 void trace_rhs(const Dims& d, int eb, const T* K, const TU* U, long su, double* Rh, hipStream_t s);
+// Xo of small face blocks with one wave per superelement (bilu.hip); false: the shape needs another kernel
+template <typename T>
+bool bilu_apply_small(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Xo, const double* act,
+                      hipStream_t s);
 template <typename T>
 void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Y, double* Xo,
                 double* out, hipStream_t s, const double* act = nullptr);

@@ -583,6 +583,7 @@ void Solver::setup_bilu0() {
       wvec.push_back(ilu.nfse * d.ncf);
       wseg.push_back(static_cast<int>(wblk.size()));
     }
+    ilud.nprog = static_cast<int>(wblk.size());
     ilud.wseg = up(iwseg, wseg);
     ilud.wblk = up(iwblk, wblk);
     ilud.wvec = up(iwvec, wvec);
