@@ -60,8 +60,7 @@ void Solver::gmres_step(const GmresDev& g, int i, double* xv) {
   const long N = d.N;
   double* vi = V.p + N * i;
   double* vm = V.p + N * (i + 1);
-  matvec(vi, tmp.p);
-  apply_precond_to(tmp.p, vm);
+  matvec_precond(vi, vm);
   hipEvent_t t0{};
   tic(T_ORTHO, &t0);
   SegMap ma = segT.map;

@@ -1231,22 +1231,6 @@ __global__ void k_bj_extract(Dims d, const double* aug, double* BE) {
   BE[q] = aug[f * 2 * per + per + q % per];
 }
 
-// x_f <- BE_f x_f (preconditioner.cpp:282-292); one thread per row.
-template <typename T>
-__global__ void k_bj_apply(Dims d, const T* BE, const double* x, double* y, const double* act) {
-  if (act && act[0] == 0.0) return;
-  const int ncf = d.ncf;
-  const long q = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (q >= static_cast<long>(ncf) * d.nf) return;
-  const long f = q / ncf;
-  const int r = static_cast<int>(q % ncf);
-  const T* B = BE + f * ncf * static_cast<long>(ncf);
-  const double* xf = x + f * ncf;
-  double s = 0.0;
-  for (int c = 0; c < ncf; ++c) s += static_cast<double>(B[r + static_cast<long>(ncf) * c]) * xf[c];
-  y[q] = s;
-}
-
 // hdgGetDUDG (matvec.cpp:219-238): du_e = Ru_e + DinvF_e * x_e.  One workgroup per element: the
 // element's trace values x_e are gathered into LDS once, then one thread per row reads DinvF_e
 // along its columns (the sum runs over t in order).
@@ -2376,13 +2360,6 @@ void bj_extract(const Dims& d, const double* aug, double* BE, hipStream_t s) {
 }
 
 template <typename T>
-void bj_apply(const Dims& d, const T* BE, const double* x, double* y, hipStream_t s, const double* act) {
-  long n1 = static_cast<long>(d.ncf) * d.nf;
-  k_bj_apply<T><<<nblocks(n1, 256), 256, 0, s>>>(d, BE, x, y, act);
-  EXA_HIP(hipGetLastError());
-}
-
-template <typename T>
 void dudg(const Dims& d, const double* RuS, const T* DinvF, const int* elemcon, const double* x,
           double* du, hipStream_t s) {
   if (d.ne <= 0) return;
@@ -2542,8 +2519,6 @@ void fill(double* y, double v, long n, hipStream_t s) {
   EXA_HIP(hipGetLastError());
 }
 
-template void bj_apply<double>(const Dims&, const double*, const double*, double*, hipStream_t, const double*);
-template void bj_apply<float>(const Dims&, const float*, const double*, double*, hipStream_t, const double*);
 template void dudg<double>(const Dims&, const double*, const double*, const int*, const double*, double*,
                            hipStream_t);
 template void dudg<float>(const Dims&, const double*, const float*, const int*, const double*, double*,

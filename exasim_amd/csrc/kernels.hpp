@@ -200,6 +200,13 @@ void refine_rhs(const Dims& d, const float* LU, const int* piv, const float* K, 
                 double* Rh, hipStream_t s);
 
 // ---- global system ----
+// Input of the element and face products: the trace vector v, or the element products v of a preceding
+// matvec_elem to be summed per face node through src1 / src2 (as face_gather does).  con: the nodes' map.
+struct TraceIn {
+  const double* v;
+  const int* con;
+  const long *src1, *src2;
+};
 void face_gather(long nnodes, int ncu, const long* src1, const long* src2, const double* we, double* w,
                  hipStream_t s);
 void bj_assemble(const Dims& d, const int* f2e, const int* elemcon, const double* H, double* aug,
@@ -209,7 +216,7 @@ void bj_extract(const Dims& d, const double* aug, double* BE, hipStream_t s);
 // act (optional, device): the apply, dot and update kernels below do nothing when act[0] == 0 (a
 // solve that has finished while later steps were already queued)
 template <typename T>
-void bj_apply(const Dims& d, const T* BE, const double* x, double* y, hipStream_t s, const double* act = nullptr);
+void bj_apply(const Dims& d, const T* BE, const TraceIn& in, double* y, hipStream_t s, const double* act = nullptr);
 // elemental additive Schwarz: augmented [block | I] for elements [e0, e0+eb), and the
 // inverse (columns m..2m-1 after lu_solve) into BEe (the block's first element)
 void eas_assemble(const Dims& d, int e0, int eb, const double* H, const int* f2e, const int* elemcon,
@@ -221,7 +228,7 @@ void eas_assemble(const Dims& d, int e0, int eb, const float* H, const int* f2e,
 void eas_extract(const Dims& d, int eb, const double* aug, double* BEe, hipStream_t s);
 void eas_extract(const Dims& d, int eb, const float* aug, float* BEe, hipStream_t s);
 template <typename T>
-void matvec_elem(const Dims& d, const T* H, const int* elemcon, const double* v, double* we, hipStream_t s,
+void matvec_elem(const Dims& d, const T* H, const TraceIn& in, double* we, hipStream_t s,
                  const int* einst = nullptr, const double* emask = nullptr);
 template <typename T>
 void dudg(const Dims& d, const double* RuS, const T* DinvF, const int* elemcon, const double* x,

@@ -76,8 +76,8 @@ void matvec_noalloc(Solver& S, const double* v, double* w, int max_chunk) {
     dc.ne = eb;
     const int* ec = S.elemcon.p + static_cast<long>(d.ndf) * e0;
     const long off = e0 * static_cast<long>(d.m) * d.m;
-    if (S.precision) matvec_elem(dc, S.H32.p + off, ec, v, ws, S.s);
-    else matvec_elem(dc, S.H.p + off, ec, v, ws, S.s);
+    if (S.precision) matvec_elem(dc, S.H32.p + off, {v, ec, nullptr, nullptr}, ws, S.s);
+    else matvec_elem(dc, S.H.p + off, {v, ec, nullptr, nullptr}, ws, S.s);
     k_scatter_add<<<static_cast<unsigned>((static_cast<long>(eb) * d.m + 255) / 256), 256, 0, S.s>>>(
         d, e0, eb, S.elemcon.p, ws, w);
     EXA_HIP(hipGetLastError());

@@ -527,6 +527,7 @@ void Solver::setup_eas() {
   const double per = 16.0 * d.m * d.m;  // bytes of one augmented [block | I]
   eas_chunk = static_cast<int>(std::max(1.0, std::min<double>(d.ne, ws_budget_bytes / per)));
   BEeas.alloc(static_cast<size_t>(d.m) * d.m * d.ne);
+  we2.alloc(static_cast<size_t>(d.m) * d.ne);
   easaug.alloc(static_cast<size_t>(eas_chunk) * 2 * d.m * d.m);
   if (info.n < static_cast<size_t>(eas_chunk)) info.alloc(eas_chunk + 1);
 }
@@ -1069,12 +1070,19 @@ void Solver::residual_fields() {
   face_gather(static_cast<long>(d.npf) * d.nf, d.ncu, src1.p, src2.p, Rh.p, bres.p, s);
 }
 
-void Solver::matvec(const double* v, double* w) {
+// we = the element products H_e v_e
+void Solver::matvec_products(const double* v) {
+  const TraceIn in{v, elemcon.p, nullptr, nullptr};
   hipEvent_t t0{};
   tic(T_MATVEC, &t0);
-  if (precision) matvec_elem(d, H32.p, elemcon.p, v, we.p, s, einst.p, elem_active);
-  else matvec_elem(d, H.p, elemcon.p, v, we.p, s, einst.p, elem_active);
+  if (precision) matvec_elem(d, H32.p, in, we.p, s, einst.p, elem_active);
+  else matvec_elem(d, H.p, in, we.p, s, einst.p, elem_active);
   toc(T_MATVEC, t0);
+}
+
+void Solver::matvec(const double* v, double* w) {
+  matvec_products(v);
+  hipEvent_t t0{};
   tic(T_OTHER, &t0);
   face_gather(static_cast<long>(d.npf) * d.nf, d.ncu, src1.p, src2.p, we.p, w, s);
   toc(T_OTHER, t0);
@@ -1087,17 +1095,37 @@ void Solver::apply_precond(double* xv) {
 
 // out = P in (in and out distinct)
 void Solver::apply_precond_to(const double* in, double* out) {
+  precond_from(TraceIn{in, nullptr, nullptr, nullptr}, we.p, out);
+}
+
+// out = P A v.  Block Jacobi and the Schwarz blocks sum the element products of A v as they read them (the
+// same two values per trace unknown, added in the same order), instead of in a pass of its own that writes
+// A v first; block-ILU(0) reads a node's values once per superelement row and takes the assembled vector.
+void Solver::matvec_precond(const double* v, double* out) {
+  if (precond == 2) {
+    matvec(v, tmp.p);
+    apply_precond_to(tmp.p, out);
+  } else {
+    matvec_products(v);
+    precond_from(TraceIn{we.p, nullptr, src1.p, src2.p}, we2.p, out);
+  }
+}
+
+// The preconditioner on a trace vector or on element products to be summed; prod holds the products of the
+// Schwarz blocks and is not in.v.
+void Solver::precond_from(const TraceIn& in, double* prod, double* out) {
   hipEvent_t t0{};
   tic(T_PRECOND, &t0);
   if (precond == 2) {
-    if (precision && precond_bf16) bilu_apply(d, ilud, BEilu16.p, in, Yilu.p, Xilu.p, out, s, gm_act);
-    else if (precision) bilu_apply(d, ilud, BEilu32.p, in, Yilu.p, Xilu.p, out, s, gm_act);
-    else bilu_apply(d, ilud, BEilu.p, in, Yilu.p, Xilu.p, out, s, gm_act);
+    if (precision && precond_bf16) bilu_apply(d, ilud, BEilu16.p, in.v, Yilu.p, Xilu.p, out, s, gm_act);
+    else if (precision) bilu_apply(d, ilud, BEilu32.p, in.v, Yilu.p, Xilu.p, out, s, gm_act);
+    else bilu_apply(d, ilud, BEilu.p, in.v, Yilu.p, Xilu.p, out, s, gm_act);
   } else if (precond == 1) {  // x = sum_e scatter(BE_e^{-1} gather_e(x)), as hdgMatVec with BE
-    if (precision && precond_bf16) matvec_elem(d, BEeas16.p, elemcon.p, in, we.p, s, einst.p, elem_active);
-    else if (precision) matvec_elem(d, BEeas32.p, elemcon.p, in, we.p, s, einst.p, elem_active);
-    else matvec_elem(d, BEeas.p, elemcon.p, in, we.p, s, einst.p, elem_active);
-    face_gather(static_cast<long>(d.npf) * d.nf, d.ncu, src1.p, src2.p, we.p, out, s);
+    const TraceIn el{in.v, elemcon.p, in.src1, in.src2};
+    if (precision && precond_bf16) matvec_elem(d, BEeas16.p, el, prod, s, einst.p, elem_active);
+    else if (precision) matvec_elem(d, BEeas32.p, el, prod, s, einst.p, elem_active);
+    else matvec_elem(d, BEeas.p, el, prod, s, einst.p, elem_active);
+    face_gather(static_cast<long>(d.npf) * d.nf, d.ncu, src1.p, src2.p, prod, out, s);
   } else {
     if (precision) bj_apply(d, BE32.p, in, out, s, gm_act);
     else bj_apply(d, BE.p, in, out, s, gm_act);

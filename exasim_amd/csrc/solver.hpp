@@ -83,7 +83,7 @@ struct Solver {
   DevBuf<long> src1, src2;
   DevBuf<double> xdg, egeo, fgeo, odg, og, ogf;
   DevBuf<double> udg, uh, udg0, uh0, MCs, MEs, Mass;
-  DevBuf<double> H, DinvF, RuS, Rh, b, BE, bjaug, we, du, RuR, bres;
+  DevBuf<double> H, DinvF, RuS, Rh, b, BE, bjaug, we, we2, du, RuR, bres;
   // per-block workspace
   int neb = 0;
   DevBuf<double> aug, Bfull, Kt, Gc, K0c, H0c, rv, rJ, W, fpt;
@@ -227,8 +227,11 @@ struct Solver {
   void residual(double* nb, double* nru);
   void residual_fields();  // RuR, Rh and the assembled trace residual bres
   void matvec(const double* v, double* w);
+  void matvec_products(const double* v);
+  void matvec_precond(const double* v, double* out);
   void apply_precond(double* x);
   void apply_precond_to(const double* in, double* out);
+  void precond_from(const TraceIn& in, double* prod, double* out);
   int gmres(const double* bvec, double* xvec, double tol_rel = -1.0, int maxit = -1);
   // every instance's GMRES at once; iters[i] = instance i's count; returns the largest
   // maxit < 0: gmres_maxit
