@@ -925,28 +925,39 @@ __global__ __launch_bounds__(64) void k_face_bou_points(Dims d, AsmArgs a) {
   }
 }
 
-// Residual parts of face l: Ru[perm[a,l] + npe*k] -= int phi_a fhI; Rh = -int phi_a fhB
-// (assembleRu, kokkosimpl.h:1650-1659; uequation.cpp:426-427).
+// Residual parts of the faces: Ru[perm[a,l] + npe*k] -= int phi_a fhI; Rh = -int phi_a fhB
+// (assembleRu, kokkosimpl.h:1650-1659; uequation.cpp:426-427).  A workgroup takes epb elements: the
+// integrals of all their face nodes at once, then the faces' parts of Ru in order (an element's faces share
+// edge nodes).  Bound by launches in small meshes: one launch per face took 2.5-6.6 us each there.
 template <typename T>
-__global__ void k_face_res(Dims d, AsmArgs a, int l, int nf1, T* ru, long ldru, double* Rh) {
-  const int npf = d.npf, ngf = d.ngf, ncu = d.ncu;
-  const long per = static_cast<long>(npf) * ncu;
-  const long q = blockIdx.x * static_cast<long>(blockDim.x) + threadIdx.x;
-  if (q >= per * a.eb) return;
-  const long e = q / per;
-  const int r = static_cast<int>(q % per);
-  const int aa = r % npf, k = r / npf;
+__global__ __launch_bounds__(256) void k_face_res(Dims d, AsmArgs a, int epb, int nf1, T* ru, long ldru, double* Rh) {
+  extern __shared__ double fr_sm[];  // epb m
+  const int npf = d.npf, ngf = d.ngf, ncu = d.ncu, m = d.m, per = npf * ncu;
+  const long eb0 = blockIdx.x * static_cast<long>(epb);
+  const int ne = static_cast<int>(min(static_cast<long>(epb), a.eb - eb0));
   const long P = static_cast<long>(a.eb) * d.nfe * ngf;
-  const long pb = (e * d.nfe + l) * ngf;
-  double sI = 0.0, sB = 0.0;
-  for (int g = 0; g < ngf; ++g) {
-    const double w = a.shapfgw[aa + npf * g];
-    sI += w * a.fpt[k * P + pb + g];
-    sB += w * a.fpt[(nf1 + k) * P + pb + g];
+  for (int q = threadIdx.x; q < ne * m; q += 256) {
+    const long e = eb0 + q / m;
+    const int l = (q % m) / per, r = (q % m) % per;
+    const int aa = r % npf, k = r / npf;
+    const long pb = (e * d.nfe + l) * ngf;
+    double sI = 0.0, sB = 0.0;
+    for (int g = 0; g < ngf; ++g) {
+      const double w = a.shapfgw[aa + npf * g];
+      sI += w * a.fpt[k * P + pb + g];
+      sB += w * a.fpt[(nf1 + k) * P + pb + g];
+    }
+    fr_sm[q] = sI;
+    Rh[(a.e0 + e) * m + k + ncu * (aa + npf * l)] = -sB;
   }
-  T& dst = ru[e * ldru + a.perm[aa + npf * l] + d.npe * k];
-  dst = static_cast<T>(static_cast<double>(dst) - sI);
-  Rh[(a.e0 + e) * d.m + k + ncu * (aa + npf * l)] = -sB;
+  for (int l = 0; l < d.nfe; ++l) {
+    __syncthreads();
+    for (int q = threadIdx.x; q < ne * per; q += 256) {
+      const int el = q / per, r = q % per;
+      T& dst = ru[(eb0 + el) * ldru + a.perm[r % npf + npf * l] + d.npe * (r / npf)];
+      dst = static_cast<T>(static_cast<double>(dst) - fr_sm[el * m + l * per + r]);
+    }
+  }
 }
 
 // Jacobian parts of face l: D/B += int phi_a phi_b fhI_uq, F += int phi_a phi_b fhI_uh,
@@ -2163,17 +2174,19 @@ void vol_W(const Dims& d, const AsmArgs& a, hipStream_t s) { vol_W_t(d, a, a.W, 
 void vol_W(const Dims& d, const AsmArgs& a, float* W, hipStream_t s) { vol_W_t(d, a, W, s); }
 
 template <typename T>
-void face_res_t(const Dims& d, const AsmArgs& a, int l, bool jac, T* ru, long ldru, double* Rh, hipStream_t s) {
-  int nf1 = jac ? (d.ncu + d.ncu * d.nc + d.ncu * d.ncu) : d.ncu;
-  long n1 = static_cast<long>(d.npf) * d.ncu * a.eb;
-  k_face_res<T><<<nblocks(n1, 256), 256, 0, s>>>(d, a, l, nf1, ru, ldru, Rh);
+void face_res_t(const Dims& d, const AsmArgs& a, bool jac, T* ru, long ldru, double* Rh, hipStream_t s) {
+  if (a.eb <= 0) return;
+  const int nf1 = jac ? (d.ncu + d.ncu * d.nc + d.ncu * d.ncu) : d.ncu;
+  const int epb = std::max(1, 256 / d.m);  // as many elements as the workgroup has threads for
+  k_face_res<T><<<(a.eb + epb - 1) / epb, 256, static_cast<size_t>(epb) * d.m * sizeof(double), s>>>(
+      d, a, epb, nf1, ru, ldru, Rh);
   EXA_HIP(hipGetLastError());
 }
-void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, double* ru, long ldru, double* Rh, hipStream_t s) {
-  face_res_t(d, a, l, jac, ru, ldru, Rh, s);
+void face_res(const Dims& d, const AsmArgs& a, bool jac, double* ru, long ldru, double* Rh, hipStream_t s) {
+  face_res_t(d, a, jac, ru, ldru, Rh, s);
 }
-void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, float* ru, long ldru, double* Rh, hipStream_t s) {
-  face_res_t(d, a, l, jac, ru, ldru, Rh, s);
+void face_res(const Dims& d, const AsmArgs& a, bool jac, float* ru, long ldru, double* Rh, hipStream_t s) {
+  face_res_t(d, a, jac, ru, ldru, Rh, s);
 }
 
 template <typename T>
@@ -2424,8 +2437,8 @@ void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const float* L
   bilu_put_l_t(d, I, k0, ne_i, Ltmp, BE, s);
 }
 
-// the block-ILU(0) apply for BF16 factors: one wave per superelement (1) or the 256-thread kernel
-// (0); -1 follows EXA_BILU_WAVE (default 1)
+// the block-ILU(0) apply: one wave per superelement where that is faster (1) or always the 256-thread
+// kernel (0); -1 follows EXA_BILU_WAVE (default 1)
 std::atomic<int> g_bilu_wave{-1};
 void set_bilu_wave(int mode) { g_bilu_wave.store(mode); }
 bool bilu_wave_enabled() {

@@ -76,7 +76,7 @@ void lu_solve(double* A, int n, int ncols, long stride, int batch, int* info, hi
 void lu_solve(float* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s,
               int* pivout = nullptr, int* piv_ws = nullptr, void* tri_ws = nullptr);
 // piv_ws (optional, device, >= LU_PIV_WS*batch ints, owned by the caller): with it, panels of up
-// to 256 rows are factored with the panel in registers (k_lu_panel_reg + k_lu_u12)
+// to 256 rows are factored with one wave per matrix (k_lu_panel_wave, k_lu_swap, k_lu_u12)
 // tri_ws (optional, device, >= LU_TRI_WS*batch doubles, owned by the caller): with it, the FP32
 // LU runs the triangular solves of each panel (U12 = L11^{-1} A12, X = U11^{-1} X) as an explicit
 // triangle inverse and an in-place GEMM (the FP64 LU always uses substitution)
@@ -171,9 +171,9 @@ void vol_res(const Dims& d, const AsmArgs& a, float* out, long ldo, hipStream_t 
 // W into a.W, or into an FP32 buffer of the same layout
 void vol_W(const Dims& d, const AsmArgs& a, hipStream_t s);
 void vol_W(const Dims& d, const AsmArgs& a, float* W, hipStream_t s);
-void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, double* ru, long ldru, double* Rh,
+void face_res(const Dims& d, const AsmArgs& a, bool jac, double* ru, long ldru, double* Rh,
               hipStream_t s);
-void face_res(const Dims& d, const AsmArgs& a, int l, bool jac, float* ru, long ldru, double* Rh,
+void face_res(const Dims& d, const AsmArgs& a, bool jac, float* ru, long ldru, double* Rh,
               hipStream_t s);
 // Jacobian parts of every face of the block's elements (face by face, in local order): added to D, F
 // (aug) and B; K, G and H written without their zeros (FaceElim's K0c, G and H0c)

@@ -685,7 +685,7 @@ void Solver::set_option(const std::string& name, double v) {
     set_gemm_autotune(static_cast<int>(v));
   } else if (name == "lu_inverses") {  // FP32 LU: 1 triangle inverses on MFMA, 0 substitution
     lu_inverses = v != 0.0;
-  } else if (name == "ilu_wave") {  // process-wide: FP32/BF16 block-ILU(0) apply, 1 one wave per superelement
+  } else if (name == "ilu_wave") {  // process-wide: block-ILU(0) apply, 1 one wave per superelement where faster
     if (v != 0.0 && v != 1.0 && v != -1.0) throw Error(1, "ilu_wave: 1, 0 or -1 (the environment's choice)");
     set_bilu_wave(static_cast<int>(v));
   } else if (name == "gemm_tile") {  // process-wide: every MFMA product on tile v (0..4), -1 the tuner's
@@ -923,12 +923,10 @@ void Solver::assemble() {
       g.fp32 = precision;
       gemm(g, s);
     }
-    // face terms; residual parts one local face at a time (no two writes of a launch collide)
+    // face terms
     face_points(d, a, true, s);
-    for (int l = 0; l < d.nfe; ++l) {
-      if (f32) face_res(d, a, l, true, aug32.p + n * (n + m), augs, Rh.p, s);
-      else face_res(d, a, l, true, aug.p + n * (n + m), augs, Rh.p, s);
-    }
+    if (f32) face_res(d, a, true, aug32.p + n * (n + m), augs, Rh.p, s);
+    else face_res(d, a, true, aug.p + n * (n + m), augs, Rh.p, s);
     if (f32) face_jac(d, a, aug32.p, Bfull32.p, K0c32.p, Gc32.p, H0c32.p, s);
     else face_jac(d, a, aug.p, Bfull.p, K0c.p, Gc.p, H0c.p, s);
     // eliminate q: D += B*MinvC, F -= B*MinvE, K += G*MinvC, H -= G*MinvE (uequation.cpp:614-681)
@@ -1065,7 +1063,7 @@ void Solver::residual_fields() {
     vol_points(d, a, false, s);
     vol_res(d, a, RuR.p + e0 * n, n, s);
     face_points(d, a, false, s);
-    for (int l = 0; l < d.nfe; ++l) face_res(d, a, l, false, RuR.p + e0 * n, n, Rh.p, s);
+    face_res(d, a, false, RuR.p + e0 * n, n, Rh.p, s);
   }
   face_gather(static_cast<long>(d.npf) * d.nf, d.ncu, src1.p, src2.p, Rh.p, bres.p, s);
 }
