@@ -26,7 +26,7 @@ __device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&&
 // panel and solves L11 U12 = A12; the trailing update A22 -= L21 U12 and the
 // back substitution's updates run on the MFMA GEMM.
 // ---------------------------------------------------------------------------
-constexpr int BLU_MIN_N = 64;  // smaller blocks use the single-kernel k_lu_solve
+constexpr int BLU_MIN_N = 64;  // smaller blocks use the single-kernel k_lu_small
 
 template <typename T, int BLU_NB>
 __global__ __launch_bounds__(256) void k_lu_panel(T* Aall, int n, int ncols, long stride, int k0,
@@ -424,165 +424,81 @@ __global__ __launch_bounds__(256) void k_lu_back(T* Aall, int n, int ncols, long
 }
 
 // ---------------------------------------------------------------------------
-// Blocked LU with partial pivoting + back substitution, one workgroup per matrix.
+// LU with partial pivoting and back substitution of a matrix below 64 rows, one wave per matrix
 // ---------------------------------------------------------------------------
-constexpr int LU_NB = 16;
-constexpr int LU_CH = 64;
-
-__global__ __launch_bounds__(256) void k_lu_solve(double* Aall, int n, int ncols, long stride,
-                                                  int* info) {
+// Lane t holds row t of [A | R] in registers.  A step takes the pivot by a reduction over the lanes and the
+// pivot row by lane reads; rows are not moved, each lane knows the position its row has come to.  The row moves
+// down by one entry per step, so the loop over steps needs no register index, and the entries of U that leave it
+// wait in LDS, each for its own lane: no barrier.  Blocks of CH columns that the step has left behind are
+// skipped.  More right-hand sides than NC - n take several waves, each with its own factorisation.  Bound by
+// the FP64 FMAs and lane reads of a step.  n = 25, 46 columns, the elements of 24 2D meshes: 0.82 ms (a
+// 256-thread workgroup per matrix with eleven barriers per column: 1.68 ms).
+template <int NC>
+__global__ __launch_bounds__(64) void k_lu_small(double* Aall, int n, int ncols, long stride, int* info) {
+  constexpr int CH = 8;
+  extern __shared__ double U[];  // column k of U: U[64 k + lane]
   double* A = Aall + stride * blockIdx.x;
-  extern __shared__ double P[];  // n x LU_NB panel (ld n)
-  __shared__ double Us[LU_NB][LU_CH + 1];
-  __shared__ double redv[256];
-  __shared__ int redi[256];
-  __shared__ int piv[LU_NB];
-  const int tid = threadIdx.x;
+  const int lane = threadIdx.x;
+  const int j0 = n + (NC - n) * static_cast<int>(blockIdx.y);  // the wave's right-hand sides
+  const int R = min(NC - n, ncols - j0), w = n + R;
+  double x[NC];
+#pragma unroll
+  for (int j = 0; j < NC; ++j)
+    x[j] = lane < n && j < w ? A[lane + static_cast<long>(n) * (j < n ? j : j0 + j - n)] : 0.0;
+  int pos = lane < n ? lane : -1;
   int singular = 0;
-  for (int k0 = 0; k0 < n; k0 += LU_NB) {
-    const int nb = min(LU_NB, n - k0);
-    const int rows = n - k0;
-    for (int idx = tid; idx < rows * nb; idx += 256) {
-      int r = k0 + idx % rows, kk = idx / rows;
-      P[r + n * kk] = A[r + static_cast<long>(n) * (k0 + kk)];
+  for (int k = 0; k < n; ++k) {
+    // (a column without a comparable entry, all NaN, keeps its row)
+    double bv = -1.0;
+    int bp = k;
+    const double v = fabs(x[0]);
+    if (pos >= k && v > bv) {
+      bv = v;
+      bp = pos;
     }
-    __syncthreads();
-    for (int kk = 0; kk < nb; ++kk) {
-      const int col = k0 + kk;
-      double best = -1.0;
-      int bi = col;
-      for (int r = col + tid; r < n; r += 256) {
-        double v = fabs(P[r + n * kk]);
-        if (v > best) { best = v; bi = r; }
-      }
-      redv[tid] = best;
-      redi[tid] = bi;
-      __syncthreads();
-      for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) {
-          double o = redv[tid + s];
-          int oi = redi[tid + s];
-          if (o > redv[tid] || (o == redv[tid] && oi < redi[tid])) { redv[tid] = o; redi[tid] = oi; }
-        }
-        __syncthreads();
-      }
-      const int p = redi[0];
-      if (tid == 0) piv[kk] = p;
-      if (p != col && tid < nb) {
-        double t = P[col + n * tid];
-        P[col + n * tid] = P[p + n * tid];
-        P[p + n * tid] = t;
-      }
-      __syncthreads();
-      const double pv = P[col + n * kk];
-      if (pv == 0.0) singular = 1;
-      for (int r = col + 1 + tid; r < n; r += 256) P[r + n * kk] /= pv;
-      __syncthreads();
-      const int rr = n - col - 1, cc = nb - kk - 1;
-      for (int idx = tid; idx < rr * cc; idx += 256) {
-        int r = col + 1 + idx % rr, c = kk + 1 + idx / rr;
-        P[r + n * c] -= P[r + n * kk] * P[col + n * c];
-      }
-      __syncthreads();
-    }
-    for (int idx = tid; idx < rows * nb; idx += 256) {
-      int r = k0 + idx % rows, kk = idx / rows;
-      A[r + static_cast<long>(n) * (k0 + kk)] = P[r + n * kk];
-    }
-    for (int j = tid; j < ncols; j += 256) {
-      if (j >= k0 && j < k0 + nb) continue;
-      double* colj = A + static_cast<long>(n) * j;
-      for (int kk = 0; kk < nb; ++kk) {
-        int p = piv[kk], r = k0 + kk;
-        if (p != r) { double t = colj[r]; colj[r] = colj[p]; colj[p] = t; }
-      }
-    }
-    __syncthreads();
-    for (int j = k0 + nb + tid; j < ncols; j += 256) {
-      double* colj = A + static_cast<long>(n) * j;
-      double x[LU_NB];
+    const int p = argmax_lanes(bv, bp);
+    const int l = __builtin_ctzll(__ballot(pos == p));
+    const double pv = lane_value(x[0], l);
+    if (pv == 0.0) singular = 1;
+    U[64 * k + lane] = x[0];
+    pos = pos == p ? k : pos == k ? p : pos;
+    const double f = pos > k ? x[0] / pv : 0.0;
 #pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk) x[kk] = (kk < nb) ? colj[k0 + kk] : 0.0;
+    for (int c = 0; c < NC; c += CH)
+      if (c + 1 < w - k) {
 #pragma unroll
-      for (int kk = 1; kk < LU_NB; ++kk)
-#pragma unroll
-        for (int t = 0; t < kk; ++t)
-          if (kk < nb) x[kk] -= P[k0 + kk + n * t] * x[t];
-#pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk)
-        if (kk < nb) colj[k0 + kk] = x[kk];
-    }
-    __syncthreads();
-    const int R = n - k0 - nb;
-    if (R > 0) {
-      for (int j0 = k0 + nb; j0 < ncols; j0 += LU_CH) {
-        const int cw = min(LU_CH, ncols - j0);
-        for (int idx = tid; idx < nb * cw; idx += 256) {
-          int t = idx % nb, c = idx / nb;
-          Us[t][c] = A[k0 + t + static_cast<long>(n) * (j0 + c)];
-        }
-        __syncthreads();
-        for (int idx = tid; idx < R * cw; idx += 256) {
-          int r = k0 + nb + idx % R, c = idx / R;
-          double* a = A + r + static_cast<long>(n) * (j0 + c);
-          double s = *a;
-          for (int t = 0; t < nb; ++t) s -= P[r + n * t] * Us[t][c];
-          *a = s;
-        }
-        __syncthreads();
+        for (int j = c; j < c + CH; ++j)
+          if (j + 1 < NC) x[j] = fma(-f, lane_value(x[j + 1], l), x[j + 1]);
       }
-    }
   }
-  // back substitution U X = Y for the right-hand-side columns
-  const int last = ((n - 1) / LU_NB) * LU_NB;
-  for (int k0 = last; k0 >= 0; k0 -= LU_NB) {
-    const int nb = min(LU_NB, n - k0);
-    const int rows = k0 + nb;
-    for (int idx = tid; idx < rows * nb; idx += 256) {
-      int r = idx % rows, kk = idx / rows;
-      P[r + n * kk] = A[r + static_cast<long>(n) * (k0 + kk)];
-    }
-    __syncthreads();
-    for (int j = n + tid; j < ncols; j += 256) {
-      double* colj = A + static_cast<long>(n) * j;
-      double x[LU_NB];
+  for (int k = n - 1; k >= 0; --k) {
+    const int l = __builtin_ctzll(__ballot(pos == k));
+    const double u = U[64 * k + lane];
+    const double ukk = lane_value(u, l), inv = 1.0 / ukk;
+    const double f = pos < k ? u : 0.0;
 #pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk) x[kk] = (kk < nb) ? colj[k0 + kk] : 0.0;
+    for (int c = 0; c < NC; c += CH)
+      if (c < R) {
 #pragma unroll
-      for (int kk = LU_NB - 1; kk >= 0; --kk) {
-        if (kk < nb) {
-          double s = x[kk];
-#pragma unroll
-          for (int t = kk + 1; t < LU_NB; ++t)
-            if (t < nb) s -= P[k0 + kk + n * t] * x[t];
-          x[kk] = s / P[k0 + kk + n * kk];
+        for (int j = c; j < c + CH; ++j) {
+          const double y = lane_value(x[j], l);
+          const double q = y * inv;
+          const double t = fma(fma(-q, ukk, y), inv, q);  // y / ukk, the quotient corrected by its remainder
+          x[j] = pos == k ? t : fma(-f, t, x[j]);
         }
       }
-#pragma unroll
-      for (int kk = 0; kk < LU_NB; ++kk)
-        if (kk < nb) colj[k0 + kk] = x[kk];
-    }
-    __syncthreads();
-    if (k0 > 0) {
-      for (int j0 = n; j0 < ncols; j0 += LU_CH) {
-        const int cw = min(LU_CH, ncols - j0);
-        for (int idx = tid; idx < nb * cw; idx += 256) {
-          int t = idx % nb, c = idx / nb;
-          Us[t][c] = A[k0 + t + static_cast<long>(n) * (j0 + c)];
-        }
-        __syncthreads();
-        for (int idx = tid; idx < k0 * cw; idx += 256) {
-          int r = idx % k0, c = idx / k0;
-          double* a = A + r + static_cast<long>(n) * (j0 + c);
-          double s = *a;
-          for (int t = 0; t < nb; ++t) s -= P[r + n * t] * Us[t][c];
-          *a = s;
-        }
-        __syncthreads();
-      }
-    }
   }
-  if (tid == 0 && info) info[blockIdx.x] = singular;
+  if (lane < n)
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if (j < R) A[pos + static_cast<long>(n) * (j0 + j)] = x[j];
+  if (lane == 0 && blockIdx.y == 0 && info) info[blockIdx.x] = singular;
+}
+
+template <int NC>
+void lu_small(double* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s) {
+  const int chunks = (ncols - n + NC - n - 1) / (NC - n);
+  k_lu_small<NC><<<dim3(batch, chunks), 64, static_cast<size_t>(n) * 64 * sizeof(double), s>>>(A, n, ncols, stride, info);
 }
 
 // RuS = D'^{-1} Ru from the stored FP32 LU factors of D' (replaying the blocked factorisation: each panel's
@@ -850,15 +766,17 @@ void lu_solve(double* A, int n, int ncols, long stride, int batch, int* info, hi
   // the FP64 form keeps the substitution kernels (k_lu_u12, k_lu_back): explicit triangle inverses
   // amplify rounding by the triangle's condition number, which the FP64 form is not allowed to lose
   (void)tri_ws;
-  if ((n >= BLU_MIN_N || pivout) && ncols > n) {
+  if (ncols <= n) throw Error(5, "LU needs right-hand-side columns");
+  if (n >= BLU_MIN_N || pivout) {
     lu_blocked_any(A, n, ncols, stride, batch, info, s, pivout, piv_ws, static_cast<double*>(nullptr));
     return;
   }
-  if (pivout) throw Error(5, "pivot output needs right-hand-side columns");
-  // dynamic LDS panel n x LU_NB doubles next to ~12 KB of static LDS, kept within 64 KB
-  if (n > 400) throw Error(5, "dense block larger than 400 rows");
-  size_t shm = static_cast<size_t>(n) * LU_NB * sizeof(double);
-  k_lu_solve<<<batch, 256, shm, s>>>(A, n, ncols, stride, info);
+  // the narrowest registers that hold a row; beyond 96 columns the right-hand sides are split
+  if (ncols <= 16) lu_small<16>(A, n, ncols, stride, batch, info, s);
+  else if (ncols <= 32) lu_small<32>(A, n, ncols, stride, batch, info, s);
+  else if (ncols <= 48) lu_small<48>(A, n, ncols, stride, batch, info, s);
+  else if (ncols <= 64) lu_small<64>(A, n, ncols, stride, batch, info, s);
+  else lu_small<96>(A, n, ncols, stride, batch, info, s);
   EXA_HIP(hipGetLastError());
 }
 
