@@ -686,7 +686,7 @@ def mfma_roofline(summary, fp32=None):
     r = big[0]
     return {"bound": "mfma", "achieved": r["tflops"], "peak": MFMA_PEAK_FP32 if r["fp32"] else MFMA_PEAK_FP64,
             "unit": "TFLOP/s", "frac": r["mfma_frac"], "traffic": None,
-            "kernel": "k_gemm_mfma<%s> %dx%dx%d, %d products, tile %s" % (
+            "kernel": "k_gemm<%s> %dx%dx%d, %d products, tile %s" % (
                 "float" if r["fp32"] else "double", r["M"], r["N"], r["K"], r["batch"], r["tile"]),
             "flop_per_launch": 2.0 * r["M"] * r["N"] * r["K"] * r["batch"], "avg_launch_ms": r["us_chosen"] / 1e3}
 
