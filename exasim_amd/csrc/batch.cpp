@@ -207,9 +207,9 @@ void Solver::seg_setup() {
 // never overwritten by the next one.
 void Solver::seg_alloc() {
   const long ns = ninst, n1 = restart + 1;
-  const long nb = std::max(segT.map.nblk, segU.map.nblk);
+  const int np = static_cast<int>(n1 + 1);
   EXA_HIP(hipStreamSynchronize(s));
-  segpart.alloc(static_cast<size_t>(std::max(nb, 1L)) * std::max(n1 + 1, SEG_CHUNK / 64));
+  segpart.alloc(static_cast<size_t>(std::max(seg_partials(segT.map, np), seg_partials(segU.map, np))));
   hcol.alloc(static_cast<size_t>(n1 + 1) * ns);
   segy.alloc(static_cast<size_t>(n1) * ns);
   segcoef.alloc(static_cast<size_t>(4 * ns));

@@ -335,7 +335,8 @@ void seg_multidot(const SegMap& m, const double* V, long ldv, int k, const doubl
                   double* out, int sqrt_out, hipStream_t s);
 // Arnoldi step (column i of the cycle): w orthogonalised against V_0..V_i (CGS, gmres.cpp:81-88, or MGS,
 // getpoly.cpp:24-42) and normalised, and every instance's rotations and convergence test; the new
-// Hessenberg column in hcol[k*ns + s]; partial: nblk * max(i + 1, 8) values
+// Hessenberg column in hcol[k*ns + s]; partial: seg_partials(m, i + 2) values
+long seg_partials(const SegMap& m, int k);
 void seg_arnoldi(const SegMap& m, const GmresDev& g, const double* V, long n, int i, int mgs, double* w,
                  double* partial, double* hcol, hipStream_t s);
 // y += scale * coef[s] * x on each segment s

@@ -356,6 +356,7 @@ namespace {
 
 constexpr int SEG_BS = 256;
 constexpr int PIECES = static_cast<int>(SEG_CHUNK / 64);  // 64-entry pieces of a chunk
+constexpr int GROUP = 2048;  // partials of a norm that one block sums
 static_assert(SEG_CHUNK == 2 * SEG_BS, "two entries of a chunk per thread");
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -374,8 +375,8 @@ __device__ __forceinline__ double block_sum(double v, double* sh) {
 }
 
 // sum of count partials by a block of 256 threads; the same order wherever it is done.  Eight loads are in
-// flight per thread: the norm's 19,700 partials of 1.3 million entries are 77 rounds for the one block
-// (13.4 us per reduction on average over a step's two with one load at a time, 6.0 us here).
+// flight per thread: one block on a norm's 19,700 partials of 1.3 million entries took 13.4 us per reduction on
+// average over a step's two with one load at a time, 6.0 us here (and a block per GROUP 4.7 us, with 79,200).
 __device__ __forceinline__ double partials_sum(const double* p, int count, double* sh) {
   double acc = 0.0;
   int i = threadIdx.x;
@@ -391,9 +392,11 @@ __device__ __forceinline__ double partials_sum(const double* p, int count, doubl
 }
 
 // partial[v*nblk + b] = <V_v, w> over block b for the vectors v < k.  Bound by reading V.  The chunk of w is
-// staged in LDS; each wave sums four vectors at a time, so that 16 loads are in flight per lane; the
-// vectors are split over gridDim.y where the chunks alone leave the device idle.  24 instances, 330,000
-// entries together, 25 vectors on average: 16 us (one vector per wave at a time, one block per chunk: 40 us).
+// staged in LDS; each wave sums C vectors at a time (four, or fewer vectors' share of them), with up to 16
+// loads in flight per lane; the vectors are split over gridDim.y where the chunks alone leave the device idle.
+// 24 instances, 330,000 entries together, 25 vectors on average: 16 us (one vector per wave at a time, one block
+// per chunk: 40 us).
+template <int C>
 __global__ __launch_bounds__(SEG_BS) void k_seg_dots(SegMap m, const double* V, long ldv, int k, const double* w,
                                                      double* partial) {
   __shared__ double wl[SEG_CHUNK];
@@ -408,28 +411,32 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_dots(SegMap m, const double* V, 
   const int len = static_cast<int>(m.bend[b] - i0);
   for (int t = threadIdx.x; t < len; t += SEG_BS) wl[t] = w[i0 + t];
   __syncthreads();
-  for (int v0 = 16 * blockIdx.y + 4 * wave; v0 < k; v0 += 16 * gridDim.y) {
-    const double* x[4];
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+  constexpr int U = C <= 2 ? 8 : 4;
+  for (int v0 = 4 * C * blockIdx.y + C * wave; v0 < k; v0 += 4 * C * gridDim.y) {
+    const double* x[C];
+    double acc[C];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) x[q] = V + ldv * min(v0 + q, k - 1) + i0;
+    for (int q = 0; q < C; ++q) {
+      x[q] = V + ldv * min(v0 + q, k - 1) + i0;
+      acc[q] = 0.0;
+    }
     int t = lane;
-    for (; t + 192 < len; t += 256) {
-      double h[4][4];
+    for (; t + 64 * (U - 1) < len; t += 64 * U) {
+      double h[U][C];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) h[u][q] = x[q][t + 64 * u];
+        for (int q = 0; q < C; ++q) h[u][q] = x[q][t + 64 * u];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[q] = fma(h[u][q], wl[t + 64 * u], acc[q]);
+        for (int q = 0; q < C; ++q) acc[q] = fma(h[u][q], wl[t + 64 * u], acc[q]);
     }
     for (; t < len; t += 64)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) acc[q] = fma(x[q][t], wl[t], acc[q]);
+      for (int q = 0; q < C; ++q) acc[q] = fma(x[q][t], wl[t], acc[q]);
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < C; ++q) {
       const double s = wave_sum(acc[q]);
       if (lane == 0 && v0 + q < k) partial[static_cast<long>(v0 + q) * m.nblk + b] = s;
     }
@@ -464,52 +471,66 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_reduce(SegMap m, const double* p
 }
 
 // x += alpha * sum_j V_j * y[j*nseg + seg]; NORM: npart[b*PIECES + piece] = <x, x> over the piece.  Bound by
-// reading V.  One block per 64 entries, its four waves a quarter of the columns each with 8 loads in
-// flight: 45,000 entries, 50 columns on average 6.5 us (a thread per entry walking all columns, with one
-// load in flight and few blocks: 14.2 us).
+// reading V.  Four waves take 8 columns of a 64-entry piece in turn: 45,000 entries, 50 columns on average 6.5 us (a
+// thread per entry walking all columns, with one load in flight and few blocks: 14.2 us).  Two turns or fewer
+// leave waves idle: WHOLE then gives a wave a piece of its own (the same sums).  The turns do not depend on k: for
+// the solution's update a batch's longest solve sets k, and an instance's sum may not depend on it.
+// The coefficients are uniform and, the arguments being restrict, come by scalar loads: through the vector
+// caches, which V streams through, they cost 445 us instead of 368 at 5,068,800 entries and 49 columns.
 // SKIPZ: columns whose coefficient is zero are not read (a basis column the solve has not written in this
 // cycle may hold anything)
-template <bool SKIPZ, bool NORM>
-__global__ __launch_bounds__(SEG_BS) void k_seg_gemv(SegMap m, double* x, const double* V, long ldv, int k,
-                                                     const double* y, double alpha, double* npart) {
-  __shared__ double red[4][64];
-  const int b = blockIdx.x / PIECES, piece = blockIdx.x % PIECES;
+template <bool SKIPZ, bool NORM, bool WHOLE>
+__global__ __launch_bounds__(SEG_BS) void k_seg_gemv(SegMap m, double* __restrict__ x, const double* __restrict__ V,
+                                                     long ldv, int k, const double* __restrict__ y, double alpha,
+                                                     double* __restrict__ npart) {
+  constexpr int PB = WHOLE ? 4 : 1;  // pieces of the block
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.x / (PIECES / PB), piece = blockIdx.x % (PIECES / PB) * PB + (WHOLE ? wave : 0);
   const int sg = m.bseg[b];
   const long i0 = m.bbeg[b] + 64 * piece, end = m.bend[b];
-  if (i0 >= end || (m.act && m.act[sg] == 0.0)) {  // block-uniform
-    if (NORM && threadIdx.x == 0) npart[static_cast<long>(b) * PIECES + piece] = 0.0;
+  if (i0 >= end || (m.act && m.act[sg] == 0.0)) {  // uniform over the waves of a piece
+    if (NORM && lane == 0 && (WHOLE || wave == 0)) npart[static_cast<long>(b) * PIECES + piece] = 0.0;
     return;
   }
   const double* Vi = V + min(i0 + lane, end - 1);
-  // SKIPZ: the waves take 8 columns in turn, which does not depend on k: a batch's longest solve sets k, and
-  // an instance's sum may not depend on it
-  const int kc = (k + 3) / 4;
-  const int j0 = SKIPZ ? 8 * wave : wave * kc, j1 = SKIPZ ? k : min(k, j0 + kc);
-  double acc = 0.0;
-  for (int j = j0; j < j1; j += SKIPZ ? 32 : 8) {
+  const bool in = i0 + lane < end;
+  double xn = in && (WHOLE || wave == 0) ? x[i0 + lane] : 0.0;
+  const double* ys = y + sg;
+  auto turn = [&](int j, double acc) {  // columns j .. j + 7 (past the end: the last one, times 0)
     double v[8], c[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int jj = min(j + u, j1 - 1);
-      c[u] = j + u < j1 ? y[static_cast<long>(jj) * m.nseg + sg] : 0.0;
-      v[u] = 0.0;
-      if (SKIPZ ? c[u] != 0.0 : j + u < j1) v[u] = Vi[ldv * jj];
+      const int jj = min(j + u, k - 1);
+      c[u] = ys[static_cast<long>(jj) * m.nseg];
+      if (j + u >= k) c[u] = 0.0;
+      if (!SKIPZ) v[u] = Vi[ldv * jj];
+      else if (c[u] != 0.0) v[u] = Vi[ldv * jj];
+      else v[u] = 0.0;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) acc = fma(v[u], c[u], acc);
+    return acc;
+  };
+  double r[4] = {0.0, 0.0, 0.0, 0.0};
+  if (WHOLE) {  // k <= 32
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (8 * q < k) r[q] = turn(8 * q, 0.0);
+  } else {
+    __shared__ double red[4][64];
+    double acc = 0.0;
+    for (int j = 8 * wave; j < k; j += 32) acc = turn(j, acc);
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = red[q][lane];
   }
-  red[wave][lane] = acc;
-  __syncthreads();
-  if (wave == 0) {
-    const double s = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
-    const bool in = i0 + lane < end;
-    const double xn = in ? fma(alpha, s, x[i0 + lane]) : 0.0;
-    if (in) x[i0 + lane] = xn;
-    if (NORM) {
-      const double q = wave_sum(xn * xn);
-      if (lane == 0) npart[static_cast<long>(b) * PIECES + piece] = q;
-    }
+  xn = in ? fma(alpha, ((r[0] + r[1]) + r[2]) + r[3], xn) : 0.0;
+  if (in) x[i0 + lane] = xn;
+  if (NORM) {
+    const double q = wave_sum(xn * xn);
+    if (lane == 0) npart[static_cast<long>(b) * PIECES + piece] = q;
   }
 }
 
@@ -549,23 +570,37 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_mgs(SegMap m, double* w, const d
   if (threadIdx.x == 0) pout[b] = acc;
 }
 
-// End of an Arnoldi step: the norm of w from its partials (per per block; pre: already in
-// hcol[(i+1)*nseg + seg]), w /= norm (0 where the norm is 0), and each instance's rotations and
+// gsum[s*gmax + g] = the g-th GROUP of segment s's partials (per per block, contiguous), by block (s, g)
+__global__ __launch_bounds__(SEG_BS) void k_seg_groups(SegMap m, const double* partial, int per, double* gsum, int gmax) {
+  __shared__ double sh[4];
+  const int sg = blockIdx.x, i0 = GROUP * blockIdx.y;
+  const int count = per * (m.sbptr[sg + 1] - m.sbptr[sg]);
+  if (i0 >= count) return;  // block-uniform
+  const double s = partials_sum(partial + static_cast<long>(per) * m.sbptr[sg] + i0, min(GROUP, count - i0), sh);
+  if (threadIdx.x == 0) gsum[static_cast<long>(sg) * gmax + blockIdx.y] = s;
+}
+
+// End of an Arnoldi step: the norm of w from its partials (per per block; gmax: from the sums of their
+// groups, gmax of them per segment), w /= norm (0 where the norm is 0), and each instance's rotations and
 // convergence test.  Blocks [0, nseg): one instance each; the others: a chunk of w each.
 __global__ __launch_bounds__(SEG_BS) void k_seg_finish(SegMap m, GmresDev g, int i, double* w, const double* npart,
-                                                       int per, int pre, double* hcol) {
+                                                       int per, int gmax, double* hcol) {
   __shared__ double sh[4];
   __shared__ ArnoldiLds lds;
   const int blk = static_cast<int>(blockIdx.x) - m.nseg;
   const int sg = blk < 0 ? static_cast<int>(blockIdx.x) : m.bseg[blk];
-  const int first = m.sbptr[sg];
-  double* hn = hcol + static_cast<long>(i + 1) * m.nseg + sg;
-  const double nrm = pre ? *hn
-                         : sqrt(partials_sum(npart + static_cast<long>(per) * first,
-                                             per * (m.sbptr[sg + 1] - first), sh));
+  const int first = m.sbptr[sg], count = per * (m.sbptr[sg + 1] - first);
+  const long t0 = blk < 0 ? 0 : m.bbeg[blk] + threadIdx.x, t1 = blk < 0 ? 0 : m.bend[blk];
+  double wv[2];  // the chunk's values come while the norm is summed
+#pragma unroll
+  for (int q = 0; q < 2; ++q) wv[q] = t0 + SEG_BS * q < t1 ? w[t0 + SEG_BS * q] : 0.0;
+  const double nrm = sqrt(gmax ? partials_sum(npart + static_cast<long>(sg) * gmax, (count + GROUP - 1) / GROUP, sh)
+                               : partials_sum(npart + static_cast<long>(per) * first, count, sh));
   if (blk >= 0) {
     const double c = nrm != 0.0 ? 1.0 / nrm : 0.0;
-    for (long t = m.bbeg[blk] + threadIdx.x; t < m.bend[blk]; t += SEG_BS) w[t] *= c;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (t0 + SEG_BS * q < t1) w[t0 + SEG_BS * q] = wv[q] * c;
     return;
   }
   const int j = g.jcount[0];
@@ -575,7 +610,7 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_finish(SegMap m, GmresDev g, int
       for (int k = threadIdx.x; k <= i; k += SEG_BS) lds.h[k] = hcol[static_cast<long>(k) * m.nseg + sg];
     if (threadIdx.x == 0) {
       lds.h[min(i + 1, GM_LDS_N1)] = nrm;
-      *hn = nrm;
+      hcol[static_cast<long>(i + 1) * m.nseg + sg] = nrm;
     }
   }
   __syncthreads();
@@ -662,21 +697,49 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_scale(SegMap m, double* y, const
   for (long i = m.bbeg[b] + threadIdx.x; i < m.bend[b]; i += SEG_BS) y[i] = c * x[i];
 }
 
-// Partials of a segment up to these counts are summed again by every block that needs the sum (one more
-// read of a few KB from the L2); longer segments' sums get a launch of their own.  The order is the same.
-constexpr int MGS_AGAIN = 1024, NORM_AGAIN = 2048;
+// Partials of a segment up to this count (and one GROUP of a norm's) are summed again by every block that needs
+// the sum (one more read of a few KB from the L2); longer segments' sums get a launch of their own, in which
+// every GROUP of a norm's partials is a block's.  A segment's order is the same in both.
+constexpr int MGS_AGAIN = 1024;
+
+int norm_groups(const SegMap& m) { return (m.maxblk * PIECES + GROUP - 1) / GROUP; }
+
+template <int C>
+void launch_dots(const SegMap& m, const double* V, long ldv, int k, const double* w, double* partial, hipStream_t s) {
+  // about 1024 blocks, one turn of the waves to a block at least
+  const int ny = std::max(1, std::min((k + 4 * C - 1) / (4 * C), 1024 / m.nblk));
+  k_seg_dots<C><<<dim3(m.nblk, ny), SEG_BS, 0, s>>>(m, V, ldv, k, w, partial);
+}
+
+// k_seg_gemv with WHOLE: up to two turns, on chunks enough to fill the device without the idle waves.  An Arnoldi
+// step with 5 and 13 columns, four waves per piece / one: 330,000 entries 23.4 / 23.3 and 30.6 / 30.2 us; 630,000
+// 32.6 / 29.6 and 42.5 / 40.9; 1,260,000 49.2 / 41.6 and 64.5 / 61.1; 40,000 14.8 / 15.5 and 16.5 / 17.6.  With 25
+// columns 1,260,000 95.8 / 96.8.
+constexpr int WHOLE_COLS = 16, WHOLE_CHUNKS = 640;
+
+template <bool SKIPZ, bool NORM>
+void launch_gemv(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double alpha,
+                 double* npart, hipStream_t s) {
+  if (k <= WHOLE_COLS && m.nblk >= WHOLE_CHUNKS)
+    k_seg_gemv<SKIPZ, NORM, true><<<m.nblk * (PIECES / 4), SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha, npart);
+  else
+    k_seg_gemv<SKIPZ, NORM, false><<<m.nblk * PIECES, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha, npart);
+}
 
 }  // namespace
+
+long seg_partials(const SegMap& m, int k) {
+  return static_cast<long>(std::max(m.nblk, 1)) * std::max(k, PIECES) + static_cast<long>(m.nseg) * norm_groups(m);
+}
 
 void seg_multidot(const SegMap& m, const double* V, long ldv, int k, const double* w, double* partial,
                   double* out, int sqrt_out, hipStream_t s) {
   if (m.nblk == 0 || k == 0) return;
-  if (k < 4) {
-    k_seg_dot<<<dim3(m.nblk, k), SEG_BS, 0, s>>>(m, V, ldv, w, partial);
-  } else {  // about 1024 blocks, 16 vectors to a block at least
-    const int ny = std::max(1, std::min((k + 15) / 16, 1024 / m.nblk));
-    k_seg_dots<<<dim3(m.nblk, ny), SEG_BS, 0, s>>>(m, V, ldv, k, w, partial);
-  }
+  if (k < 4) k_seg_dot<<<dim3(m.nblk, k), SEG_BS, 0, s>>>(m, V, ldv, w, partial);
+  else if (k == 4) launch_dots<1>(m, V, ldv, k, w, partial, s);
+  else if (k <= 8) launch_dots<2>(m, V, ldv, k, w, partial, s);
+  else if (k <= 12) launch_dots<3>(m, V, ldv, k, w, partial, s);
+  else launch_dots<4>(m, V, ldv, k, w, partial, s);
   k_seg_reduce<<<dim3(m.nseg, k), SEG_BS, 0, s>>>(m, partial, 1, out, sqrt_out);
   EXA_HIP(hipGetLastError());
 }
@@ -707,11 +770,16 @@ void seg_arnoldi(const SegMap& m, const GmresDev& g, const double* V, long n, in
     seg_multidot(m, V, n, i + 1, w, partial, hcol, 0, s);
     np = partial;
     per = PIECES;
-    k_seg_gemv<false, true><<<m.nblk * PIECES, SEG_BS, 0, s>>>(m, w, V, n, i + 1, hcol, -1.0, np);
+    launch_gemv<false, true>(m, w, V, n, i + 1, hcol, -1.0, np, s);
   }
-  const int pre = m.maxblk * per > NORM_AGAIN;
-  if (pre) k_seg_reduce<<<ns, SEG_BS, 0, s>>>(m, np, per, hcol + static_cast<long>(i + 1) * ns, 1);
-  k_seg_finish<<<ns + m.nblk, SEG_BS, 0, s>>>(m, g, i, w, np, per, pre, hcol);
+  int gmax = 0;
+  if (m.maxblk * per > GROUP) {
+    gmax = (m.maxblk * per + GROUP - 1) / GROUP;
+    double* gsum = partial + static_cast<long>(m.nblk) * std::max(i + 2, PIECES);
+    k_seg_groups<<<dim3(ns, gmax), SEG_BS, 0, s>>>(m, np, per, gsum, gmax);
+    np = gsum;
+  }
+  k_seg_finish<<<ns + m.nblk, SEG_BS, 0, s>>>(m, g, i, w, np, per, gmax, hcol);
   EXA_HIP(hipGetLastError());
 }
 
@@ -730,7 +798,7 @@ void seg_scale(const SegMap& m, double* y, const double* x, const double* coef, 
 void seg_gemv_cols(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double alpha,
                    hipStream_t s) {
   if (m.nblk == 0 || k == 0) return;
-  k_seg_gemv<true, false><<<m.nblk * PIECES, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha, nullptr);
+  launch_gemv<true, false>(m, x, V, ldv, k, y, alpha, nullptr, s);
   EXA_HIP(hipGetLastError());
 }
 

@@ -5,6 +5,7 @@ beyond 256); Hessenberg columns staged in LDS and not (restart above 127); and r
 same algorithm: the counts of equal restarts agree, and the solutions to the solve's tolerance."""
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,79 @@ def test_forms_agree(tmp_path, kw, ortho):
         # grows as (p^2 / h)^2 ~ 1e5 at most over these meshes
         assert norm < 1e-8
         assert np.abs(uh - ref[3]).max() < 1e-6 * np.abs(ref[3]).max()
+
+
+@pytest.mark.parametrize("kw", [dict(n=2, porder=1, pgauss=2), dict(n=32, porder=3, pgauss=6),
+                                dict(n=17, porder=3, pgauss=6, nd=3), dict(n=20, porder=4, pgauss=8, nd=3)])
+@pytest.mark.parametrize("ortho", [0, 1])
+def test_steps(tmp_path, kw, ortho):
+    """The solution after k steps against the minimiser over the same Krylov space, formed with torch and
+    orthogonalised twice: k where the dots' and the update's waves take other shares of the vectors, on one
+    chunk, many, and enough for the norm's partials to be summed in groups."""
+    from exasim_amd import cases
+    from exasim_amd.hdg import HDGSolver
+    cases.poisson2d(str(tmp_path), model="poisson_poly", precond="eas", gmres_tol=1e-14, ortho=ortho, **kw)
+    eps = np.finfo(float).eps
+    with HDGSolver(str(tmp_path), "poisson_poly") as S:
+        S.get_q()
+        S.assemble()
+        N = S.sizes["N"]
+        b = torch.from_numpy(np.random.default_rng(N).standard_normal(N)).cuda()
+
+        def product(v):
+            w = torch.empty_like(v)
+            torch.cuda.synchronize()
+            S.matvec(v.data_ptr(), w.data_ptr())
+            S.precond(w.data_ptr())
+            S.sync()
+            return w
+        steps = [k for k in (1, 3, 4, 5, 8, 9, 12, 13, 16, 17, 33) if k <= N // 2]
+        z = b.clone()
+        torch.cuda.synchronize()
+        S.precond(z.data_ptr())
+        S.sync()
+        V, H, beta = [z / z.norm()], np.zeros((steps[-1] + 1, steps[-1])), float(z.norm())
+        for k in range(steps[-1]):
+            w = product(V[k])
+            for _ in range(2):
+                for i, v in enumerate(V):
+                    h = torch.dot(v, w)
+                    H[i, k] += float(h)
+                    w = w - h * v
+            H[k + 1, k] = float(w.norm())
+            V.append(w / w.norm())
+        for k in steps:
+            h = H[:k + 1, :k]
+            y = np.linalg.lstsq(h, beta * np.eye(k + 1)[0], rcond=None)[0]
+            ref = sum(float(c) * v for c, v in zip(y, V))
+            S.set_option("gmres_maxit", k)
+            x = torch.zeros_like(b)
+            torch.cuda.synchronize()
+            S.gmres(b.data_ptr(), x.data_ptr())
+            S.sync()
+            # orthogonalised once, the basis is orthogonal to about eps cond^2 (CGS) or eps cond (MGS), cond the
+            # projected operator's, and the solution over it moves by as much; N-term sums keep well below N eps
+            c = np.linalg.cond(h)
+            print(kw, "ortho", ortho, "k", k, "cond", c, "err", float((x - ref).norm() / ref.norm()), flush=True)
+            assert float((x - ref).norm()) <= 10 * k * eps * c ** 2 * float(ref.norm())
+
+
+@pytest.mark.parametrize("ortho", [0, 1])
+def test_batch_with_a_long_instance(tmp_path, ortho):
+    """A short instance's sums do not depend on the batch it is in, also where the norm of another one is long
+    enough to be summed in groups (157,920 entries)."""
+    from exasim_amd import cases
+    from exasim_amd.hdg import HDGSolver
+    paths = []
+    for n in (16, 140):
+        paths.append(str(tmp_path / str(n)))
+        cases.poisson2d(paths[-1], n=n, porder=3, pgauss=6, model="poisson_poly", precond="eas", gmres_tol=1e-10,
+                        restart=60, gmres_maxit=300, ortho=ortho)
+    alone = []
+    for p in paths:
+        with HDGSolver.batch([p], "poisson_poly") as S:
+            S.solve()
+            alone.append(S.get("uh"))
+    with HDGSolver.batch(paths, "poisson_poly") as S:
+        S.solve()
+        assert np.array_equal(S.get("uh"), np.concatenate(alone))
