@@ -36,14 +36,16 @@ namespace {
 // product run side by side and share operands through the caches.  Lane l of a 16x16x4 step supplies
 // A[l%16][k] and B[k][l%16] with k = l/16 of the step; since a product's sum may take its K values in
 // any order, step s of a block uses k = 4 (l/16) + s, so that a lane's four B values are contiguous
-// and load as one vector.
+// and load as vectors.
 //
 // Bound by MFMA issue at the clock that the power limit leaves (counters of the 250 x 275 x 375 FP64
 // product: the matrix cores busy 71 % of the cycles at 1.9 GHz), small K by the traffic of C.  Against
 // the form with K tiles staged through LDS between two barriers, each on its best tile:
 //   250 x 275 x 375, batch 2400:   FP64 3.77 -> 2.72 ms (33 -> 46 TFLOP/s), FP32 1.99 -> 1.67 ms (62 -> 74)
 //   300 x 300 x 250, batch 1200:   FP64 1.94 -> 1.38 ms, FP32 1.10 -> 0.82 ms
-//   186 x 487 x 64, batch 1200:    FP64 0.76 -> 0.80 ms, FP32 0.47 -> 0.40 ms (reads and writes C)
+//   186 x 487 x 64, batch 1200:    FP32 0.47 -> 0.40 ms (reads and writes C)
+//   trailing updates of the FP64 LU, K = 32, n = 250, batch 2670 / n = 196, batch 1000 / n = 64, batch 1331
+//                                  10.0 -> 9.5 ms / 1.13 -> 0.97 ms / 65 -> 58 us (reads and writes C)
 //   144 x 36 x 72, batch 8100:     FP64 0.62 -> 0.40 ms, FP32 0.35 -> 0.20 ms
 //   25 x 25 x 25, batch 25000:     FP64 117 -> 70 us
 // ---------------------------------------------------------------------------
@@ -58,19 +60,25 @@ __device__ __forceinline__ dbl4 mfma_step(double a, double b, dbl4 c) {
 __device__ __forceinline__ flt4 mfma_step(float a, float b, flt4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-// The matrix row that row r of the A operand's tile holds: chosen so that register i of lane l is
-// row 4 (l/16) + i of the output tile in both types (four contiguous rows per lane).
-__device__ __forceinline__ int a_row(double, int r) { return 4 * (r & 3) + (r >> 2); }
+// The matrix row that row r of the A operand's tile holds: chosen so that the lane's registers are pieces of
+// 16 bytes of consecutive rows, piece h of lane l at row PSTEP h + PW (l/16) of the output tile: one access
+// of the four lane groups then covers 64 contiguous bytes of a column.  (With all four FP64 rows of a lane
+// contiguous, its two accesses each took every other 16 bytes: the trailing updates of an FP64 LU of 2,670
+// matrices of 250 rows and 301 right-hand sides, bound by C, 10.25 ms; in pieces 9.45.)
+__device__ __forceinline__ int a_row(double, int r) { return 8 * (r >> 3) + 2 * (r & 3) + ((r >> 2) & 1); }
 __device__ __forceinline__ int a_row(float, int r) { return r; }
 
-// four consecutive values at the alignment of one (global loads need no more)
-template <typename T> struct Vec4;
-template <> struct Vec4<double> {
-  typedef double type __attribute__((ext_vector_type(4), aligned(8)));
+// 16 bytes of consecutive values at the alignment of one (global loads need no more)
+template <typename T> struct Piece;
+template <> struct Piece<double> {
+  typedef double type __attribute__((ext_vector_type(2), aligned(8)));
 };
-template <> struct Vec4<float> {
+template <> struct Piece<float> {
   typedef float type __attribute__((ext_vector_type(4), aligned(4)));
 };
+template <typename T> constexpr int PW = 16 / sizeof(T);    // values of a piece
+template <typename T> constexpr int NP = 4 / PW<T>;         // pieces of a lane's four registers
+template <typename T> constexpr int PSTEP = 16 / NP<T>;     // rows from a piece to the lane's next
 
 // operands in the product's type
 template <typename T> __device__ __forceinline__ T* gsel(double* d, float* f);
@@ -92,7 +100,7 @@ template <typename T, int FM, int FN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) * FM * FN > 64 ? 1 : 2)))
 void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
-  typedef typename Vec4<T>::type v4;
+  typedef typename Piece<T>::type piece;
   typedef T acc4 __attribute__((ext_vector_type(4)));
   const unsigned nwg = gridDim.x;  // a multiple of NXCD
   const unsigned L = (blockIdx.x % NXCD) * (nwg / NXCD) + blockIdx.x / NXCD;
@@ -129,7 +137,7 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
   // MFMA tiles of the wave that hold output (the others' loads are harmless, their products skipped)
   const int fm = min(FM, (M - row0 + 15) / 16), fn = min(FN, (N - col0 + 15) / 16);
   T av[2][FM][4];
-  v4 bv[2][FN];
+  T bv[2][FN][4];
   auto load = [&](int buf, int k0) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -137,9 +145,16 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) av[buf][i][s] = *reinterpret_cast<const T*>(at_byte(Ak, oa[i]));
     }
-    const T* Bk = B + k0;
 #pragma unroll
-    for (int j = 0; j < FN; ++j) bv[buf][j] = *reinterpret_cast<const v4*>(at_byte(Bk, ob[j]));
+    for (int h = 0; h < NP<T>; ++h) {
+      const T* Bk = B + k0 + PW<T> * h;
+#pragma unroll
+      for (int j = 0; j < FN; ++j) {
+        const piece x = *reinterpret_cast<const piece*>(at_byte(Bk, ob[j]));
+#pragma unroll
+        for (int q = 0; q < PW<T>; ++q) bv[buf][j][PW<T> * h + q] = x[q];
+      }
+    }
   };
   // the products of the block in buffer buf, interleaved with the loads of the next one into the
   // other (one load after every few products keeps both queues fed)
@@ -151,7 +166,7 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step(av[buf][i][s], bv[buf][j][s], acc[i][j]);
-    constexpr int NLOAD = 4 * FM + FN * (sizeof(T) == 8 ? 2 : 1), PER = 4 * FM * FN / NLOAD;
+    constexpr int NLOAD = 4 * FM + FN * NP<T>, PER = 4 * FM * FN / NLOAD;
 #pragma unroll
     for (int q = 0; q < NLOAD; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);   // one global load
@@ -176,16 +191,18 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
   // its latency would otherwise follow theirs)
   constexpr bool EARLY_C = sizeof(T) * FM * FN <= 32;
   const T alpha = static_cast<T>(g.alpha), beta = static_cast<T>(g.beta);
-  v4 cv[FM][FN];
-  auto load_c = [&](int i, int j) {
-    const int r = row0 + 16 * i + 4 * lk, c = col0 + 16 * j + li;
-    if (c < N && r + 4 <= M) cv[i][j] = *reinterpret_cast<const v4*>(C + r + g.ldc * c);
+  piece cv[FM][FN][NP<T>];
+  auto load_c = [&](int i, int j, int h) {
+    const int r = row0 + 16 * i + PSTEP<T> * h + PW<T> * lk, c = col0 + 16 * j + li;
+    if (c < N && r + PW<T> <= M) cv[i][j][h] = *reinterpret_cast<const piece*>(C + r + g.ldc * c);
   };
   if (EARLY_C && beta != T(0)) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int j = 0; j < FN; ++j) load_c(i, j);
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int h = 0; h < NP<T>; ++h) load_c(i, j, h);
   }
   // A block's loads are always issued (past the end: the last block again, unused), so that the wait
   // before the products counts only older loads.
@@ -237,27 +254,32 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-      const int r = row0 + 16 * i + 4 * lk, c = col0 + 16 * j + li;
-      if (c >= N || r >= M) continue;
-      T* p = C + r + g.ldc * c;
-      if (r + 4 <= M) {
-        v4 x;
-        if (beta != T(0)) {
-          if (!EARLY_C) load_c(i, j);
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
-          for (int q = 0; q < 4; ++q) x[q] = fma(beta, cv[i][j][q], alpha * acc[i][j][q]);
+      for (int h = 0; h < NP<T>; ++h) {
+        const int r = row0 + 16 * i + PSTEP<T> * h + PW<T> * lk, c = col0 + 16 * j + li;
+        if (c >= N || r >= M) continue;
+        T* p = C + r + g.ldc * c;
+        if (r + PW<T> <= M) {
+          piece x;
+          if (beta != T(0)) {
+            if (!EARLY_C) load_c(i, j, h);
+#pragma unroll
+            for (int q = 0; q < PW<T>; ++q) x[q] = fma(beta, cv[i][j][h][q], alpha * acc[i][j][PW<T> * h + q]);
+          } else {
+#pragma unroll
+            for (int q = 0; q < PW<T>; ++q) x[q] = alpha * acc[i][j][PW<T> * h + q];
+          }
+          *reinterpret_cast<piece*>(p) = x;
         } else {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) x[q] = alpha * acc[i][j][q];
+          for (int q = 0; q < PW<T> - 1; ++q)
+            if (r + q < M) {
+              const T v = alpha * acc[i][j][PW<T> * h + q];
+              p[q] = beta != T(0) ? fma(beta, p[q], v) : v;
+            }
         }
-        *reinterpret_cast<v4*>(p) = x;
-      } else {
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-          if (r + q < M) p[q] = beta != T(0) ? fma(beta, p[q], alpha * acc[i][j][q]) : alpha * acc[i][j][q];
       }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -314,7 +336,7 @@ MfmaLaunch mfma_launcher(int fp32, int tile) {
 // ---------------------------------------------------------------------------
 template <typename T, int FM, int FN, bool STAGE>
 __global__ __launch_bounds__(256) void k_face_elim(FaceElim<T> f, int kpad, int tilesM, int tilesK, int tilesH) {
-  typedef typename Vec4<T>::type v4;
+  typedef typename Piece<T>::type piece;
   typedef T acc4 __attribute__((ext_vector_type(4)));
   extern __shared__ double face_sm[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -419,22 +441,25 @@ __global__ __launch_bounds__(256) void k_face_elim(FaceElim<T> f, int kpad, int 
         if (v >= 0) x0 = v + npf * cp;
       }
 #pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const int r = row0 + 16 * i + 4 * lk;
-        T* p = C + m * at + l * M + r;
-        const T* x = X + m * max(x0, 0L) + l * M + r;
-        T v[4];
+      for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          v[t] = isH ? -acc[i][j][t] : acc[i][j][t];
-          if (x0 >= 0 && r + t < M) v[t] += x[t];
+        for (int h = 0; h < NP<T>; ++h) {
+          const int r = row0 + 16 * i + PSTEP<T> * h + PW<T> * lk;
+          T* p = C + m * at + l * M + r;
+          const T* x = X + m * max(x0, 0L) + l * M + r;
+          piece v;
+#pragma unroll
+          for (int t = 0; t < PW<T>; ++t) {
+            const T y = acc[i][j][PW<T> * h + t];
+            v[t] = isH ? -y : y;
+            if (x0 >= 0 && r + t < M) v[t] += x[t];
+          }
+          if (r + PW<T> <= M) *reinterpret_cast<piece*>(p) = v;
+          else
+#pragma unroll
+            for (int t = 0; t < PW<T> - 1; ++t)
+              if (r + t < M) p[t] = v[t];
         }
-        if (r + 4 <= M) *reinterpret_cast<v4*>(p) = v4{v[0], v[1], v[2], v[3]};
-        else
-#pragma unroll
-          for (int t = 0; t < 3; ++t)
-            if (r + t < M) p[t] = v[t];
-      }
     }
   }
 }
