@@ -474,7 +474,13 @@ __global__ __launch_bounds__(64) void k_lu_small(double* Aall, int n, int ncols,
   for (int k = n - 1; k >= 0; --k) {
     const int l = __builtin_ctzll(__ballot(pos == k));
     const double u = U[64 * k + lane];
-    const double ukk = lane_value(u, l), inv = 1.0 / ukk;
+    double ukk = lane_value(u, l);
+    if (fabs(ukk) < 0x1p-1021) {  // its reciprocal may overflow: the row times 2^128, which is exact
+      ukk *= 0x1p128;
+#pragma unroll
+      for (int j = 0; j < NC; ++j) x[j] = pos == k ? x[j] * 0x1p128 : x[j];
+    }
+    const double inv = 1.0 / ukk;
     const double f = pos < k ? u : 0.0;
 #pragma unroll
     for (int c = 0; c < NC; c += CH)

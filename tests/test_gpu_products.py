@@ -185,6 +185,19 @@ def test_lu_backward_error(n, nr, f32, inverses):
     assert np.all(res <= c * eps * scale)
 
 
+def test_lu_tiny_pivots():
+    """Pivots that have no finite reciprocal: the quotients are what the division gives."""
+    n, nr = 5, 4
+    rng = np.random.default_rng(3)
+    T = np.triu(rng.uniform(1.0, 2.0, (n, n)), 0) * 2.0 ** -1030
+    X0 = rng.integers(1, 9, (n, nr)).astype(float)
+    T, R = np.diag(np.diag(T))[None], (np.diag(np.diag(T)) @ X0)[None]
+    _, X, info, _ = factor(T, R, 0)
+    assert info[0] == 0
+    # the products carry the denormals' spacing 2^-1074 relative to 2^-1030
+    assert np.all(np.abs(X[0] - X0) <= 2.0 ** -43 * X0 * 2)
+
+
 @pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 100, 128, 144, 192, 193, 250, 256, 257, 343])
 def test_refinement_solve(n):
     """RuS = U^-1 L^-1 P Ru with the FP32 factors and the panels' pivots, in 64 bits; Rh -= K RuS."""
