@@ -519,7 +519,7 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
   const long e = blockIdx.x;
   const int lane = threadIdx.x;
   const float* Le = LU + e * static_cast<long>(n) * n;
-  double y[RPL], dinv[RPL];
+  double y[RPL], diag[RPL], dinv[RPL];
   int pv[RPL];
   int row[RPL];
 #pragma unroll
@@ -528,7 +528,8 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
     row[q] = min(r, n - 1);
     y[q] = Ru[e * n + row[q]];
     pv[q] = piv[e * n + row[q]];
-    dinv[q] = 1.0 / static_cast<double>(Le[row[q] + static_cast<long>(n) * row[q]]);
+    diag[q] = static_cast<double>(Le[row[q] + static_cast<long>(n) * row[q]]);
+    dinv[q] = 1.0 / diag[q];
   }
   // entry k (uniform) of a vector held like y
   auto pick = [&](const double (&v)[RPL], int k) {
@@ -582,7 +583,9 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
 #pragma unroll
     for (int u = 7; u >= 0; --u)
       if (k + u >= 0) {
-        const double yk = pick(y, k + u) * pick(dinv, k + u);
+        const double yr = pick(y, k + u), dk = pick(diag, k + u), di = pick(dinv, k + u);
+        const double qt = yr * di;
+        const double yk = fma(fma(-qt, dk, yr), di, qt);  // yr / dk, the quotient corrected by its remainder
 #pragma unroll
         for (int q = 0; q < RPL; ++q) {
           const int r = lane + 64 * q;

@@ -230,3 +230,19 @@ def test_refinement_solve(n):
     Kd = K.astype(float)
     ref, a = Rh - (Kd @ x[..., None])[..., 0], np.abs(Rh) + (np.abs(Kd) @ np.abs(x)[..., None])[..., 0]
     assert np.all(np.abs(rh.cpu().numpy() - ref) <= (n + 2) * eps * a)
+
+
+def test_refinement_quotients():
+    """The rows of a diagonal matrix are divided, not multiplied by a rounded reciprocal."""
+    n, ne = 100, 3
+    rng = np.random.default_rng(5)
+    D = rng.uniform(0.5, 2.0, (ne, n)).astype(np.float32)
+    LU, Ru = np.zeros((ne, n, n), dtype=np.float32), rng.standard_normal((ne, n))
+    LU[:, np.arange(n), np.arange(n)] = D
+    pv = np.tile((np.arange(n) % 64).astype(np.int32), (ne, 1))
+    lu, piv, k, ru, rh = dev(LU), dev(pv), dev(np.zeros((ne, n, 4), dtype=np.float32)), dev(Ru), dev(np.zeros((ne, 4)))
+    rus = torch.zeros((ne, n), dtype=torch.float64).cuda()
+    d = Dims(m=4, n=n, ne=ne)
+    call("_ZN3exa10refine_rhsERKNS_4DimsEPKfPKiS4_PKdPdS9_P12ihipStream_t", ctypes.byref(d), ptr(lu), ptr(piv), ptr(k),
+         ptr(ru), ptr(rus), ptr(rh), None)
+    assert np.array_equal(rus.cpu().numpy(), Ru / D.astype(float))
