@@ -75,12 +75,12 @@ void lu_solve(double* A, int n, int ncols, long stride, int batch, int* info, hi
 // The same in FP32 storage and arithmetic (blocked path only: ncols > n)
 void lu_solve(float* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s,
               int* pivout = nullptr, int* piv_ws = nullptr, void* tri_ws = nullptr);
-// piv_ws (optional, device, >= LU_PIV_WS*batch ints, owned by the caller): with it, panels of up
+// piv_ws (optional, device, >= lu_piv_ws(n, FP32)*batch ints, owned by the caller): with it, panels of up
 // to 256 rows are factored with one wave per matrix (k_lu_panel_wave, k_lu_swap, k_lu_u12)
 // tri_ws (optional, device, >= LU_TRI_WS*batch doubles, owned by the caller): with it, the FP32
 // LU runs the triangular solves of each panel (U12 = L11^{-1} A12, X = U11^{-1} X) as an explicit
 // triangle inverse and an in-place GEMM (the FP64 LU always uses substitution)
-constexpr int LU_PIV_WS = 260;  // the moved rows of a panel of 64 columns: their number, (new, old) of each
+int lu_piv_ws(int n, bool fp32);  // 0 where the LU (without pivots returned) reads no piv_ws
 constexpr long LU_TRI_WS = 64L * 64L;
 
 // ---- setup ----

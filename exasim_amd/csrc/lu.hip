@@ -179,13 +179,13 @@ __device__ __forceinline__ float lane_value(float v, int l) {
 // the pivot row reaches every lane through scalar registers, and rows are written to their positions at
 // the end.  A column's chain is the argmax, the broadcast, one reciprocal and the update, without a
 // barrier, and a SIMD runs the chains of its waves side by side.  The operations on every entry are those
-// of k_lu_panel, so the factors are the same.  piv_ws[blockIdx.x]: the number of rows that moved, then
+// of k_lu_panel, so the factors are the same.  piv_ws + blockIdx.x*pws: the number of rows that moved, then
 // (new, old) row of each, for the columns right of the panel.  Per launch, against a workgroup of four waves per
 // matrix with two barriers per column: 2025 FP64 matrices of up to 144 rows, 32 columns 156 -> 53 us; 2667 of up
 // to 250 rows 200 us -> 112 us; 4096 FP32 matrices of 100 rows, 64 columns 484 -> 190 us.
 template <typename T, int NB, int RPL>
 __global__ __launch_bounds__(64) void k_lu_panel_wave(T* Aall, int n, long stride, int k0, int* info, int* pivout,
-                                                      int* piv_ws) {
+                                                      int* piv_ws, int pws) {
   T* A = Aall + stride * blockIdx.x + k0 + static_cast<long>(n) * k0;
   const int nb = min(NB, n - k0);
   const int rows = n - k0;  // <= 64 RPL
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64) void k_lu_panel_wave(T* Aall, int n, long strid
       }
     }
   });
-  int* ws = piv_ws + static_cast<long>(blockIdx.x) * LU_PIV_WS;
+  int* ws = piv_ws + static_cast<long>(blockIdx.x) * pws;
   int moved = 0;
 #pragma unroll
   for (int q = 0; q < RPL; ++q) {
@@ -269,9 +269,10 @@ __global__ __launch_bounds__(64) void k_lu_panel_wave(T* Aall, int n, long strid
 // cache lines, which all lanes then share, where a lane per column touched a line per row and lane (n = 100,
 // 4096 FP32 matrices: 52 us against 249; n = 144, 2025 FP64 matrices 46 us against 111).  All of a column's values are read before any is written.
 template <typename T, int NB>
-__global__ __launch_bounds__(256) void k_lu_swap(T* Aall, int n, int ncols, long stride, int k0, const int* piv_ws) {
+__global__ __launch_bounds__(256) void k_lu_swap(T* Aall, int n, int ncols, long stride, int k0, const int* piv_ws,
+                                                 int pws) {
   constexpr int SL = (2 * NB + 63) / 64;
-  const int* ws = piv_ws + static_cast<long>(blockIdx.x) * LU_PIV_WS;
+  const int* ws = piv_ws + static_cast<long>(blockIdx.x) * pws;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nm = ws[0];
   const int first = k0 + min(NB, n - k0) + blockIdx.y * 64 + 16 * wave;
@@ -658,6 +659,10 @@ int lu_panel_width_f32(int n) {
   return (static_cast<size_t>(n) * 32 * sizeof(float) <= 64000) ? 32 : 16;
 }
 
+// a matrix's ints of piv_ws: the moved rows of a panel, their number and (new, old) of each.  An exchange moves
+// two rows, so a panel of NB columns moves at most 2 NB of the n.
+int piv_ints(int n, int NB) { return 1 + 2 * std::min(2 * NB, n); }
+
 // operands of a GEMM inside the LU: FP64 storage and products, or FP32 storage and products
 inline void lu_gemm_ptrs(Gemm& g, const double* A, const double* B, double* C) {
   g.A = A;
@@ -686,17 +691,18 @@ void blocked_lu(T* A, int n, int ncols, long stride, int batch, int* info, int* 
     g.nb0 = batch; g.nb1 = 1; g.nb2 = 1;
     gemm(g, s);
   };
+  const int pws = piv_ints(n, NB);
   for (int k0 = 0; k0 < n; k0 += NB) {
     const int nb = std::min(NB, n - k0);
     if (piv_ws && n - k0 <= 256) {
       const int rows = n - k0;
-      if (rows <= 64) k_lu_panel_wave<T, NB, 1><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws);
-      else if (rows <= 128) k_lu_panel_wave<T, NB, 2><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws);
-      else if (rows <= 192) k_lu_panel_wave<T, NB, 3><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws);
-      else k_lu_panel_wave<T, NB, 4><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws);
+      if (rows <= 64) k_lu_panel_wave<T, NB, 1><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws, pws);
+      else if (rows <= 128) k_lu_panel_wave<T, NB, 2><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws, pws);
+      else if (rows <= 192) k_lu_panel_wave<T, NB, 3><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws, pws);
+      else k_lu_panel_wave<T, NB, 4><<<batch, 64, 0, s>>>(A, n, stride, k0, info, pivout, piv_ws, pws);
       const int right = ncols - k0 - nb;
       if (right > 0) {
-        k_lu_swap<T, NB><<<dim3(batch, (right + 63) / 64), 256, 0, s>>>(A, n, ncols, stride, k0, piv_ws);
+        k_lu_swap<T, NB><<<dim3(batch, (right + 63) / 64), 256, 0, s>>>(A, n, ncols, stride, k0, piv_ws, pws);
         if (tri_ws) {
           k_lu_tri_inv<T, NB, true><<<batch, 64, 0, s>>>(A, n, stride, k0, tri_ws);
           apply_tri(nb, k0, k0 + nb, right);
@@ -768,6 +774,11 @@ void lu_blocked_any(T* A, int n, int ncols, long stride, int batch, int* info, h
 }
 
 }  // namespace
+
+int lu_piv_ws(int n, bool fp32) {
+  if (!fp32 && n < BLU_MIN_N) return 0;  // k_lu_small
+  return piv_ints(n, fp32 ? lu_panel_width_f32(n) : lu_panel_width(n));
+}
 
 void lu_solve(double* A, int n, int ncols, long stride, int batch, int* info, hipStream_t s, int* pivout,
               int* piv_ws, void* tri_ws) {

@@ -106,8 +106,9 @@ void* Solver::lu_tri(long batch) {
   return lutri.p;
 }
 
-int* Solver::lu_ws(long batch) {
-  const size_t need = static_cast<size_t>(std::max(1L, batch)) * LU_PIV_WS;
+int* Solver::lu_ws(long batch, long rows, bool fp32) {
+  const size_t need = static_cast<size_t>(std::max(1L, batch)) * lu_piv_ws(static_cast<int>(rows), fp32);
+  if (need == 0) return nullptr;
   if (lupiv.n < need) {
     EXA_HIP(hipStreamSynchronize(s));
     lupiv.alloc(need);
@@ -384,7 +385,7 @@ void Solver::setup_q(long e_begin, long ne) {
     EXA_HIP(hipMemsetAsync(qaug.p, 0, static_cast<size_t>(eb) * per * sizeof(double), s));
     qsetup(d, static_cast<int>(e0), eb, shapegt.p, shapegw.p, shapfgt.p, shapfgw.p, perm.p, egeo.p, fgeo.p,
            qaug.p, Mass.p, s, qA.p);
-    lu_solve(qaug.p, d.npe, static_cast<int>(ncq), per, eb, info.p, s, nullptr, lu_ws(eb), lu_tri(eb));
+    lu_solve(qaug.p, d.npe, static_cast<int>(ncq), per, eb, info.p, s, nullptr, lu_ws(eb, d.npe, false));
     const int bad = first_nonzero(info.p, eb);
     if (bad >= 0) throw Error(4, "singular mass matrix at element " + std::to_string(e0 + bad));
     qpack(d, static_cast<int>(e0), eb, qaug.p, MCs.p, MEs.p, s);
@@ -529,6 +530,8 @@ void Solver::setup_eas() {
   BEeas.alloc(static_cast<size_t>(d.m) * d.m * d.ne);
   we2.alloc(static_cast<size_t>(d.m) * d.ne);
   easaug.alloc(static_cast<size_t>(eas_chunk) * 2 * d.m * d.m);
+  lu_ws(eas_chunk, d.m, precision != 0);
+  if (precision) lu_tri(eas_chunk);
   if (info.n < static_cast<size_t>(eas_chunk)) info.alloc(eas_chunk + 1);
 }
 
@@ -647,6 +650,8 @@ void Solver::alloc_workspace() {
   if (model == MODEL_PLUGIN) pbuf.alloc(static_cast<size_t>(plugin_buffer_doubles(d, plugin_fns.nbc, neb)));
   V.alloc(static_cast<size_t>(restart + 1) * d.N);
   partial.alloc(DOT_PARTIALS);
+  lu_ws(neb, n, precision != 0);  // the condensation's, before the first solve
+  if (precision) lu_tri(neb);
   seg_alloc();
 }
 
@@ -959,10 +964,10 @@ void Solver::assemble() {
     tic(T_LU, &t0);
     if (f32)
       lu_solve(aug32.p, static_cast<int>(n), static_cast<int>(augcols()), augs, eb, info.p, s,
-               piv32.p + static_cast<long>(e0) * n, lu_ws(eb), lu_tri(eb));
+               piv32.p + static_cast<long>(e0) * n, lu_ws(eb, n, true), lu_tri(eb));
     else
-      lu_solve(aug.p, static_cast<int>(n), static_cast<int>(augcols()), augs, eb, info.p, s, nullptr, lu_ws(eb),
-               lu_tri(eb));
+      lu_solve(aug.p, static_cast<int>(n), static_cast<int>(augcols()), augs, eb, info.p, s, nullptr,
+               lu_ws(eb, n, false));
     toc(T_LU, t0);
     tic(T_ASSEMBLY, &t0);
     {  // H += K * DinvF (= -K X_F), Rh -= K * (D^{-1} Ru)
@@ -1002,10 +1007,10 @@ void Solver::assemble() {
       const int eb = std::min(eas_chunk, d.ne - e0);
       if (precision) {
         eas_assemble(d, e0, eb, H32.p, f2e.p, elemcon.p, easaug32.p, s);
-        lu_solve(easaug32.p, d.m, 2 * d.m, 2 * mm, eb, info.p, s, nullptr, lu_ws(eb), lu_tri(eb));
+        lu_solve(easaug32.p, d.m, 2 * d.m, 2 * mm, eb, info.p, s, nullptr, lu_ws(eb, d.m, true), lu_tri(eb));
       } else {
         eas_assemble(d, e0, eb, H.p, f2e.p, elemcon.p, easaug.p, s);
-        lu_solve(easaug.p, d.m, 2 * d.m, 2 * mm, eb, info.p, s, nullptr, lu_ws(eb), lu_tri(eb));
+        lu_solve(easaug.p, d.m, 2 * d.m, 2 * mm, eb, info.p, s, nullptr, lu_ws(eb, d.m, false));
       }
       const int bad = first_nonzero(info.p, eb);
       if (bad >= 0) throw Error(4, "singular Schwarz block at element " + std::to_string(e0 + bad));
@@ -1017,7 +1022,7 @@ void Solver::assemble() {
     // hdgBlockJacobi (matvec.cpp:190-217)
     if (precision) bj_assemble(d, f2e.p, elemcon.p, H32.p, bjaug.p, s);
     else bj_assemble(d, f2e.p, elemcon.p, H.p, bjaug.p, s);
-    lu_solve(bjaug.p, d.ncf, 2 * d.ncf, 2L * d.ncf * d.ncf, d.nf, info.p, s, nullptr, lu_ws(d.nf));
+    lu_solve(bjaug.p, d.ncf, 2 * d.ncf, 2L * d.ncf * d.ncf, d.nf, info.p, s, nullptr, lu_ws(d.nf, d.ncf, false));
     bj_extract(d, bjaug.p, BE.p, s);
   } else {
     // hdgBlockILU0 (matvec.cpp:119-166)

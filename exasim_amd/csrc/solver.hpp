@@ -100,7 +100,7 @@ struct Solver {
   int precond_bf16 = 0;
   DevBuf<unsigned short> BEilu16, BEeas16;
   DevBuf<int> piv32;  // row exchanges of the blocked LU of D' ([n, ne], panel-relative)
-  DevBuf<int> lupiv;     // this handle's pivots of the current LU panel (LU_PIV_WS per matrix of a batched LU)
+  DevBuf<int> lupiv;     // this handle's pivots of the current LU panel (lu_piv_ws per matrix of a batched LU)
   DevBuf<double> lutri;  // this handle's triangle inverses of the current LU panel (LU_TRI_WS per matrix)
   // elemental additive Schwarz: inverted element blocks, inversion scratch
   DevBuf<double> BEeas, easaug;
@@ -192,7 +192,7 @@ struct Solver {
   Solver(const std::vector<std::string>& datains, const std::string& model, int device);
   ~Solver();
   void set_dims();
-  int* lu_ws(long batch);
+  int* lu_ws(long batch, long rows, bool fp32);
   // FP32 LU of D' and of the Schwarz blocks: explicit triangle inverses applied by GEMMs (true) or
   // substitution (false, option lu_inverses = 0)
   bool lu_inverses = true;

@@ -4,6 +4,7 @@ with a narrow last one, and blocks whose pivots are off the diagonal.  Assembled
 oracle through D^{-1} F, and the inverted face blocks against their inverses."""
 import numpy as np
 import pytest
+import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,25 @@ def test_solves(tmp_path, builder, kw, n, m, ncf):
         for f in range(len(K)):
             c = np.linalg.cond(K[f])
             assert np.abs(B[f] @ K[f] - np.eye(ncf)).max() < 10 * ncf * c * eps
+
+
+def test_no_workspace(tmp_path):
+    """Matrices below 64 FP64 rows take no workspace: a handle of many small elements holds its fields, geometry,
+    element blocks and Krylov basis (13.7 KB per element here), and the inversion of the face blocks allocates
+    nothing.  (A pivot workspace per matrix was 1 KB, one for triangle inverses 32 KB.)"""
+    from exasim_amd import cases
+    from exasim_amd.hdg import HDGSolver
+    info = cases.poisson2d(str(tmp_path), n=200, porder=1, pgauss=2, precond="bjacobi")
+    torch.cuda.synchronize()
+    free = [torch.cuda.mem_get_info()[0]]
+    with HDGSolver(str(tmp_path), info["model"]) as S:
+        S.sync()
+        free.append(torch.cuda.mem_get_info()[0])
+        S.get_q()
+        S.assemble()
+        S.sync()
+        free.append(torch.cuda.mem_get_info()[0])
+        z = S.sizes
+    print("created", free[0] - free[1], "assembled", free[1] - free[2], z, flush=True)
+    assert free[0] - free[1] < 18e3 * z["ne"]
+    assert free[1] - free[2] < 128 * z["nf"]
