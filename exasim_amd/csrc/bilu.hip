@@ -21,7 +21,7 @@ constexpr int blocks_ahead() {
 // One wave per superelement: lane (rr, part) accumulates rows VW rr .. VW rr + VW - 1 over columns
 // CW part .. CW part + CW - 1 of every block.  The sweeps are one flat program of (block, vector offset)
 // pairs in 3 nfse segments: forward rows 0 .. nfse-1, then for i = nfse-1 .. 0 the U row and the diagonal
-// block, whose vector z lies after v.  A block of 16 to 36 rows is only a few loads per lane, so the sweep
+// block, whose vector z lies after v.  A block of up to 32 rows is only a few loads per lane, so the sweep
 // is a chain of load latencies unless several blocks are in flight: D of them are loaded ahead (no load
 // waits for a row's result), and the program lies in LDS, read an entry ahead.  A segment's parts are added
 // through LDS in a fixed order.
@@ -146,14 +146,15 @@ __global__ __launch_bounds__(64) void k_bilu_apply_small(Dims d, IluDev I, const
   }
 }
 
+size_t small_lds(int ncf, int bytes, int nfse, int nprog, int VW) {
+  return (64 * VW + nprog + PAD + (3 * nfse + 2) / 2) * sizeof(double) +
+         static_cast<size_t>(nfse + 1) * ncf * (bytes == 8 ? sizeof(double) : sizeof(float));
+}
+
 template <typename T, int VW>
-bool apply_small_vw(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Xo, const double* act,
+void apply_small_vw(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Xo, const double* act, int cw,
                     hipStream_t s) {
-  if (d.ncf / VW > 64) return false;
-  const int nparts = 64 / (d.ncf / VW), cw = (d.ncf + nparts - 1) / nparts;
-  using VT = typename std::conditional<sizeof(T) == 8, double, float>::type;
-  const size_t shm = (64 * VW + I.nprog + PAD + (3 * I.nfse + 2) / 2) * sizeof(double) + static_cast<size_t>(I.nfse + 1) * d.ncf * sizeof(VT);
-  if (cw > 8 || shm > 64 * 1024) return false;
+  const size_t shm = small_lds(d.ncf, sizeof(T), I.nfse, I.nprog, VW);
   const auto go = [&](auto kern) { kern<<<I.nse, 64, shm, s>>>(d, I, BE, x, Xo, act); };
   if (cw == 1) go(&k_bilu_apply_small<T, VW, 1>);
   else if (cw == 2) go(&k_bilu_apply_small<T, VW, 2>);
@@ -161,16 +162,36 @@ bool apply_small_vw(const Dims& d, const IluDev& I, const T* BE, const double* x
   else if (cw == 4) go(&k_bilu_apply_small<T, VW, 4>);
   else if (cw <= 6) go(&k_bilu_apply_small<T, VW, 6>);
   else go(&k_bilu_apply_small<T, VW, 8>);
-  return true;
 }
 
 }  // namespace
 
+// Time per apply with 256 threads / one wave (us), FP64, FP32 and BF16 factors, the scatter with it:
+//   1 to 6 columns a lane: ncf 2 to 8, 1.6 to 2.5 times as fast; 9, 12, 16, 18: 1.2 to 2.4; 20, 24: 1.02 to 2.0
+//   (2D and 3D superelements of 2 to 4 elements a side, 27 to 4,096 of them);
+//   7 columns, ncf 28, 2D: 61/58 58/54 59/53 (512 of 2 x 2), 149/149 132/86 96/64 (2,048), 182/186 170/173 172/162 (128
+//   of 4 x 4);
+//   8 columns, ncf 32: 180/202 171/187 169/170 (27 of 2 x 2 x 2), 246/242 171/188 170/177 (216), 279/257 210/213 193/188
+//   (512), 390/408 259/246 234/220 (1,000), 1730/1731 1293/1489 1208/1303 (64 of 4 x 4 x 4); 2D 48/50 52/50 52/49 (32 of
+//   2 x 2), 61/59 56/53 56/52 (512), 186/194 140/108 96/74 (2,048), 165/183 164/172 163/162 (128 of 4 x 4), 251/231
+//   201/195 180/169 (512).
+// So: up to 7 columns always; 8, where few blocks fit the registers ahead, in FP32 and BF16 from 512 superelements.
+int bilu_small_columns(int ncf, int bytes, int nse, int nfse, int nprog) {
+  const int VW = ncf % 2 == 0 ? 2 : 1;
+  if (ncf / VW > 64) return 0;
+  const int nparts = 64 / (ncf / VW), cw = (ncf + nparts - 1) / nparts;
+  if (cw > 8 || (cw == 8 && (bytes == 8 || nse < 512))) return 0;
+  return small_lds(ncf, bytes, nfse, nprog, VW) <= 64 * 1024 ? cw : 0;
+}
+
 template <typename T>
 bool bilu_apply_small(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Xo, const double* act,
                       hipStream_t s) {
-  if (!I.wseg) return false;
-  return d.ncf % 2 == 0 ? apply_small_vw<T, 2>(d, I, BE, x, Xo, act, s) : apply_small_vw<T, 1>(d, I, BE, x, Xo, act, s);
+  const int cw = I.wseg ? bilu_small_columns(d.ncf, sizeof(T), I.nse, I.nfse, I.nprog) : 0;
+  if (cw == 0) return false;
+  if (d.ncf % 2 == 0) apply_small_vw<T, 2>(d, I, BE, x, Xo, act, cw, s);
+  else apply_small_vw<T, 1>(d, I, BE, x, Xo, act, cw, s);
+  return true;
 }
 template bool bilu_apply_small<double>(const Dims&, const IluDev&, const double*, const double*, double*,
                                        const double*, hipStream_t);

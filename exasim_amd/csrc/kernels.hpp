@@ -266,7 +266,10 @@ void bilu_put_l(const Dims& d, const IluDev& I, int k0, int ne_i, const float* L
 // Rh_e -= K_e u_e of the eb elements of a block: K [m, n, eb], u_e = U + su e (n values), Rh [m, eb]
 template <typename T, typename TU>
 void trace_rhs(const Dims& d, int eb, const T* K, const TU* U, long su, double* Rh, hipStream_t s);
-// Xo of small face blocks with one wave per superelement (bilu.hip); false: the shape needs another kernel
+// columns of a block that a lane takes in the one-wave apply (bilu.hip) of factors of bytes each, or 0: the
+// shape needs another kernel
+int bilu_small_columns(int ncf, int bytes, int nse, int nfse, int nprog);
+// Xo of small face blocks with one wave per superelement; false: the shape needs another kernel
 template <typename T>
 bool bilu_apply_small(const Dims& d, const IluDev& I, const T* BE, const double* x, double* Xo, const double* act,
                       hipStream_t s);

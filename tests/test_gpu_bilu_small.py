@@ -1,7 +1,10 @@
 """The block-ILU(0) apply with one wave per superelement for small face blocks (bilu.hip) against the
 256-thread kernel on the same factors: block rows of 2 to 32 (one to eight columns per lane, idle lanes,
 blocks of fewer columns than the lanes cover), odd sizes (one row per lane), programs shorter than the
-blocks loaded ahead and longer than 64 entries, FP64, FP32 and BF16 factors."""
+blocks loaded ahead and longer than 64 entries, FP64, FP32 and BF16 factors.  The shape rule's answer is checked
+with each: a shape it left to the 256-thread kernel would compare that with itself."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -18,7 +21,26 @@ CASES = [  # builder, arguments, ncf
     ("poisson2d", dict(n=2, porder=2, pgauss=4, nd=3, cartgridpart=[3, 2, 2, 2, 2, 2, 2, 0]), 9),
     ("convdiff3d", dict(n=2, porder=2, cartgridpart=[3, 2, 2, 2, 2, 2, 2, 0]), 18),
     ("convdiff3d", dict(n=4, porder=3, cartgridpart=[3, 4, 4, 4, 2, 2, 2, 0]), 32),
+    ("navierstokes2d", dict(nx=8, ny=8, porder=6, nsteps=1), 28),
+    ("navierstokes2d", dict(nx=64, ny=32, porder=7, nsteps=1), 32),
+    ("poisson2d", dict(n=4, porder=4, pgauss=8, nd=3, cartgridpart=[3, 4, 4, 4, 2, 2, 2, 0]), 25),
 ]
+
+
+def columns_per_lane(z, ncf, size):
+    from exasim_amd import hdg
+    f = hdg.load()._ZN3exa18bilu_small_columnsEiiiii
+    f.restype = ctypes.c_int
+    # a block of the factors occurs once in the sweeps' program
+    return f(ncf, size, z["ilu_nse"], z["ilu_nfse"], z["ilu_nnz"])
+
+
+def expected(ncf, size, nse):
+    """Two rows per lane in even sizes, one in odd ones; at most 7 columns per lane, and 8 in the smaller types on
+    512 superelements or more."""
+    parts = 64 // (ncf // 2 if ncf % 2 == 0 else ncf)
+    c = -(-ncf // parts)
+    return c if c < 8 or (c == 8 and size < 8 and nse >= 512) else 0
 
 
 @pytest.mark.parametrize("builder,kw,ncf", CASES)
@@ -35,6 +57,9 @@ def test_apply(tmp_path, builder, kw, ncf):
             S.set_option("precond_bf16", bf16)
             z = S.sizes
             assert z["npf"] * z["ncu"] == ncf
+            z, size = S.state(), (2 if bf16 else 4) if precision else 8
+            assert columns_per_lane(z, ncf, size) == expected(ncf, size, z["ilu_nse"])
+            z["N"] = S.sizes["N"]
             S.get_q()
             S.assemble()
             x = np.random.default_rng(ncf).standard_normal(z["N"])
