@@ -491,7 +491,7 @@ void face_elim_fm(const FaceElim<T>& f, hipStream_t s) {
 // ---------------------------------------------------------------------------
 // The autotuner
 // ---------------------------------------------------------------------------
-typedef std::tuple<int, int, int, int, int, int, int> TuneKey;  // device, M, N, K, log2 batch, fp32, storage
+typedef std::tuple<int, int, int, int, int, int> TuneKey;  // device, M, N, K, log2 batch, fp32
 struct TuneEntry {
   int tile = 0;
   long batch = 0;  // products in the timed call
@@ -557,7 +557,7 @@ long c_extent(const Gemm& g) {
 // run, the fastest run kept, so that work of other streams inflates no tile's time), or the
 // default when the shape cannot be timed.  A product that cannot be rerun on its own C is timed
 // writing into a scratch copy of C's extent (its values are not used).
-int pick_tile(const Gemm& g, int store, long batch, hipStream_t s) {
+int pick_tile(const Gemm& g, long batch, hipStream_t s) {
   if (forced_tile() >= 0) return tile_ok(g, forced_tile()) ? forced_tile() : 0;
   const int mode = tune_override() >= 0 ? tune_override() : tune_mode();
   if (mode == 0) return 0;
@@ -565,7 +565,7 @@ int pick_tile(const Gemm& g, int store, long batch, hipStream_t s) {
   if (work < 64) return tile_ok(g, 1) ? 1 : 0;  // a launch of a few workgroups: the smallest tile spreads widest
   int dev = 0;
   EXA_HIP(hipGetDevice(&dev));
-  const TuneKey key{dev, g.M, g.N, g.K, log2_bucket(batch), g.fp32, store};
+  const TuneKey key{dev, g.M, g.N, g.K, log2_bucket(batch), g.fp32};
   {
     std::lock_guard<std::mutex> lk(tune_mu);
     auto it = tune_table().find(key);
@@ -638,11 +638,14 @@ void gemm(const Gemm& g, hipStream_t s) {
   if (batch <= 0) return;
   const int store = (g.Af ? 1 : 0) | (g.Bf ? 2 : 0) | (g.Cf ? 4 : 0);
   if (store != (g.fp32 ? 7 : 0)) throw Error(5, "GEMM operands must be stored in the product's type");
+  // the scaling and the sum with C are exact up to the one rounding of the result for these
+  if (g.fp32 && ((g.alpha != 1.0 && g.alpha != -1.0) || (g.beta != 0.0 && g.beta != 1.0)))
+    throw Error(5, "FP32 GEMM coefficients must be alpha = 1 or -1, beta = 0 or 1");
   // the kernel's offsets within one A or B are 32-bit
   if (g.lda * static_cast<long>(g.K) + g.M > 0x1fffffffL || g.ldb * static_cast<long>(g.N) + g.K > 0x1fffffffL)
     throw Error(5, "GEMM operand too large");
   // products of at most one 32 x 32 tile run on it; the tuner picks the others' tile
-  const int tile = g.M <= 32 && g.N <= 32 && forced_tile() < 0 ? 1 : pick_tile(g, store, batch, s);
+  const int tile = g.M <= 32 && g.N <= 32 && forced_tile() < 0 ? 1 : pick_tile(g, batch, s);
   // (a product timed on its own C has left its result there; one more run writes the same values)
   mfma_launcher(g.fp32, tile)(g, s);
   EXA_HIP(hipGetLastError());
@@ -675,8 +678,9 @@ std::string gemm_tuning_report() {
   for (const auto& kv : tune_table()) {
     const TuneKey& k = kv.first;
     const TuneEntry& e = kv.second;
+    const int fp32 = std::get<5>(k);  // the storage field: bits of the operands in FP32, all or none
     std::snprintf(line, sizeof line, "%d %d %d %d %d %d %dx%d %ld", std::get<1>(k), std::get<2>(k), std::get<3>(k),
-                  std::get<4>(k), std::get<5>(k), std::get<6>(k), TILES[e.tile].bm, TILES[e.tile].bn, e.batch);
+                  std::get<4>(k), fp32, fp32 ? 7 : 0, TILES[e.tile].bm, TILES[e.tile].bn, e.batch);
     out += line;
     for (int t = 0; t < NTILE; ++t) {
       std::snprintf(line, sizeof line, " %.3f", e.us[t]);

@@ -30,15 +30,10 @@ inline unsigned nblocks(long n, int bs) { return static_cast<unsigned>((n + bs -
 
 // MFMA operand vectors (the batched GEMMs themselves are in gemm.hip)
 typedef double dbl4 __attribute__((ext_vector_type(4)));
-typedef float flt4 __attribute__((ext_vector_type(4)));
 
-// One 16x16x4 step.  FP64: register i of lane l holds D[l/16 + 4i][l%16];
-// FP32 (inputs rounded to FP32, FP32 accumulation): D[4(l/16) + i][l%16].
+// One 16x16x4 step: register i of lane l holds D[l/16 + 4i][l%16].
 __device__ inline dbl4 mfma_step(double a, double b, dbl4 c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ inline flt4 mfma_step(float a, float b, flt4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1748,8 +1743,7 @@ __global__ void k_to_float_2d(float* dst, const S* src, long per, long sstride, 
 constexpr int DOT_BS = 256;
 
 __global__ __launch_bounds__(DOT_BS) void k_dot_partial(const double* x, const double* y, long n,
-                                                        double* partial, const double* act) {
-  if (act && act[0] == 0.0) return;  // a finished solve: nothing to do (grid-uniform)
+                                                        double* partial) {
   __shared__ double sh[DOT_BS];
   double s = 0.0;
   for (long i = blockIdx.x * static_cast<long>(DOT_BS) + threadIdx.x; i < n;
@@ -1766,8 +1760,7 @@ __global__ __launch_bounds__(DOT_BS) void k_dot_partial(const double* x, const d
 
 // partial is [nvec][nb]; out[v] = sum_b partial[v][b] (sqrt when sqrt_out)
 __global__ __launch_bounds__(DOT_BS) void k_reduce(const double* partial, int nb, double* out,
-                                                   int sqrt_out, const double* act) {
-  if (act && act[0] == 0.0) return;
+                                                   int sqrt_out) {
   __shared__ double sh[DOT_BS];
   const double* pv = partial + static_cast<long>(blockIdx.x) * nb;
   double s = 0.0;
@@ -2494,11 +2487,10 @@ static int dot_partials_count(long n) {
   return static_cast<int>(std::max(1L, std::min<long>(DOT_PARTIALS, b)));
 }
 
-void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out,
-         hipStream_t s, const double* act) {
+void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out, hipStream_t s) {
   int nb = dot_partials_count(n);
-  k_dot_partial<<<nb, DOT_BS, 0, s>>>(x, y, n, partial, act);
-  k_reduce<<<1, DOT_BS, 0, s>>>(partial, nb, out, sqrt_out, act);
+  k_dot_partial<<<nb, DOT_BS, 0, s>>>(x, y, n, partial);
+  k_reduce<<<1, DOT_BS, 0, s>>>(partial, nb, out, sqrt_out);
   EXA_HIP(hipGetLastError());
 }
 

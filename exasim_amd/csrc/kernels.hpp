@@ -213,8 +213,8 @@ void bj_assemble(const Dims& d, const int* f2e, const int* elemcon, const double
                  hipStream_t s);
 void bj_assemble(const Dims& d, const int* f2e, const int* elemcon, const float* H, double* aug, hipStream_t s);
 void bj_extract(const Dims& d, const double* aug, double* BE, hipStream_t s);
-// act (optional, device): the apply, dot and update kernels below do nothing when act[0] == 0 (a
-// solve that has finished while later steps were already queued)
+// act (optional, device): the apply kernels below do nothing when act[0] == 0 (a solve that has finished while
+// later steps were already queued)
 template <typename T>
 void bj_apply(const Dims& d, const T* BE, const TraceIn& in, double* y, hipStream_t s, const double* act = nullptr);
 // elemental additive Schwarz: augmented [block | I] for elements [e0, e0+eb), and the
@@ -279,8 +279,7 @@ void bilu_apply(const Dims& d, const IluDev& I, const T* BE, const double* x, do
 
 // ---- vector kernels (results stay on the device) ----
 constexpr int DOT_PARTIALS = 1024;  // partial sums of dot, at most
-void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out,
-         hipStream_t s, const double* act = nullptr);
+void dot(const double* x, const double* y, long n, double* partial, double* out, int sqrt_out, hipStream_t s);
 // y = a x + b y; with b == 0 y is only written
 void axpby(double* y, const double* x, double a, double b, long n, hipStream_t s);
 void copy(double* y, const double* x, long n, hipStream_t s);

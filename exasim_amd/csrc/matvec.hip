@@ -233,19 +233,24 @@ void products(const Blocks& b, const T* H, const TraceIn& in, double* we, hipStr
   constexpr int VMAX = 16 / sizeof(T);
   const int vw = rows_per_load<T>(b.m);
   if (b.m <= 64 * vw) {  // a column is at most one load of a wave
-    if (vw == VMAX) small_vw<T, VMAX>(b, H, in, we, s);
-    else if (vw == 4) small_vw<T, 4>(b, H, in, we, s);
-    else if (vw == 2) small_vw<T, 2>(b, H, in, we, s);
-    else small_vw<T, 1>(b, H, in, we, s);
+    if (vw == VMAX) {
+      small_vw<T, VMAX>(b, H, in, we, s);
+    } else if (vw == 4) {
+      if constexpr (VMAX > 4) small_vw<T, 4>(b, H, in, we, s);
+    } else if (vw == 2) {
+      if constexpr (VMAX > 2) small_vw<T, 2>(b, H, in, we, s);
+    } else {
+      small_vw<T, 1>(b, H, in, we, s);
+    }
   } else if (vw == VMAX) {
     const int nrb = (b.m + 64 * VMAX - 1) / (64 * VMAX);
     if (nrb == 2) launch_rows<T, VMAX, 2>(b, H, in, we, s);
     else if (nrb == 3) launch_rows<T, VMAX, 3>(b, H, in, we, s);
     else launch_rows<T, VMAX, 0>(b, H, in, we, s);
   } else if (vw == 4) {  // BF16 blocks: 8-byte loads
-    launch_rows<T, 4, 0>(b, H, in, we, s);
+    if constexpr (VMAX > 4) launch_rows<T, 4, 0>(b, H, in, we, s);
   } else if (vw == 2) {
-    launch_rows<T, 2, 0>(b, H, in, we, s);
+    if constexpr (VMAX > 2) launch_rows<T, 2, 0>(b, H, in, we, s);
   } else {
     launch_rows<T, 1, 0>(b, H, in, we, s);
   }
