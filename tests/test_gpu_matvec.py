@@ -1,7 +1,7 @@
 """The element products (matvec.hip) against numpy over the trace block sizes m where the kernels
 differ: loads of 1, 2 and 4 rows per lane (odd m, m = 2 mod 4, multiples of 4), one and four waves per
 element, several columns per load (m < 64) and one, the last lanes idle, and the row-block kernel
-above.  FP64 and FP32 operators, and the Schwarz blocks in FP64, FP32 and BF16 (8 rows per load)."""
+above (m = 2 mod 4: its form of two rows per lane, in FP32 and BF16).  FP64 and FP32 operators, and the Schwarz blocks in FP64, FP32 and BF16 (8 rows per load)."""
 import numpy as np
 import pytest
 import torch
@@ -17,6 +17,7 @@ CASES = [  # builder arguments, m
     ("poisson2d", dict(n=2, porder=2, pgauss=4, nd=3), 54),
     ("poisson2d", dict(n=2, porder=3, pgauss=6, nd=3), 96),
     ("convdiff3d", dict(n=2, porder=2), 108),
+    ("poisson2d", dict(n=2, porder=4, pgauss=8, nd=3), 150),
     ("convdiff3d", dict(n=2, porder=3), 192),
     ("convdiff3d", dict(n=2, porder=4), 300),
 ]
@@ -65,3 +66,27 @@ def test_element_products(tmp_path, builder, kw, m):
                 w, a = products(blocks, con, z["ncu"], z["N"], v)
                 # m products and sums of one element and the two sides' sum, each within eps/2
                 assert np.all(np.abs(out.cpu().numpy() - w) <= (m + 2) * eps * a + 1e-300)
+
+
+@pytest.mark.parametrize("mixed", [0, 1])
+def test_operator_of_large_blocks(tmp_path, mixed):
+    """m = 432: four row blocks in FP64, two in FP32 (Schwarz blocks have at most 400 rows)."""
+    from exasim_amd import cases
+    from exasim_amd.hdg import HDGSolver
+    info = cases.convdiff3d(str(tmp_path), n=2, porder=5, precond="bjacobi")
+    m = 432
+    with HDGSolver(str(tmp_path), info["model"]) as S:
+        S.set_option("precision", mixed)
+        S.get_q()
+        S.assemble()
+        z = S.sizes
+        assert z["m"] == m
+        v = np.random.default_rng(m).standard_normal(z["N"])
+        vd = torch.from_numpy(v).cuda()
+        wd = torch.empty_like(vd)
+        torch.cuda.synchronize()
+        S.matvec(vd.data_ptr(), wd.data_ptr())
+        S.sync()
+        H = S.get("H").reshape(z["ne"], m, m).transpose(0, 2, 1)
+        w, a = products(H, S.get("elemcon").astype(np.int64), z["ncu"], z["N"], v)
+        assert np.all(np.abs(wd.cpu().numpy() - w) <= (m + 2) * np.finfo(float).eps * a + 1e-300)
