@@ -365,6 +365,12 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// lane l's value (l uniform), to every lane
+__device__ __forceinline__ double lane_value(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
 // sum of the block's 256 values v in a fixed order, to every thread (sh: 4 values of LDS, free again at
 // the next barrier)
 __device__ __forceinline__ double block_sum(double v, double* sh) {
@@ -471,18 +477,20 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_reduce(SegMap m, const double* p
 }
 
 // x += alpha * sum_j V_j * y[j*nseg + seg]; NORM: npart[b*PIECES + piece] = <x, x> over the piece.  Bound by
-// reading V.  Four waves take 8 columns of a 64-entry piece in turn: 45,000 entries, 50 columns on average 6.5 us (a
-// thread per entry walking all columns, with one load in flight and few blocks: 14.2 us).  Two turns or fewer
-// leave waves idle: WHOLE then gives a wave a piece of its own (the same sums).  The turns do not depend on k: for
-// the solution's update a batch's longest solve sets k, and an instance's sum may not depend on it.
-// The coefficients are uniform and, the arguments being restrict, come by scalar loads: through the vector
-// caches, which V streams through, they cost 445 us instead of 368 at 5,068,800 entries and 49 columns.
+// reading V.  One block per 64 entries, its four waves a quarter of the columns each with 8 loads in
+// flight: 45,000 entries, 50 columns on average 6.5 us (a thread per entry walking all columns, with one
+// load in flight and few blocks: 14.2 us).
+// A turn's coefficients come with one load, a lane each, and lane reads: eight loads of all lanes through the
+// caches that V streams through cost 445 us instead of 368 at 5,068,800 entries and 49 columns.
+// KC > 0: at most KC columns in a quarter, and one wave takes all of them, four pieces to a block; the same sums.
 // SKIPZ: columns whose coefficient is zero are not read (a basis column the solve has not written in this
-// cycle may hold anything)
-template <bool SKIPZ, bool NORM, bool WHOLE>
+// cycle may hold anything), and the waves take 8 columns in turn, which does not depend on k: a batch's longest
+// solve sets k there, and an instance's sum may not depend on it.
+template <bool SKIPZ, bool NORM, int KC>
 __global__ __launch_bounds__(SEG_BS) void k_seg_gemv(SegMap m, double* __restrict__ x, const double* __restrict__ V,
                                                      long ldv, int k, const double* __restrict__ y, double alpha,
                                                      double* __restrict__ npart) {
+  constexpr bool WHOLE = KC > 0;
   constexpr int PB = WHOLE ? 4 : 1;  // pieces of the block
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.x / (PIECES / PB), piece = blockIdx.x % (PIECES / PB) * PB + (WHOLE ? wave : 0);
@@ -493,40 +501,53 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_gemv(SegMap m, double* __restric
     return;
   }
   const double* Vi = V + min(i0 + lane, end - 1);
-  const bool in = i0 + lane < end;
-  double xn = in && (WHOLE || wave == 0) ? x[i0 + lane] : 0.0;
-  const double* ys = y + sg;
-  auto turn = [&](int j, double acc) {  // columns j .. j + 7 (past the end: the last one, times 0)
-    double v[8], c[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int jj = min(j + u, k - 1);
-      c[u] = ys[static_cast<long>(jj) * m.nseg];
-      if (j + u >= k) c[u] = 0.0;
-      if (!SKIPZ) v[u] = Vi[ldv * jj];
-      else if (c[u] != 0.0) v[u] = Vi[ldv * jj];
-      else v[u] = 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < 8; ++u) acc = fma(v[u], c[u], acc);
-    return acc;
-  };
-  double r[4] = {0.0, 0.0, 0.0, 0.0};
-  if (WHOLE) {  // k <= 32
+  const int kc = (k + 3) / 4;
+  double s = 0.0;
+  if constexpr (WHOLE) {
+    const double yv = y[static_cast<long>(min(lane, k - 1)) * m.nseg + sg];
+    double v[4][KC];
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      if (8 * q < k) r[q] = turn(8 * q, 0.0);
+#pragma unroll
+      for (int u = 0; u < KC; ++u) v[q][u] = Vi[ldv * min(kc * q + u, k - 1)];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      double acc = 0.0;
+#pragma unroll
+      for (int u = 0; u < KC; ++u)
+        acc = fma(v[q][u], u < kc && kc * q + u < k ? lane_value(yv, min(kc * q + u, 63)) : 0.0, acc);
+      s += acc;
+    }
   } else {
     __shared__ double red[4][64];
+    const int j0 = SKIPZ ? 8 * wave : wave * kc, j1 = SKIPZ ? k : min(k, j0 + kc);
     double acc = 0.0;
-    for (int j = 8 * wave; j < k; j += 32) acc = turn(j, acc);
+    for (int j = j0; j < j1; j += SKIPZ ? 32 : 8) {
+      const double yv = y[static_cast<long>(min(j + (lane & 7), j1 - 1)) * m.nseg + sg];
+      double v[8], c[8];
+      if (SKIPZ) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          c[u] = j + u < j1 ? lane_value(yv, u) : 0.0;
+          v[u] = 0.0;
+          if (c[u] != 0.0) v[u] = Vi[ldv * (j + u)];
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = j + u < j1 ? Vi[ldv * (j + u)] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = j + u < j1 ? lane_value(yv, u) : 0.0;
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc = fma(v[u], c[u], acc);
+    }
     red[wave][lane] = acc;
     __syncthreads();
     if (wave != 0) return;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) r[q] = red[q][lane];
+    s = ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
   }
-  xn = in ? fma(alpha, ((r[0] + r[1]) + r[2]) + r[3], xn) : 0.0;
+  const bool in = i0 + lane < end;
+  const double xn = in ? fma(alpha, s, x[i0 + lane]) : 0.0;
   if (in) x[i0 + lane] = xn;
   if (NORM) {
     const double q = wave_sum(xn * xn);
@@ -580,9 +601,10 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_groups(SegMap m, const double* p
   if (threadIdx.x == 0) gsum[static_cast<long>(sg) * gmax + blockIdx.y] = s;
 }
 
-// End of an Arnoldi step: the norm of w from its partials (per per block; gmax: from the sums of their
+// End of an Arnoldi step: the norm of w from its partials (per per block; LONG: from the sums of their
 // groups, gmax of them per segment), w /= norm (0 where the norm is 0), and each instance's rotations and
 // convergence test.  Blocks [0, nseg): one instance each; the others: a chunk of w each.
+template <bool LONG>
 __global__ __launch_bounds__(SEG_BS) void k_seg_finish(SegMap m, GmresDev g, int i, double* w, const double* npart,
                                                        int per, int gmax, double* hcol) {
   __shared__ double sh[4];
@@ -590,17 +612,27 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_finish(SegMap m, GmresDev g, int
   const int blk = static_cast<int>(blockIdx.x) - m.nseg;
   const int sg = blk < 0 ? static_cast<int>(blockIdx.x) : m.bseg[blk];
   const int first = m.sbptr[sg], count = per * (m.sbptr[sg + 1] - first);
-  const long t0 = blk < 0 ? 0 : m.bbeg[blk] + threadIdx.x, t1 = blk < 0 ? 0 : m.bend[blk];
-  double wv[2];  // the chunk's values come while the norm is summed
+  double* hn = hcol + static_cast<long>(i + 1) * m.nseg + sg;
+  double wv[2];
+  if (LONG && blk >= 0)  // the chunk's values come while the norm is summed
 #pragma unroll
-  for (int q = 0; q < 2; ++q) wv[q] = t0 + SEG_BS * q < t1 ? w[t0 + SEG_BS * q] : 0.0;
-  const double nrm = sqrt(gmax ? partials_sum(npart + static_cast<long>(sg) * gmax, (count + GROUP - 1) / GROUP, sh)
+    for (int q = 0; q < 2; ++q) {
+      const long t = m.bbeg[blk] + threadIdx.x + SEG_BS * q;
+      wv[q] = t < m.bend[blk] ? w[t] : 0.0;
+    }
+  const double nrm = sqrt(LONG ? partials_sum(npart + static_cast<long>(sg) * gmax, (count + GROUP - 1) / GROUP, sh)
                                : partials_sum(npart + static_cast<long>(per) * first, count, sh));
   if (blk >= 0) {
     const double c = nrm != 0.0 ? 1.0 / nrm : 0.0;
+    if (LONG) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
-      if (t0 + SEG_BS * q < t1) w[t0 + SEG_BS * q] = wv[q] * c;
+      for (int q = 0; q < 2; ++q) {
+        const long t = m.bbeg[blk] + threadIdx.x + SEG_BS * q;
+        if (t < m.bend[blk]) w[t] = wv[q] * c;
+      }
+    } else {
+      for (long t = m.bbeg[blk] + threadIdx.x; t < m.bend[blk]; t += SEG_BS) w[t] *= c;
+    }
     return;
   }
   const int j = g.jcount[0];
@@ -610,7 +642,7 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_finish(SegMap m, GmresDev g, int
       for (int k = threadIdx.x; k <= i; k += SEG_BS) lds.h[k] = hcol[static_cast<long>(k) * m.nseg + sg];
     if (threadIdx.x == 0) {
       lds.h[min(i + 1, GM_LDS_N1)] = nrm;
-      hcol[static_cast<long>(i + 1) * m.nseg + sg] = nrm;
+      *hn = nrm;
     }
   }
   __syncthreads();
@@ -711,19 +743,24 @@ void launch_dots(const SegMap& m, const double* V, long ldv, int k, const double
   k_seg_dots<C><<<dim3(m.nblk, ny), SEG_BS, 0, s>>>(m, V, ldv, k, w, partial);
 }
 
-// k_seg_gemv with WHOLE: up to two turns, on chunks enough to fill the device without the idle waves.  An Arnoldi
-// step with 5 and 13 columns, four waves per piece / one: 330,000 entries 23.4 / 23.3 and 30.6 / 30.2 us; 630,000
-// 32.6 / 29.6 and 42.5 / 40.9; 1,260,000 49.2 / 41.6 and 64.5 / 61.1; 40,000 14.8 / 15.5 and 16.5 / 17.6.  With 25
-// columns 1,260,000 95.8 / 96.8.
-constexpr int WHOLE_COLS = 16, WHOLE_CHUNKS = 640;
+// k_seg_gemv with one wave per piece: few columns leave most of a wave's loads in flight unused otherwise.  A
+// step with 3, 5, 9 and 13 columns, four waves per piece / one: 24 instances, 330,000 entries 21.7/19.7,
+// 22.0/20.6, 24.5/23.8, 27.8/27.8 us; one problem, 5 columns, 630,000 entries 32.6/29.6, 1,260,000 49.2/42.2,
+// 5,068,800 141/112; 40,000 14.8/15.5.
+constexpr int WHOLE_COLS = 12, WHOLE_CHUNKS = 640;
 
-template <bool SKIPZ, bool NORM>
-void launch_gemv(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double alpha,
-                 double* npart, hipStream_t s) {
-  if (k <= WHOLE_COLS && m.nblk >= WHOLE_CHUNKS)
-    k_seg_gemv<SKIPZ, NORM, true><<<m.nblk * (PIECES / 4), SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha, npart);
-  else
-    k_seg_gemv<SKIPZ, NORM, false><<<m.nblk * PIECES, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha, npart);
+template <int KC>
+void launch_gemv_whole(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double* npart,
+                       hipStream_t s) {
+  k_seg_gemv<false, true, KC><<<m.nblk * (PIECES / 4), SEG_BS, 0, s>>>(m, x, V, ldv, k, y, -1.0, npart);
+}
+void launch_cgs_update(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double* npart,
+                       hipStream_t s) {
+  if (k > WHOLE_COLS || m.nblk < WHOLE_CHUNKS)
+    k_seg_gemv<false, true, 0><<<m.nblk * PIECES, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, -1.0, npart);
+  else if (k <= 4) launch_gemv_whole<1>(m, x, V, ldv, k, y, npart, s);
+  else if (k <= 8) launch_gemv_whole<2>(m, x, V, ldv, k, y, npart, s);
+  else launch_gemv_whole<3>(m, x, V, ldv, k, y, npart, s);
 }
 
 }  // namespace
@@ -770,7 +807,7 @@ void seg_arnoldi(const SegMap& m, const GmresDev& g, const double* V, long n, in
     seg_multidot(m, V, n, i + 1, w, partial, hcol, 0, s);
     np = partial;
     per = PIECES;
-    launch_gemv<false, true>(m, w, V, n, i + 1, hcol, -1.0, np, s);
+    launch_cgs_update(m, w, V, n, i + 1, hcol, np, s);
   }
   int gmax = 0;
   if (m.maxblk * per > GROUP) {
@@ -779,7 +816,8 @@ void seg_arnoldi(const SegMap& m, const GmresDev& g, const double* V, long n, in
     k_seg_groups<<<dim3(ns, gmax), SEG_BS, 0, s>>>(m, np, per, gsum, gmax);
     np = gsum;
   }
-  k_seg_finish<<<ns + m.nblk, SEG_BS, 0, s>>>(m, g, i, w, np, per, gmax, hcol);
+  if (gmax) k_seg_finish<true><<<ns + m.nblk, SEG_BS, 0, s>>>(m, g, i, w, np, per, gmax, hcol);
+  else k_seg_finish<false><<<ns + m.nblk, SEG_BS, 0, s>>>(m, g, i, w, np, per, 0, hcol);
   EXA_HIP(hipGetLastError());
 }
 
@@ -798,7 +836,7 @@ void seg_scale(const SegMap& m, double* y, const double* x, const double* coef, 
 void seg_gemv_cols(const SegMap& m, double* x, const double* V, long ldv, int k, const double* y, double alpha,
                    hipStream_t s) {
   if (m.nblk == 0 || k == 0) return;
-  launch_gemv<true, false>(m, x, V, ldv, k, y, alpha, nullptr, s);
+  k_seg_gemv<true, false, 0><<<m.nblk * PIECES, SEG_BS, 0, s>>>(m, x, V, ldv, k, y, alpha, nullptr);
   EXA_HIP(hipGetLastError());
 }
 
