@@ -520,7 +520,8 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
   const long e = blockIdx.x;
   const int lane = threadIdx.x;
   const float* Le = LU + e * static_cast<long>(n) * n;
-  double y[RPL], diag[RPL], dinv[RPL];
+  __shared__ double diag[64 * RPL], dinv[64 * RPL];
+  double y[RPL];
   int pv[RPL];
   int row[RPL];
 #pragma unroll
@@ -529,16 +530,20 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
     row[q] = min(r, n - 1);
     y[q] = Ru[e * n + row[q]];
     pv[q] = piv[e * n + row[q]];
-    diag[q] = static_cast<double>(Le[row[q] + static_cast<long>(n) * row[q]]);
-    dinv[q] = 1.0 / diag[q];
+    const double dq = static_cast<double>(Le[row[q] + static_cast<long>(n) * row[q]]);
+    diag[r] = dq;
+    dinv[r] = 1.0 / dq;
   }
-  // entry k (uniform) of a vector held like y
+  // entry k (uniform) of a vector held like y (every register's lane read, then the choice: choosing the
+  // register first, the compiler may put the vector in memory and index it)
   auto pick = [&](const double (&v)[RPL], int k) {
-    double x = v[0];
+    double x = lane_value(v[0], k & 63);
 #pragma unroll
-    for (int q = 1; q < RPL; ++q)
-      if (k >= 64 * q) x = v[q];
-    return lane_value(x, k & 63);
+    for (int q = 1; q < RPL; ++q) {
+      const double t = lane_value(v[q], k & 63);
+      x = k >= 64 * q ? t : x;
+    }
+    return x;
   };
   float col[2][8][RPL];
   auto load = [&](int b, int k) {  // columns k .. k + 7 (past either end: the nearest one, unused)
@@ -584,8 +589,7 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
 #pragma unroll
     for (int u = 7; u >= 0; --u)
       if (k + u >= 0) {
-        const double yr = pick(y, k + u), dk = pick(diag, k + u), di = pick(dinv, k + u);
-        const double qt = yr * di;
+        const double dk = diag[k + u], di = dinv[k + u], yr = pick(y, k + u), qt = yr * di;
         const double yk = fma(fma(-qt, dk, yr), di, qt);  // yr / dk, the quotient corrected by its remainder
 #pragma unroll
         for (int q = 0; q < RPL; ++q) {
@@ -595,6 +599,7 @@ __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float
         }
       }
   };
+  __syncthreads();
   load(0, n - 8);
   for (int k = n - 8; k > -8; k -= 16) {
     load(1, k - 8);
