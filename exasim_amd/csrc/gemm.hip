@@ -36,7 +36,7 @@ namespace {
 // product run side by side and share operands through the caches.  Lane l of a 16x16x4 step supplies
 // A[l%16][k] and B[k][l%16] with k = l/16 of the step; since a product's sum may take its K values in
 // any order, step s of a block uses k = 4 (l/16) + s, so that a lane's four B values are contiguous
-// and load as vectors.
+// and load as one vector.
 //
 // Bound by MFMA issue at the clock that the power limit leaves (counters of the 250 x 275 x 375 FP64
 // product: the matrix cores busy 71 % of the cycles at 1.9 GHz), small K by the traffic of C.  Against
@@ -44,8 +44,8 @@ namespace {
 //   250 x 275 x 375, batch 2400:   FP64 3.77 -> 2.72 ms (33 -> 46 TFLOP/s), FP32 1.99 -> 1.67 ms (62 -> 74)
 //   300 x 300 x 250, batch 1200:   FP64 1.94 -> 1.38 ms, FP32 1.10 -> 0.82 ms
 //   186 x 487 x 64, batch 1200:    FP32 0.47 -> 0.40 ms (reads and writes C)
-//   trailing updates of the FP64 LU, K = 32, n = 250, batch 2670 / n = 196, batch 1000 / n = 64, batch 1331
-//                                  10.0 -> 9.5 ms / 1.13 -> 0.97 ms / 65 -> 58 us (reads and writes C)
+//   all updates of one FP64 LU, K = 32, n = 250, batch 2670 / batch 1200 / n = 196, batch 1000 / n = 64, batch 1331
+//                                  9.95 -> 9.93 ms / 4.54 -> 4.26 / 1.13 -> 0.96 / 65 -> 54 us (read and write C)
 //   144 x 36 x 72, batch 8100:     FP64 0.62 -> 0.40 ms, FP32 0.35 -> 0.20 ms
 //   25 x 25 x 25, batch 25000:     FP64 117 -> 70 us
 // ---------------------------------------------------------------------------
@@ -60,25 +60,23 @@ __device__ __forceinline__ dbl4 mfma_step(double a, double b, dbl4 c) {
 __device__ __forceinline__ flt4 mfma_step(float a, float b, flt4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-// The matrix row that row r of the A operand's tile holds: chosen so that the lane's registers are pieces of
-// 16 bytes of consecutive rows, piece h of lane l at row PSTEP h + PW (l/16) of the output tile: one access
-// of the four lane groups then covers 64 contiguous bytes of a column.  (With all four FP64 rows of a lane
-// contiguous, its two accesses each took every other 16 bytes: the trailing updates of an FP64 LU of 2,670
-// matrices of 250 rows and 301 right-hand sides, bound by C, 10.25 ms; in pieces 9.45.)
-__device__ __forceinline__ int a_row(double, int r) { return 8 * (r >> 3) + 2 * (r & 3) + ((r >> 2) & 1); }
+// A lane's four registers of an output tile hold pieces of W consecutive rows, piece h of lane l at row
+// 4 W h + W (l/16) of the tile.  The matrix row that row r of the A operand's tile holds for this:
+template <int W>
+__device__ __forceinline__ int a_row(double, int r) {
+  return W == 4 ? 4 * (r & 3) + (r >> 2) : 8 * (r >> 3) + 2 * (r & 3) + ((r >> 2) & 1);
+}
+template <int W>
 __device__ __forceinline__ int a_row(float, int r) { return r; }
 
-// 16 bytes of consecutive values at the alignment of one (global loads need no more)
-template <typename T> struct Piece;
-template <> struct Piece<double> {
-  typedef double type __attribute__((ext_vector_type(2), aligned(8)));
+// W consecutive values at the alignment of one (global loads need no more)
+template <typename T, int W> struct Vec;
+template <int W> struct Vec<double, W> {
+  typedef double type __attribute__((ext_vector_type(W), aligned(8)));
 };
-template <> struct Piece<float> {
-  typedef float type __attribute__((ext_vector_type(4), aligned(4)));
+template <int W> struct Vec<float, W> {
+  typedef float type __attribute__((ext_vector_type(W), aligned(4)));
 };
-template <typename T> constexpr int PW = 16 / sizeof(T);    // values of a piece
-template <typename T> constexpr int NP = 4 / PW<T>;         // pieces of a lane's four registers
-template <typename T> constexpr int PSTEP = 16 / NP<T>;     // rows from a piece to the lane's next
 
 // operands in the product's type
 template <typename T> __device__ __forceinline__ T* gsel(double* d, float* f);
@@ -94,13 +92,23 @@ template <> __device__ __forceinline__ const float* gsel<float>(const double*, c
 // that share an operand run together on one XCD and reuse it from its L2.
 constexpr int NXCD = 8;
 
+// Rows of a piece (W above).  In FP64 a lane's four rows lie together, 32 bytes, or in two pieces of 16, of which
+// one access of the four lane groups covers 64 contiguous bytes of a column, where else its two accesses each take
+// every other 16.  The small tile, which products bound by C run on, gains: 218 x 519 x 32, batch 2699, 1718 ->
+// 1572 us; 154 x 455 x 32 1116 -> 1031; 90 x 391 x 32 614 -> 567.  The larger ones, with C read after the K loop, lose
+// (four rows / two pieces): 4 x 4 MFMA tiles 1964/2467, 4 x 2 1999/1994, 2 x 4 1990/2094 us in the first.
+template <typename T, int FM, int FN>
+constexpr int rows_piece() { return sizeof(T) == 8 && FM * FN <= 4 ? 2 : 4; }
+
 // A workgroup of WM x WN waves; T: double or float throughout.  Two waves per SIMD (256 registers),
 // except for the FP64 4 x 4 tiles, whose accumulators and operand blocks take more.
 template <typename T, int FM, int FN, int WM, int WN>
 __global__ __launch_bounds__(64 * WM * WN)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) * FM * FN > 64 ? 1 : 2)))
 void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
-  typedef typename Piece<T>::type piece;
+  constexpr int W = rows_piece<T, FM, FN>(), NP = 4 / W, STEP = 4 * W;
+  typedef typename Vec<T, 4>::type v4;
+  typedef typename Vec<T, W>::type piece;
   typedef T acc4 __attribute__((ext_vector_type(4)));
   const unsigned nwg = gridDim.x;  // a multiple of NXCD
   const unsigned L = (blockIdx.x % NXCD) * (nwg / NXCD) + blockIdx.x / NXCD;
@@ -124,7 +132,7 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
   const unsigned ka = lda * (4 * lk), kb = 4 * lk;
   unsigned oa[FM], ob[FN];
 #pragma unroll
-  for (int i = 0; i < FM; ++i) oa[i] = (min(row0 + 16 * i + a_row(T(0), li), M - 1) + ka) * sizeof(T);
+  for (int i = 0; i < FM; ++i) oa[i] = (min(row0 + 16 * i + a_row<W>(T(0), li), M - 1) + ka) * sizeof(T);
 #pragma unroll
   for (int j = 0; j < FN; ++j)
     ob[j] = (static_cast<unsigned>(g.ldb) * min(col0 + 16 * j + li, N - 1) + kb) * sizeof(T);
@@ -137,7 +145,7 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
   // MFMA tiles of the wave that hold output (the others' loads are harmless, their products skipped)
   const int fm = min(FM, (M - row0 + 15) / 16), fn = min(FN, (N - col0 + 15) / 16);
   T av[2][FM][4];
-  T bv[2][FN][4];
+  v4 bv[2][FN];
   auto load = [&](int buf, int k0) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -145,16 +153,9 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
 #pragma unroll
       for (int i = 0; i < FM; ++i) av[buf][i][s] = *reinterpret_cast<const T*>(at_byte(Ak, oa[i]));
     }
+    const T* Bk = B + k0;
 #pragma unroll
-    for (int h = 0; h < NP<T>; ++h) {
-      const T* Bk = B + k0 + PW<T> * h;
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const piece x = *reinterpret_cast<const piece*>(at_byte(Bk, ob[j]));
-#pragma unroll
-        for (int q = 0; q < PW<T>; ++q) bv[buf][j][PW<T> * h + q] = x[q];
-      }
-    }
+    for (int j = 0; j < FN; ++j) bv[buf][j] = *reinterpret_cast<const v4*>(at_byte(Bk, ob[j]));
   };
   // the products of the block in buffer buf, interleaved with the loads of the next one into the
   // other (one load after every few products keeps both queues fed)
@@ -166,7 +167,7 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
       for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = mfma_step(av[buf][i][s], bv[buf][j][s], acc[i][j]);
-    constexpr int NLOAD = 4 * FM + FN * NP<T>, PER = 4 * FM * FN / NLOAD;
+    constexpr int NLOAD = 4 * FM + FN * (sizeof(T) == 8 ? 2 : 1), PER = 4 * FM * FN / NLOAD;
 #pragma unroll
     for (int q = 0; q < NLOAD; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x20, 1, 0);   // one global load
@@ -191,10 +192,10 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
   // its latency would otherwise follow theirs)
   constexpr bool EARLY_C = sizeof(T) * FM * FN <= 32;
   const T alpha = static_cast<T>(g.alpha), beta = static_cast<T>(g.beta);
-  piece cv[FM][FN][NP<T>];
+  piece cv[FM][FN][NP];
   auto load_c = [&](int i, int j, int h) {
-    const int r = row0 + 16 * i + PSTEP<T> * h + PW<T> * lk, c = col0 + 16 * j + li;
-    if (c < N && r + PW<T> <= M) cv[i][j][h] = *reinterpret_cast<const piece*>(C + r + g.ldc * c);
+    const int r = row0 + 16 * i + STEP * h + W * lk, c = col0 + 16 * j + li;
+    if (c < N && r + W <= M) cv[i][j][h] = *reinterpret_cast<const piece*>(C + r + g.ldc * c);
   };
   if (EARLY_C && beta != T(0)) {
 #pragma unroll
@@ -202,7 +203,7 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
 #pragma unroll
       for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int h = 0; h < NP<T>; ++h) load_c(i, j, h);
+        for (int h = 0; h < NP; ++h) load_c(i, j, h);
   }
   // A block's loads are always issued (past the end: the last block again, unused), so that the wait
   // before the products counts only older loads.
@@ -256,26 +257,26 @@ void k_gemm(Gemm g, int tilesM, int tilesN, unsigned ntiles) {
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int h = 0; h < NP<T>; ++h) {
-        const int r = row0 + 16 * i + PSTEP<T> * h + PW<T> * lk, c = col0 + 16 * j + li;
+      for (int h = 0; h < NP; ++h) {
+        const int r = row0 + 16 * i + STEP * h + W * lk, c = col0 + 16 * j + li;
         if (c >= N || r >= M) continue;
         T* p = C + r + g.ldc * c;
-        if (r + PW<T> <= M) {
+        if (r + W <= M) {
           piece x;
           if (beta != T(0)) {
             if (!EARLY_C) load_c(i, j, h);
 #pragma unroll
-            for (int q = 0; q < PW<T>; ++q) x[q] = fma(beta, cv[i][j][h][q], alpha * acc[i][j][PW<T> * h + q]);
+            for (int q = 0; q < W; ++q) x[q] = fma(beta, cv[i][j][h][q], alpha * acc[i][j][W * h + q]);
           } else {
 #pragma unroll
-            for (int q = 0; q < PW<T>; ++q) x[q] = alpha * acc[i][j][PW<T> * h + q];
+            for (int q = 0; q < W; ++q) x[q] = alpha * acc[i][j][W * h + q];
           }
           *reinterpret_cast<piece*>(p) = x;
         } else {
 #pragma unroll
-          for (int q = 0; q < PW<T> - 1; ++q)
+          for (int q = 0; q < W - 1; ++q)
             if (r + q < M) {
-              const T v = alpha * acc[i][j][PW<T> * h + q];
+              const T v = alpha * acc[i][j][W * h + q];
               p[q] = beta != T(0) ? fma(beta, p[q], v) : v;
             }
         }
@@ -336,7 +337,8 @@ MfmaLaunch mfma_launcher(int fp32, int tile) {
 // ---------------------------------------------------------------------------
 template <typename T, int FM, int FN, bool STAGE>
 __global__ __launch_bounds__(256) void k_face_elim(FaceElim<T> f, int kpad, int tilesM, int tilesK, int tilesH) {
-  typedef typename Piece<T>::type piece;
+  constexpr int W = 16 / sizeof(T), NP = 4 / W, STEP = 4 * W;  // as k_gemm's small tiles
+  typedef typename Vec<T, W>::type piece;
   typedef T acc4 __attribute__((ext_vector_type(4)));
   extern __shared__ double face_sm[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -377,7 +379,7 @@ __global__ __launch_bounds__(256) void k_face_elim(FaceElim<T> f, int kpad, int 
     const T* A = f.G + e * static_cast<long>(m) * K * ncu + static_cast<long>(m) * K * cp + l * M;
     unsigned oa[FM];
 #pragma unroll
-    for (int i = 0; i < FM; ++i) oa[i] = min(row0 + 16 * i + a_row(T(0), li), M - 1) * unsigned(sizeof(T));
+    for (int i = 0; i < FM; ++i) oa[i] = min(row0 + 16 * i + a_row<W>(T(0), li), M - 1) * unsigned(sizeof(T));
     acc4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -443,21 +445,21 @@ __global__ __launch_bounds__(256) void k_face_elim(FaceElim<T> f, int kpad, int 
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int h = 0; h < NP<T>; ++h) {
-          const int r = row0 + 16 * i + PSTEP<T> * h + PW<T> * lk;
+        for (int h = 0; h < NP; ++h) {
+          const int r = row0 + 16 * i + STEP * h + W * lk;
           T* p = C + m * at + l * M + r;
           const T* x = X + m * max(x0, 0L) + l * M + r;
           piece v;
 #pragma unroll
-          for (int t = 0; t < PW<T>; ++t) {
-            const T y = acc[i][j][PW<T> * h + t];
+          for (int t = 0; t < W; ++t) {
+            const T y = acc[i][j][W * h + t];
             v[t] = isH ? -y : y;
             if (x0 >= 0 && r + t < M) v[t] += x[t];
           }
-          if (r + PW<T> <= M) *reinterpret_cast<piece*>(p) = v;
+          if (r + W <= M) *reinterpret_cast<piece*>(p) = v;
           else
 #pragma unroll
-            for (int t = 0; t < PW<T> - 1; ++t)
+            for (int t = 0; t < W - 1; ++t)
               if (r + t < M) p[t] = v[t];
         }
     }
