@@ -512,7 +512,8 @@ void lu_small(double* A, int n, int ncols, long stride, int batch, int* info, hi
 // row exchanges, then the unit-lower elimination), then the upper-triangular solve.  One wave per element:
 // lane t holds entries t, t + 64, .. of the vector in registers, entry k reaches the others by a lane
 // read, and 8 columns of the factors are loaded ahead, so a column costs no barrier (n = 100, 4096
-// elements: 85 us, and 32 us for Rh -= K RuS, against 309 us together with a workgroup and two barriers per column).
+// elements: 85 us, and 32 us for Rh -= K RuS, against 309 us together with a workgroup and two barriers per column;
+// n = 250, with the product of 100 rows: 443 us).  The diagonal and its reciprocal wait in LDS.
 // The panel width nbp (a multiple of 16) is the one lu_solve used for the factorisation.
 template <int RPL>
 __global__ __launch_bounds__(64) void k_refine_solve(int n, int nbp, const float* LU, const int* piv,

@@ -92,8 +92,9 @@ int exa_sizes(const exa_handle* h, int* out, int len);
  * explicit triangle inverses by MFMA products (1) or solves by substitution (0);
  * "ilu_wave" (process-wide; 1 default, 0, or -1 for the EXA_BILU_WAVE environment value): the
  * block-ILU(0) apply with one wave per superelement where it is the faster one (BF16 factors of
- * 50 x 50 blocks; any factors of blocks that few lanes hold) (1) or always with a 256-thread
- * workgroup per superelement (0). */
+ * 50 x 50 blocks; any factors of blocks of up to 28 rows that few lanes hold, and of 30 and 32 rows in
+ * FP32 and BF16 on 512 superelements or more) (1) or always with a 256-thread workgroup per
+ * superelement (0). */
 int exa_set_option(exa_handle* h, const char* name, double value);
 
 /* Full steady solve (NewtonSolver).  newton_iters/gmres_iters/final_norm may be NULL. */
