@@ -54,12 +54,14 @@ def test_forms_agree(tmp_path, kw, ortho):
 
 
 @pytest.mark.parametrize("kw", [dict(n=2, porder=1, pgauss=2), dict(n=32, porder=3, pgauss=6),
-                                dict(n=17, porder=3, pgauss=6, nd=3), dict(n=20, porder=4, pgauss=8, nd=3)])
+                                dict(n=17, porder=3, pgauss=6, nd=3), dict(n=20, porder=4, pgauss=8, nd=3),
+                                dict(n=24, porder=4, pgauss=8, nd=3)])
 @pytest.mark.parametrize("ortho", [0, 1])
 def test_steps(tmp_path, kw, ortho):
     """The solution after k steps against the minimiser over the same Krylov space, formed with torch and
     orthogonalised twice: k where the dots' and the update's waves take other shares of the vectors, on one
-    chunk, many, and enough for the norm's partials to be summed in groups."""
+    chunk, many, and enough for the norm's partials to be summed in groups (MGS beyond 1,048,576 entries, CGS
+    beyond 131,072)."""
     from exasim_amd import cases
     from exasim_amd.hdg import HDGSolver
     cases.poisson2d(str(tmp_path), model="poisson_poly", precond="eas", gmres_tol=1e-14, ortho=ortho, **kw)
@@ -110,12 +112,13 @@ def test_steps(tmp_path, kw, ortho):
 
 @pytest.mark.parametrize("ortho", [0, 1])
 def test_batch_with_a_long_instance(tmp_path, ortho):
-    """A short instance's sums do not depend on the batch it is in, also where the norm of another one is long
-    enough to be summed in groups (157,920 entries)."""
+    """An instance's sums do not depend on the batch it is in: a short one beside others whose norm is long enough
+    to be summed in groups (157,920 entries and more), and all of them where the batch's chunks (1,070) give one
+    wave a piece of the update and the instances' own (404 at most) four."""
     from exasim_amd import cases
     from exasim_amd.hdg import HDGSolver
     paths = []
-    for n in (16, 140):
+    for n in (16, 140, 150, 160):
         paths.append(str(tmp_path / str(n)))
         cases.poisson2d(paths[-1], n=n, porder=3, pgauss=6, model="poisson_poly", precond="eas", gmres_tol=1e-10,
                         restart=60, gmres_maxit=300, ortho=ortho)
