@@ -601,6 +601,22 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_groups(SegMap m, const double* p
   if (threadIdx.x == 0) gsum[static_cast<long>(sg) * gmax + blockIdx.y] = s;
 }
 
+// sum of a segment's count group sums, by every wave for itself: a few as uniform values (194,400 entries, two
+// groups, 25 columns: a step 29.0 us as with one reduction in a launch of its own; by the block 29.3), many by the lanes
+__device__ __forceinline__ double groups_sum(const double* p, int count) {
+  double acc = 0.0;
+  if (count <= 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = u < count ? p[u] : 0.0;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc += v[u];
+    return acc;
+  }
+  for (int i = threadIdx.x & 63; i < count; i += 64) acc += p[i];
+  return wave_sum(acc);
+}
+
 // End of an Arnoldi step: the norm of w from its partials (per per block; LONG: from the sums of their
 // groups, gmax of them per segment), w /= norm (0 where the norm is 0), and each instance's rotations and
 // convergence test.  Blocks [0, nseg): one instance each; the others: a chunk of w each.
@@ -620,7 +636,7 @@ __global__ __launch_bounds__(SEG_BS) void k_seg_finish(SegMap m, GmresDev g, int
       const long t = m.bbeg[blk] + threadIdx.x + SEG_BS * q;
       wv[q] = t < m.bend[blk] ? w[t] : 0.0;
     }
-  const double nrm = sqrt(LONG ? partials_sum(npart + static_cast<long>(sg) * gmax, (count + GROUP - 1) / GROUP, sh)
+  const double nrm = sqrt(LONG ? groups_sum(npart + static_cast<long>(sg) * gmax, (count + GROUP - 1) / GROUP)
                                : partials_sum(npart + static_cast<long>(per) * first, count, sh));
   if (blk >= 0) {
     const double c = nrm != 0.0 ? 1.0 / nrm : 0.0;
